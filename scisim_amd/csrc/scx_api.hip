@@ -102,7 +102,7 @@ uint32_t next_pow2(uint64_t v) {
 // After a step with stats: the share of the contacts in the component phase for the next
 // step (one scene; comp_share_update).
 void comp_adapt_share(scx_ctx* c, const StepCounters& h) {
-  if (!c->comp_adapt || !c->comp_sweeps || c->nscenes || h.sweeps == 0) return;
+  if (!c->comp_adapt || !c->comp_sweeps || !c->barrier_sweeps || c->nscenes || h.sweeps == 0) return;
   comp_share_update(c->comp_share, c->comp_ceiling, h.comp_overflows, h.comp_launches, h.comp_maxw,
                     (uint32_t)kGSBlock);
 }
@@ -260,6 +260,7 @@ void free_all(scx_ctx* c) {
   dfree(&d.comp_parent);
   dfree(&d.comp_cnt);
   dfree(&d.comp_list);
+  dfree(&d.wg_arena);
   uint32_t* u32[] = {d.cells, d.ent, d.pcount, d.scan_tmp, d.pa, d.pb, d.ca, d.cb, d.mbcount, d.deg, d.adj,
                      d.perm, d.coloff};
   for (uint32_t* p : u32)
@@ -614,6 +615,13 @@ int scx_create(const scx_config* cfg, scx_ctx** out) {
       c->comp_share = std::min(100.0, std::max(1.0, atof(env)));
       c->comp_adapt = false;
     }
+    // SCX_WG_SWEEPS=0: contact sets whose bodies one workgroup's LDS holds are swept with
+    // grid barriers all the same (the same iterates bit for bit; for A/B measurements and
+    // tests). The switches of the sweeps with barriers above keep a context on them unless
+    // this one says otherwise.
+    if (getenv("SCX_COMPONENT_SWEEPS") || getenv("SCX_COMPONENT_PERCENT") || getenv("SCX_COHERENT_SWEEPS"))
+      c->wg_sweeps = false;
+    if (const char* env = getenv("SCX_WG_SWEEPS")) c->wg_sweeps = atoi(env) != 0;
     if ((e = dalloc(&d.partial, (size_t)std::max(c->gs_blocks, 1) + 1)) != hipSuccess ||
         (e = dalloc(&d.viol, (size_t)3 + kViolCap)) != hipSuccess ||
         (e = dalloc(&d.comp_cnt, (size_t)std::max(c->gs_blocks, 1) + 1)) != hipSuccess ||

@@ -203,6 +203,8 @@ struct DeviceBuffers {
   uint32_t* comp_parent = nullptr;  // N: union-find parents of the component phase (k_gs)
   uint32_t* comp_cnt = nullptr;     // 1 + gs_blocks: overflow flag, per-workgroup counts
   uint32_t* comp_list = nullptr;    // gs_blocks x kCompCap: per-workgroup contacts
+  unsigned char* wg_arena = nullptr;  // working memory of the one-workgroup sweeps (cap_wg bytes)
+  size_t cap_wg = 0;
   // warm-start cache (previous step's active set, sorted keys + impulses)
   // keys ascend in active-set order: (i << 32 | j) for body pairs, then
   // (1 << 63 | plane << 32 | i) for plane contacts
@@ -279,6 +281,8 @@ struct scx_ctx {
   bool comp_lds = true;         // component phase: hold a workgroup's components in LDS when they fit
   double comp_ceiling = 100.0;  // below the last share that overflowed (drifts back up)
   bool comp_adapt = true;
+  bool barrier_sweeps = false;  // the last solve swept with grid barriers (k_gs)
+  bool wg_sweeps = true;        // one scene: sweep in one workgroup when its LDS holds the bodies
   // The device's cooperative queues are limited in number (HSA_QUEUE_TYPE_COOPERATIVE,
   // hsa/hsa.h: "Queues of this type may be limited in number"); while another process holds
   // them a cooperative launch fails with hipErrorIllegalState. The persistent kernels need

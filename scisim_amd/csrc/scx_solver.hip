@@ -21,6 +21,7 @@
 #include "scx_device.h"
 #include "scx_flow.h"
 #include "scx_internal.h"
+#include "scx_sweep.h"
 
 #include <algorithm>
 #include <cmath>
@@ -29,158 +30,6 @@
 
 namespace scx {
 
-
-template <typename Real>
-struct Vec4 {
-  using type = double4;
-};
-template <>
-struct Vec4<float> {
-  using type = float4;
-};
-
-template <int D, typename Real>
-struct Rec {
-  uint32_t a, b;
-  Real n[3], s[3], t[3];
-  Real la, lb, wn, wt, mu, f;
-};
-
-// The rest of the contact frame from n (and s in 3D): t = n x s (3D), t = (-n_y, n_x) (2D).
-template <int D, typename Real>
-__device__ __forceinline__ void frame_from_ns(Rec<D, Real>& R) {
-  if (D == 3) {
-    R.t[0] = R.n[1] * R.s[2] - R.n[2] * R.s[1];
-    R.t[1] = R.n[2] * R.s[0] - R.n[0] * R.s[2];
-    R.t[2] = R.n[0] * R.s[1] - R.n[1] * R.s[0];
-  } else {
-    R.t[0] = -R.n[1];
-    R.t[1] = R.n[0];
-    R.t[2] = 0;
-    R.s[0] = R.s[1] = R.s[2] = 0;
-    R.la = R.lb = 0;
-  }
-}
-
-template <int D, typename Real>
-__device__ __forceinline__ void load_rec(const ContactSoA<Real>& c, uint32_t k, Rec<D, Real>& R) {
-  R.a = c.a[k];
-  R.b = c.b[k];
-#pragma unroll
-  for (int d = 0; d < 3; ++d) R.n[d] = c.n[3 * (size_t)k + d];
-  if (D == 3) {
-#pragma unroll
-    for (int d = 0; d < 3; ++d) R.s[d] = c.s[3 * (size_t)k + d];
-    R.la = c.la[k];
-    R.lb = c.lb[k];
-  }
-  frame_from_ns<D, Real>(R);
-  R.wn = c.wn[k];
-  R.wt = c.wt[k];
-  R.mu = c.mu[k];
-  R.f = c.forcing[k];
-}
-
-// Pre-impulse relative velocity in the contact frame, u = H_a v_a - H_b v_b + w,
-// computed in precision T from bodies stored in precision Real.
-template <int D, typename T, typename Real>
-__device__ __forceinline__ void rel_vel(const Rec<D, Real>& R, const typename Vec4<Real>::type& va,
-                                        const typename Vec4<Real>::type& wa, const typename Vec4<Real>::type& vb,
-                                        const typename Vec4<Real>::type& wb, T u[3]) {
-  const T dv[3] = {(T)va.x - (T)vb.x, (T)va.y - (T)vb.y, (T)va.z - (T)vb.z};
-  const T n[3] = {(T)R.n[0], (T)R.n[1], (T)R.n[2]};
-  const T t[3] = {(T)R.t[0], (T)R.t[1], (T)R.t[2]};
-  u[0] = n[0] * dv[0] + n[1] * dv[1] + n[2] * dv[2] + (T)R.f;
-  if (D == 3) {
-    const T s[3] = {(T)R.s[0], (T)R.s[1], (T)R.s[2]};
-    const T la = (T)R.la, lb = (T)R.lb;
-    const T ca[3] = {(T)wa.y * n[2] - (T)wa.z * n[1], (T)wa.z * n[0] - (T)wa.x * n[2],
-                     (T)wa.x * n[1] - (T)wa.y * n[0]};
-    const T cb[3] = {(T)wb.y * n[2] - (T)wb.z * n[1], (T)wb.z * n[0] - (T)wb.x * n[2],
-                     (T)wb.x * n[1] - (T)wb.y * n[0]};
-    T uv[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) uv[d] = dv[d] - la * ca[d] - lb * cb[d];
-    u[1] = s[0] * uv[0] + s[1] * uv[1] + s[2] * uv[2];
-    u[2] = t[0] * uv[0] + t[1] * uv[1] + t[2] * uv[2];
-  } else {
-    u[1] = t[0] * dv[0] + t[1] * dv[1];
-    u[2] = 0;
-  }
-}
-
-// Exact Coulomb solution for the block diag(w_n, w_t, w_t): separate, stick, or slide
-// on the cone boundary against the tangential pre-velocity.
-template <int D, typename Real>
-__device__ __forceinline__ void local_solve(const Rec<D, Real>& R, const Real u[3], const Real r[3], Real rn[3]) {
-  const Real bn = u[0] - R.wn * r[0];
-  const Real n0 = -bn / R.wn;
-  if (!(n0 > (Real)0)) {
-    rn[0] = rn[1] = rn[2] = 0;
-    return;
-  }
-  rn[0] = n0;
-  Real nrm2 = 0;
-#pragma unroll
-  for (int a = 1; a < D; ++a) {
-    rn[a] = -(u[a] - R.wt * r[a]) / R.wt;
-    nrm2 += rn[a] * rn[a];
-  }
-  if (D == 2) rn[2] = 0;
-  const Real lim = R.mu * n0;
-  const Real nrm = sqrt(nrm2);
-  if (nrm > lim) {
-    const Real sc = (nrm > (Real)0) ? lim / nrm : (Real)0;
-#pragma unroll
-    for (int a = 1; a < D; ++a) rn[a] *= sc;
-  }
-}
-
-// FB residual of one contact (De Saxce change of variable), ||phi||^2, in precision T
-// (FP64 for every decision on the tolerance; FP32 only for the estimate of the FP32 phase).
-template <int D, typename T = double>
-__device__ __forceinline__ T fb_err(T mu, const T* r, const T* u) {
-  T uT2 = (T)0;
-#pragma unroll
-  for (int a = 1; a < D; ++a) uT2 += u[a] * u[a];
-  const T un_hat = u[0] + mu * sqrt(uT2);
-  T xh[3], yh[3];
-  xh[0] = mu * r[0];
-  yh[0] = un_hat;
-#pragma unroll
-  for (int a = 1; a < D; ++a) {
-    xh[a] = r[a];
-    yh[a] = mu * u[a];
-  }
-  T z0 = (T)0;
-#pragma unroll
-  for (int a = 0; a < D; ++a) z0 += xh[a] * xh[a] + yh[a] * yh[a];
-  T z1[2] = {(T)0, (T)0}, nz1 = (T)0;
-#pragma unroll
-  for (int a = 1; a < D; ++a) {
-    z1[a - 1] = (T)2 * (xh[0] * xh[a] + yh[0] * yh[a]);
-    nz1 += z1[a - 1] * z1[a - 1];
-  }
-  nz1 = sqrt(nz1);
-  const T s1 = sqrt(z0 + nz1);
-  const T s2 = sqrt(fmax((T)0, z0 - nz1));
-  T e = xh[0] + yh[0] - (T)0.5 * (s1 + s2);
-  e = e * e;
-#pragma unroll
-  for (int a = 1; a < D; ++a) {
-    const T dir = nz1 > (T)0 ? z1[a - 1] / nz1 : (T)0;
-    const T p = xh[a] + yh[a] - (T)0.5 * (s1 - s2) * dir;
-    e += p * p;
-  }
-  // a NaN residual (e.g. from non-finite velocities) counts as infinitely far from the
-  // solution: the max reductions drop NaN operands, so it must never read as converged
-  return __builtin_isnan(e) ? (T)INFINITY : e;
-}
-
-// Body records per slot: 2D one vector [v (3) | minv], 3D two adjacent vectors
-// [v (3) | minv][omega (3) | Iinv].
-template <int D>
-constexpr int kBodyVecs = (D == 3) ? 2 : 1;
 
 // Coherent accesses to the body records for the colour passes between grid_sync_coherent
 // barriers: buffer loads and stores with the agent-scope coherence bit (SC1), which go to
@@ -250,60 +99,6 @@ __device__ __forceinline__ void st_imp(Real* p, Real x) {
   if (Coh) __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   else *p = x;
 }
-
-
-template <typename Real>
-struct GSArgs {
-  ContactSoA<Real> c;
-  Real* body;               // body records by slot
-  const uint32_t* sid;      // slot -> body id (nullptr: identity)
-  const double* v0;         // dim per body
-  const double* w0;         // 3 per body (3D)
-  uint32_t nbodies;
-  uint32_t C;
-  const uint32_t* coloff;   // colour offsets
-  Real* rbest;              // 3 per contact
-  double* partial;          // per-workgroup residual partials
-  StepCounters* ctr;
-  uint32_t* bar;             // grid barrier state
-  uint32_t max_iters;
-  uint32_t eval_every;
-  double tol;
-  int phase;                // 0: only phase, 1: FP32 phase, 2: FP64 polish after FP32
-  int apply_init;           // reset velocities to v0 and apply the records' impulses
-  uint32_t* lmap;           // per body slot: owning endpoint in the LDS solve (all ones when idle)
-  uint32_t tail_col;        // colours [tail_col, ncolours) are swept by workgroup 0 alone (small)
-  // ensembles (else cscene == nullptr): per contact (colour order) its scene; per scene the
-  // residual of the last two evaluations (max ||FB||^2 bits, double-buffered) and the sweep
-  // at which it met the tolerance (kNoBody until then). A scene that meets the tolerance is
-  // frozen: its contacts are skipped until the solve ends.
-  const uint32_t* cscene;
-  unsigned long long* scene_acc;  // 2 x nscenes
-  uint32_t* scene_sweeps;         // nscenes
-  uint32_t nscenes;
-  // ensembles: the contacts of scenes not yet frozen, compacted colour by colour once
-  // enough scenes have frozen (two lists of C entries, alternately rebuilt), and per-colour
-  // per-workgroup counts for the compaction (kMaxColours x gridDim); nullptr: no compaction
-  uint32_t* act_idx;
-  uint32_t* act_part;
-  // FP32 phase of one scene: contacts whose residual at the last full evaluation was at
-  // least the capture threshold (up to kViolCap, in any order; counts of the two last
-  // evaluations, double-buffered), and the word through which workgroup 0 tells the others
-  // that one of them is still above the stopping value (nullptr: every sweep is evaluated)
-  uint32_t* viol;  // 2 counts, then kViolCap contacts
-  uint32_t* vflag;
-  // One scene with coherent passes on several workgroups: colours [comp_col, ncolours) are
-  // swept as connected components (contacts linked through shared bodies), every component
-  // by one workgroup through its L2. comp_parent: per body slot, its parent in a union-find
-  // forest over the bodies of those contacts; comp_cnt: an overflow flag, then per
-  // workgroup the number of contacts it was given; comp_list: per workgroup kCompCap
-  // contacts. comp_parent == nullptr: no component phase.
-  uint32_t* comp_parent;
-  uint32_t* comp_cnt;
-  uint32_t* comp_list;
-  uint32_t comp_col;
-  int comp_lds;  // hold a workgroup's components in LDS when they fit (else through its L2)
-};
 
 
 // True if contact k belongs to a scene whose last evaluated residual is below stop.
@@ -447,15 +242,6 @@ __device__ void compact_active(const GSArgs<Real>& A, const uint32_t* src, const
   grid_barrier(A.bar);
 }
 
-// A contact's record and impulse, loaded ahead of its colour pass. Only the thread that
-// updates a contact ever writes its impulse, and the record is read-only during the
-// solve, so the load may be issued before the grid barrier that opens the pass.
-template <int D, typename Real>
-struct Loaded {
-  Rec<D, Real> R;
-  Real r[3];
-};
-
 template <int D, typename Real, bool Coh = false>
 __device__ __forceinline__ void load_contact(const GSArgs<Real>& A, uint32_t k, Loaded<D, Real>& L) {
   load_rec<D, Real>(A.c, k, L.R);
@@ -463,78 +249,6 @@ __device__ __forceinline__ void load_contact(const GSArgs<Real>& A, uint32_t k, 
   L.r[0] = ld_imp<Coh>(rp);
   L.r[1] = ld_imp<Coh>(rp + 1);
   L.r[2] = ld_imp<Coh>(rp + 2);
-}
-
-// One contact of a colour pass from its loaded record, on body vectors ia and ib (3D: ia + 1
-// and ib + 1 are the angular halves of the same records) read and written through ld/st,
-// the new impulse stored through st_r(d, x). copy_best: first store the contact's impulse
-// as it was before this sweep into rbest (the previous sweep's iterate was the best one so
-// far). Every update of a contact goes through this code, wherever its bodies are held.
-template <int D, typename Real, typename Ld, typename St, typename StR>
-__device__ __forceinline__ void update_core(const GSArgs<Real>& A, uint32_t k, const Loaded<D, Real>& L, bool init,
-                                            bool copy_best, size_t ia, size_t ib, Ld&& ld, St&& st, StR&& st_r) {
-  using V = typename Vec4<Real>::type;
-  const Rec<D, Real>& R = L.R;
-  const bool hasb = R.b != kNoBody;
-  V va = ld(ia), wa = {0, 0, 0, 0}, vb = {0, 0, 0, 0}, wb = {0, 0, 0, 0};
-  if (D == 3) wa = ld(ia + 1);
-  if (hasb) {
-    vb = ld(ib);
-    if (D == 3) wb = ld(ib + 1);
-  }
-  const Real r[3] = {L.r[0], L.r[1], L.r[2]};
-  if (copy_best) {
-    Real* rb = A.rbest + 3 * (size_t)k;
-    rb[0] = r[0];
-    rb[1] = r[1];
-    rb[2] = r[2];
-  }
-  Real dr[3];
-  if (init) {
-    dr[0] = r[0];
-    dr[1] = r[1];
-    dr[2] = r[2];
-  } else {
-    Real u[3], rn[3];
-    rel_vel<D, Real, Real>(R, va, wa, vb, wb, u);
-    local_solve<D, Real>(R, u, r, rn);
-    dr[0] = rn[0] - r[0];
-    dr[1] = rn[1] - r[1];
-    dr[2] = rn[2] - r[2];
-    st_r(0, rn[0]);
-    st_r(1, rn[1]);
-    if (D == 3) st_r(2, rn[2]);
-  }
-  Real Pi[3];  // the impulse increment in world coordinates
-#pragma unroll
-  for (int d = 0; d < 3; ++d) Pi[d] = R.n[d] * dr[0] + R.t[d] * dr[D - 1] + ((D == 3) ? R.s[d] * dr[1] : (Real)0);
-  va.x += va.w * Pi[0];
-  va.y += va.w * Pi[1];
-  va.z += va.w * Pi[2];
-  st(ia, va);
-  Real tau[3];
-  if (D == 3) {
-#pragma unroll
-    for (int d = 0; d < 3; ++d) tau[d] = dr[1] * R.t[d] - dr[2] * R.s[d];
-    const Real ka = -R.la * wa.w;
-    wa.x += ka * tau[0];
-    wa.y += ka * tau[1];
-    wa.z += ka * tau[2];
-    st(ia + 1, wa);
-  }
-  if (hasb) {
-    vb.x -= vb.w * Pi[0];
-    vb.y -= vb.w * Pi[1];
-    vb.z -= vb.w * Pi[2];
-    st(ib, vb);
-    if (D == 3) {
-      const Real kb = R.lb * wb.w;
-      wb.x -= kb * tau[0];
-      wb.y -= kb * tau[1];
-      wb.z -= kb * tau[2];
-      st(ib + 1, wb);
-    }
-  }
 }
 
 // One contact of a colour pass on the body records in global memory (Coh: coherently).
@@ -545,7 +259,7 @@ __device__ __forceinline__ void update(const GSArgs<Real>& A, uint32_t k, const 
   V* bv = reinterpret_cast<V*>(A.body);
   Real* rp = A.c.r + 3 * (size_t)k;
   update_core<D, Real>(
-      A, k, L, init, copy_best, (size_t)kBodyVecs<D> * L.R.a, (size_t)kBodyVecs<D> * L.R.b,
+      L, init, copy_best ? A.rbest + 3 * (size_t)k : nullptr, (size_t)kBodyVecs<D> * L.R.a, (size_t)kBodyVecs<D> * L.R.b,
       [&](size_t i) { return Coh ? P.ld(i) : bv[i]; },
       [&](size_t i, const V& x) {
         if (Coh) P.st(i, x);
@@ -1034,7 +748,7 @@ __device__ void comp_lds_sweep(const GSArgs<Real>& A, const uint32_t* s_list, co
       ld.r[2] = rl[2];
       Real* rp = A.c.r + 3 * (size_t)k;
       update_core<D, Real>(
-          A, k, ld, false, copy, (size_t)kBodyVecs<D> * ea, (size_t)kBodyVecs<D> * (eb == kNoLocal ? 0u : eb),
+          ld, false, copy ? A.rbest + 3 * (size_t)k : nullptr, (size_t)kBodyVecs<D> * ea, (size_t)kBodyVecs<D> * (eb == kNoLocal ? 0u : eb),
           [&](size_t i) { return L.body[i]; }, [&](size_t i, const V& x) { L.body[i] = x; },
           [&](int d, Real x) {
             rl[d] = x;
@@ -1768,6 +1482,37 @@ static hipError_t tune_after_solve(scx_ctx* c) {
   return e;
 }
 
+// One-workgroup sweeps with the bodies in LDS (k_gs_wg): their time per sweep grows with the
+// contacts (one CU). FP64 sweeps with their residuals: 2,600 sphere contacts 24 us (72 with
+// k_gs), 6,857 circle contacts 26 us (35). The LDS limit leaves room for the kernel's static
+// arrays.
+constexpr size_t kWgLdsMax = 152 * 1024;
+constexpr uint32_t kWgMaxContacts = 3072;
+
+// Their buffers, in the context's arena (grown when a larger contact set takes the path).
+template <int D, typename Real>
+static hipError_t wg_buffers(scx_ctx* c, uint32_t C, uint32_t nbodies, WgBufs<Real>& W) {
+  const size_t rec = sizeof(Real) * (D == 3 ? 16 : 8) * (size_t)C, r = sizeof(Real) * (D == 3 ? 4 : 2) * (size_t)C;
+  const size_t ids = sizeof(uint32_t) * (size_t)((C + 3) / 4 * 4), slot = sizeof(uint32_t) * (size_t)nbodies;
+  const size_t need = rec + r + ids + slot;
+  DeviceBuffers& d = c->d;
+  if (need > d.cap_wg) {
+    // the buffer may still be in use by an earlier launch on the stream; hipFree waits for it
+    if (d.wg_arena) (void)hipFree(d.wg_arena);
+    d.wg_arena = nullptr;
+    d.cap_wg = 0;
+    const hipError_t e = hipMalloc((void**)&d.wg_arena, need + need / 4);
+    if (e != hipSuccess) return e;
+    d.cap_wg = need + need / 4;
+  }
+  unsigned char* p = d.wg_arena;
+  W.rec = reinterpret_cast<Real*>(p);
+  W.r = reinterpret_cast<Real*>(p + rec);
+  W.ids = reinterpret_cast<uint32_t*>(p + rec + r);
+  W.slot = reinterpret_cast<uint32_t*>(p + rec + r + ids);
+  return hipSuccess;
+}
+
 template <int D, typename Real>
 static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint32_t* col_off) {
   // Tail: the suffix of colours no wider than one workgroup, swept by one workgroup (no
@@ -1812,11 +1557,16 @@ static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint
   const size_t lds = LdsLayout<D, Real>::bytes(A.C);
   const bool lds_path = std::min(max_blocks, model) <= 1 && c->force_blocks <= 0 && lds <= kGSLdsMax && A.lmap &&
                         !A.cscene;
-  // the autotuner picks among widths around the model's (not for the LDS solve)
+  // bodies in one workgroup's LDS: up to kWgMaxContacts contacts
+  const size_t wg_lds = wg_lds_bytes<D, Real>(A.nbodies, A.C);
+  const bool one_scene = c->force_blocks <= 0 && !A.cscene && !lds_path;
+  const bool wg = one_scene && c->wg_sweeps && A.lmap && A.C <= kWgMaxContacts && wg_lds <= kWgLdsMax;
+  // the autotuner picks among widths around the model's (not for the solves of one workgroup)
   const int phase = std::is_same<Real, double>::value ? 1 : 0;
-  const bool tune = c->tuner.enabled && c->force_blocks <= 0 && !lds_path && !c->coop_unavailable;
+  const bool tune = c->tuner.enabled && c->force_blocks <= 0 && !lds_path && !wg && !c->coop_unavailable;
   const int want = tune ? tune_pick(c, phase, tune_key(D, phase, A.cscene != nullptr, A.C, nw), model, max_blocks)
                         : model;
+  // (the launch shape of the sweeps with barriers, whose early skips k_gs_wg reproduces)
   const int blocks = c->coop_unavailable ? 1 : std::max(1, std::min(max_blocks, want));
   A.tail_col = (blocks > 1) ? (uint32_t)tail : (uint32_t)kMaxColours;
   // the component phase needs several workgroups, and lists that hold the phase's contacts
@@ -1824,6 +1574,14 @@ static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint
   // overflows a list falls back to it by itself)
   if (blocks > 1 && comp < ncol && comp_contacts <= (uint64_t)blocks * kCompCap / 2) A.comp_col = (uint32_t)comp;
   else A.comp_parent = nullptr;
+  const int skip_early = blocks > 1 && (tail < ncol || A.comp_parent) ? 1 : 0;
+  if (wg) {
+    WgBufs<Real> W;
+    hipError_t e = wg_buffers<D, Real>(c, A.C, (uint32_t)std::min<uint64_t>(A.nbodies, 2ull * A.C), W);
+    if (e != hipSuccess) return e;
+    W.skip_early = skip_early;
+    return launch_gs_wg<D, Real>(A, W, c->stream);
+  }
   if (lds_path) {
     // the whole solve in one workgroup's LDS
     hipError_t e = hipFuncSetAttribute((const void*)k_gs_lds<D, Real>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1835,8 +1593,9 @@ static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint
   void* args[] = {&A};
   hipError_t e = tune ? hipEventRecord(c->tuner.pend[phase].ev[0], c->stream) : hipSuccess;
   if (e != hipSuccess) return e;
-  const void* fn = coh ? (const void*)k_gs<D, Real, true> : (const void*)k_gs<D, Real, false>;
   bool launched = false;
+  c->barrier_sweeps = true;
+  const void* fn = coh ? (const void*)k_gs<D, Real, true> : (const void*)k_gs<D, Real, false>;
   e = launch_cooperative(c, fn, blocks, kGSBlock, args, 0, c->stream, &launched);
   if (e == hipSuccess && !launched) {
     // one workgroup (chosen, or after a refused cooperative launch: see
@@ -1885,6 +1644,7 @@ static hipError_t solve_dim(scx_ctx* c, uint32_t C, const uint32_t* col_off, con
   timing_mark(c, "gs_init");
   if (e != hipSuccess || C == 0) return e;
   const bool ens = c->nscenes > 0;
+  c->barrier_sweeps = false;
   if (ens) {
     k_contact_scene<<<(C + kBlock - 1) / kBlock, kBlock, 0, s>>>(C, c->d.c64.a, c->d.sid, c->d.bscene, c->d.cscene);
     e = hipGetLastError();

@@ -1,0 +1,76 @@
+"""The sweeps of one workgroup with the bodies in LDS (k_gs_wg) against the sweeps with grid
+barriers (SCX_WG_SWEEPS=0): every contact is updated in its colour's turn with the same expressions, so steps are the
+same bit for bit -- positions, velocities, impulses, sweep counts, residuals -- in FP64 and in
+FP32 with the FP64 polish, converging, ending at a sweep limit with the best iterate, through
+the FP32 stagnation test, with sparse residual checks; for contact sets around the passes of a
+workgroup and the smallest and largest each path takes.
+"""
+
+import numpy as np
+import pytest
+
+import scisim_amd as scx
+from scisim_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def _scene(kind):
+    if kind == "one":  # one sphere on the floor: a single contact, a single colour
+        s = scenes.spheres_pile(n=1, base=1.0, seed=3)
+    elif kind == "circles":
+        s = scenes.ball2d_rsa(n=6000, seed=11)
+        s["v"] = np.random.default_rng(11).normal(0.0, 2.0, s["v"].size)
+    elif kind == "lattice":
+        s = scenes.ball2d_lattice(m=40, side=6.25, r=0.05, vstd=0.5, seed=2)
+    else:
+        s = scenes.spheres_pile(n=int(kind), seed=13)
+    return s
+
+
+def _run(monkeypatch, s, path, prm, steps):
+    monkeypatch.setenv("SCX_WG_SWEEPS", "1" if path == "wg" else "0")
+    D = s["dim"]
+    ctx = scx.Context(D, s["r"].size, max_planes=8)
+    try:
+        ctx.set_planes(s["px"], s["pn"])
+        ctx.set_bodies(s["q"], s["v"], s["r"], s["m"], inertia=s.get("inertia"))
+        out = []
+        for _ in range(steps):
+            st = ctx.step(scx.step_params(**prm))
+            con = ctx.contacts()
+            out.append((st, *ctx.get_state(), con["alpha"], con["beta"]))
+        return out
+    finally:
+        ctx.close()
+
+
+def _params(s, precision, limit):
+    D = s["dim"]
+    prm = dict(dt=0.005, g=[0.0, -9.81] if D == 2 else [0.0, -9.81, 0.0], mu=0.4, CoR=0.0,
+               integrator=0 if D == 2 else 1, precision=scx.FP64 if precision == "fp64" else scx.FP32_POLISH,
+               warm_start=scx.WARM_TRANSPORT)
+    prm.update({"converged": dict(tol=1e-7, max_iters=3000, eval_every=1),
+                "limit": dict(tol=1e-13, max_iters=150, eval_every=1),
+                "sparse": dict(tol=1e-10, max_iters=310, eval_every=20),
+                "stagnates": dict(tol=1e-12, max_iters=3000, eval_every=1, warm_start=scx.WARM_NONE)}[limit])
+    return prm
+
+
+def _same(ref, got):
+    for a, b in zip(ref, got):
+        print(a[0], flush=True)
+        for key in ("ncontacts", "ncolours", "sweeps", "sweeps_fp32", "error", "succeeded"):
+            assert a[0][key] == b[0][key], key
+        for x, y in zip(a[1:], b[1:]):
+            assert x is None or np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("kind", ["one", "circles", "lattice", "60", "700", "2500"])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("limit", ["converged", "limit", "sparse", "stagnates"])
+def test_one_workgroup(monkeypatch, kind, precision, limit):
+    print("case", kind, precision, limit, flush=True)
+    s = _scene(kind)
+    prm = _params(s, precision, limit)
+    _same(_run(monkeypatch, s, "", prm, 3), _run(monkeypatch, s, "wg", prm, 3))
