@@ -261,6 +261,9 @@ void free_all(scx_ctx* c) {
   dfree(&d.comp_cnt);
   dfree(&d.comp_list);
   dfree(&d.wg_arena);
+  dfree(&d.flow_links);
+  dfree(&d.flow_rec);
+  dfree(&d.flow_slots);
   uint32_t* u32[] = {d.cells, d.ent, d.pcount, d.scan_tmp, d.pa, d.pb, d.ca, d.cb, d.mbcount, d.deg, d.adj,
                      d.perm, d.coloff};
   for (uint32_t* p : u32)
@@ -474,6 +477,7 @@ int step_once(scx_ctx* c, const scx_step_params* p, scx_step_stats* st, bool wan
     HIPC(hipMemcpyAsync(d.ctr_host, d.ctr, sizeof(StepCounters), hipMemcpyDeviceToHost, s));
     HIPC(hipStreamSynchronize(s));
     c->last_ncolours = d.ctr_host->ncolours;
+    if (d.ctr_host->overflow & 16u) return fail(c, SCX_E_HIP, "a wait between sweep workgroups ran out");
     comp_adapt_share(c, *d.ctr_host);
     if (c->violator_skip == 2 && p->precision == SCX_PRECISION_FP32_POLISH && c->nscenes == 0 &&
         d.ctr_host->sweeps_fp32 >= 64 && d.ctr_host->evals_skipped == 0)
@@ -615,13 +619,14 @@ int scx_create(const scx_config* cfg, scx_ctx** out) {
       c->comp_share = std::min(100.0, std::max(1.0, atof(env)));
       c->comp_adapt = false;
     }
-    // SCX_WG_SWEEPS=0: contact sets whose bodies one workgroup's LDS holds are swept with
-    // grid barriers all the same (the same iterates bit for bit; for A/B measurements and
-    // tests). The switches of the sweeps with barriers above keep a context on them unless
-    // this one says otherwise.
+    // SCX_WG_SWEEPS=0: contact sets whose bodies one workgroup's LDS holds are swept on several
+    // workgroups all the same; SCX_FLOW_SWEEPS=0: larger ones with grid barriers between the
+    // colours (the same iterates bit for bit; for A/B measurements and tests). The switches of
+    // the sweeps with barriers above keep a context on them unless these two say otherwise.
     if (getenv("SCX_COMPONENT_SWEEPS") || getenv("SCX_COMPONENT_PERCENT") || getenv("SCX_COHERENT_SWEEPS"))
-      c->wg_sweeps = false;
+      c->wg_sweeps = c->flow_sweeps = false;
     if (const char* env = getenv("SCX_WG_SWEEPS")) c->wg_sweeps = atoi(env) != 0;
+    if (const char* env = getenv("SCX_FLOW_SWEEPS")) c->flow_sweeps = atoi(env) != 0;
     if ((e = dalloc(&d.partial, (size_t)std::max(c->gs_blocks, 1) + 1)) != hipSuccess ||
         (e = dalloc(&d.viol, (size_t)3 + kViolCap)) != hipSuccess ||
         (e = dalloc(&d.comp_cnt, (size_t)std::max(c->gs_blocks, 1) + 1)) != hipSuccess ||
@@ -1177,6 +1182,7 @@ int scx_friction_solve(scx_ctx* c, uint32_t nbodies, const double* m, const doub
   }
   HIPC(hipMemcpyAsync(d.ctr_host, d.ctr, sizeof(StepCounters), hipMemcpyDeviceToHost, s));
   HIPC(hipStreamSynchronize(s));
+  if (d.ctr_host->overflow & 16u) return fail(c, SCX_E_HIP, "a wait between sweep workgroups ran out");
   for (uint32_t i = 0; i < nbodies; ++i) {
     if (v2)
       for (int q = 0; q < D; ++q) v2[(size_t)D * i + q] = bv[rec * i + q];

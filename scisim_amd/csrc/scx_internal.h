@@ -56,7 +56,7 @@ struct GridParams {
 // Device-side counters of one step, read back by the host at the sync points.
 struct StepCounters {
   unsigned long long nentries;   // grid entries
-  uint32_t overflow;             // bit 0 entries, bit 1 pairs, bit 2 contacts, bit 3 colours
+  uint32_t overflow;             // bit 0 entries, bit 1 pairs, bit 2 contacts, bit 3 colours, bit 4 a sweep wait ran out
   uint32_t ncolours;
   uint32_t nrounds;
   uint32_t remaining;            // uncoloured contacts
@@ -205,6 +205,11 @@ struct DeviceBuffers {
   uint32_t* comp_list = nullptr;    // gs_blocks x kCompCap: per-workgroup contacts
   unsigned char* wg_arena = nullptr;  // working memory of the one-workgroup sweeps (cap_wg bytes)
   size_t cap_wg = 0;
+  // sweeps without barriers: links, packed records and impulses, sync words and outbox slots
+  unsigned char* flow_links = nullptr;
+  unsigned char* flow_rec = nullptr;
+  unsigned char* flow_slots = nullptr;
+  size_t cap_flow_links = 0, cap_flow_rec = 0, cap_flow_slots = 0;
   // warm-start cache (previous step's active set, sorted keys + impulses)
   // keys ascend in active-set order: (i << 32 | j) for body pairs, then
   // (1 << 63 | plane << 32 | i) for plane contacts
@@ -282,6 +287,8 @@ struct scx_ctx {
   double comp_ceiling = 100.0;  // below the last share that overflowed (drifts back up)
   bool comp_adapt = true;
   bool barrier_sweeps = false;  // the last solve swept with grid barriers (k_gs)
+  bool flow_sweeps = true;      // one scene: sweep without barriers between the colours (k_gs_flow)
+  uint32_t flow_tag = 1;        // next unused tag of those sweeps' slots
   bool wg_sweeps = true;        // one scene: sweep in one workgroup when its LDS holds the bodies
   // The device's cooperative queues are limited in number (HSA_QUEUE_TYPE_COOPERATIVE,
   // hsa/hsa.h: "Queues of this type may be limited in number"); while another process holds

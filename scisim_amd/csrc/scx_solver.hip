@@ -1482,10 +1482,11 @@ static hipError_t tune_after_solve(scx_ctx* c) {
   return e;
 }
 
-// One-workgroup sweeps with the bodies in LDS (k_gs_wg): their time per sweep grows with the
-// contacts (one CU). FP64 sweeps with their residuals: 2,600 sphere contacts 24 us (72 with
-// k_gs), 6,857 circle contacts 26 us (35). The LDS limit leaves room for the kernel's static
-// arrays.
+// One-workgroup sweeps with the bodies in LDS (k_gs_wg). Their time per sweep grows with the
+// contacts (one CU), that of the sweeps without barriers (k_gs_flow) with the colours: FP64
+// sweeps of 2,600 sphere contacts with their residuals take 24 us in one workgroup and 31 us
+// on 32 to 256 workgroups, of 3,347 sphere contacts 18.7 and 17.7 to 19.4 us, of 6,857 circle
+// contacts 26 and 18 us. The LDS limit leaves room for the kernel's static arrays.
 constexpr size_t kWgLdsMax = 152 * 1024;
 constexpr uint32_t kWgMaxContacts = 3072;
 
@@ -1513,8 +1514,76 @@ static hipError_t wg_buffers(scx_ctx* c, uint32_t C, uint32_t nbodies, WgBufs<Re
   return hipSuccess;
 }
 
+// Sweeps without barriers between the colours (k_gs_flow): their buffers, in the context's
+// arenas (grown when a larger contact set takes the path), and the links of this contact set
+// (shared by the two phases of a solve).
+constexpr uint32_t kFlowTagMax = 1u << 30;
+// Above kFlowMaxContacts the scattered 16-byte gathers of the slots fill the L2s' request
+// rate, and the sweeps with barriers, whose late colours stay in LDS, are as fast (420,000
+// sphere contacts: 50 against 58 us per FP32 sweep, but 200 against 125 us in FP64). Workgroups:
+// 128 contacts each up to the whole chip (34,257 sphere contacts: 21.0, 20.0 and 19.8 us per FP32
+// sweep on 64, 128 and 256 workgroups; 44.6 with barriers).
+constexpr uint32_t kFlowMinContacts = 1024, kFlowMaxContacts = 1u << 18;
+constexpr uint32_t kFlowContacts = 128;  // contacts of a workgroup
+
+static hipError_t flow_arena(unsigned char** p, size_t* cap, size_t need, hipStream_t s) {
+  if (need <= *cap) return hipSuccess;
+  if (*p) (void)hipFree(*p);  // waits for earlier launches that use it
+  *p = nullptr;
+  *cap = 0;
+  const size_t want = need + need / 4;
+  hipError_t e = hipMalloc((void**)p, want);
+  if (e != hipSuccess) return e;
+  *cap = want;
+  return hipMemsetAsync(*p, 0, want, s);
+}
+
 template <int D, typename Real>
-static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint32_t* col_off) {
+static hipError_t flow_prepare(scx_ctx* c, const GSArgs<Real>& A, bool* linked, FlowBufs<Real>& F) {
+  DeviceBuffers& d = c->d;
+  const size_t C = A.C, n = c->n;
+  const size_t links = sizeof(unsigned long long) * (n + 2) + sizeof(uint32_t) * ((n + 1) / 2 * 2) +
+                       sizeof(uint2) * 3 * C + 256;
+  const size_t rec = sizeof(Real) * (D == 3 ? 16 : 8) * C, r = sizeof(Real) * (D == 3 ? 4 : 2) * C;
+  const size_t slot = (size_t)(D == 3 ? 8 : 4) * sizeof(Real) * 2 * C;  // bytes of the 2 C slots
+  const size_t sync = (size_t)kFlowMaxBlocks * (sizeof(uint32_t) + 16);
+  const unsigned char* old = d.flow_links;
+  hipError_t e = flow_arena(&d.flow_links, &d.cap_flow_links, links, c->stream);
+  if (e == hipSuccess && d.flow_links != old) *linked = false;
+  if (e == hipSuccess) e = flow_arena(&d.flow_rec, &d.cap_flow_rec, rec + r, c->stream);
+  if (e == hipSuccess) e = flow_arena(&d.flow_slots, &d.cap_flow_slots, sync + slot, c->stream);
+  if (e != hipSuccess) return e;
+  const uint32_t tags = A.max_iters + 16;
+  if (c->flow_tag + tags >= kFlowTagMax) {
+    // the tags start over on cleared slots
+    e = hipMemsetAsync(d.flow_slots, 0, d.cap_flow_slots, c->stream);
+    if (e != hipSuccess) return e;
+    c->flow_tag = 1;
+  }
+  F.tag0 = c->flow_tag;
+  c->flow_tag += tags;
+  FlowLinks L;
+  unsigned char* p = d.flow_links;
+  L.mask = reinterpret_cast<unsigned long long*>(p);
+  p += sizeof(unsigned long long) * (n + 2);
+  L.from = reinterpret_cast<uint2*>(p);
+  L.fin = L.from + C;
+  L.table = reinterpret_cast<uint32_t*>(L.fin + C);
+  L.start = L.table + 2 * C;
+  F.from = reinterpret_cast<const uint32_t*>(L.from);
+  F.fin = reinterpret_cast<const uint32_t*>(L.fin);
+  F.rec = reinterpret_cast<Real*>(d.flow_rec);
+  F.r = reinterpret_cast<Real*>(d.flow_rec + rec);
+  F.flags = reinterpret_cast<uint32_t*>(d.flow_slots);
+  F.parts = d.flow_slots + sizeof(uint32_t) * kFlowMaxBlocks;
+  F.slots = d.flow_slots + sync;
+  if (*linked) return hipSuccess;
+  *linked = true;
+  return launch_flow_links(c, A.C, A.c.a, A.c.b, L);
+}
+
+template <int D, typename Real>
+static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint32_t* col_off, bool* linked) {
   // Tail: the suffix of colours no wider than one workgroup, swept by one workgroup (no
   // grid barrier between them) when the launch has several workgroups and the suffix has
   // at least two colours.
@@ -1561,13 +1630,21 @@ static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint
   const size_t wg_lds = wg_lds_bytes<D, Real>(A.nbodies, A.C);
   const bool one_scene = c->force_blocks <= 0 && !A.cscene && !lds_path;
   const bool wg = one_scene && c->wg_sweeps && A.lmap && A.C <= kWgMaxContacts && wg_lds <= kWgLdsMax;
+  // no barriers between the colours: from there to kFlowMaxContacts, while the slots can be
+  // addressed and the tags last
+  const bool flow = one_scene && !wg && c->flow_sweeps && !c->coop_unavailable && max_blocks > 1 &&
+                    A.C >= kFlowMinContacts && A.C <= kFlowMaxContacts && A.max_iters < kFlowTagMax / 4 &&
+                    (uint64_t)A.C * (D == 3 ? 16 : 8) * sizeof(Real) < (1ull << 31);
   // the autotuner picks among widths around the model's (not for the solves of one workgroup)
   const int phase = std::is_same<Real, double>::value ? 1 : 0;
   const bool tune = c->tuner.enabled && c->force_blocks <= 0 && !lds_path && !wg && !c->coop_unavailable;
-  const int want = tune ? tune_pick(c, phase, tune_key(D, phase, A.cscene != nullptr, A.C, nw), model, max_blocks)
-                        : model;
-  // (the launch shape of the sweeps with barriers, whose early skips k_gs_wg reproduces)
-  const int blocks = c->coop_unavailable ? 1 : std::max(1, std::min(max_blocks, want));
+  const int flow_most = std::min(max_blocks, kFlowMaxBlocks);
+  const int width = flow ? std::max(2, std::min((int)((A.C + kFlowContacts - 1) / kFlowContacts), flow_most)) : model;
+  const int want = tune ? tune_pick(c, phase, tune_key(D, phase, A.cscene != nullptr, A.C, nw), width,
+                                    flow ? flow_most : max_blocks)
+                        : width;
+  // (the launch shape of the sweeps with barriers, whose early skips the others reproduce)
+  const int blocks = c->coop_unavailable ? 1 : std::max(1, std::min(max_blocks, flow ? model : want));
   A.tail_col = (blocks > 1) ? (uint32_t)tail : (uint32_t)kMaxColours;
   // the component phase needs several workgroups, and lists that hold the phase's contacts
   // with room for an uneven split (else the tail as before; a launch whose split still
@@ -1594,6 +1671,18 @@ static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint
   hipError_t e = tune ? hipEventRecord(c->tuner.pend[phase].ev[0], c->stream) : hipSuccess;
   if (e != hipSuccess) return e;
   bool launched = false;
+  if (flow) {
+    FlowBufs<Real> F;
+    e = flow_prepare<D, Real>(c, A, linked, F);
+    if (e != hipSuccess) return e;
+    F.skip_early = skip_early;
+    int fb = std::max(2, std::min(want, flow_most));
+    // SCX_FLOW_BLOCKS: a fixed workgroup count (the results do not depend on it; for tests)
+    if (const char* env = getenv("SCX_FLOW_BLOCKS")) fb = std::max(2, std::min(atoi(env), flow_most));
+    e = launch_gs_flow<D, Real>(c, A, F, fb, &launched);
+    if (e == hipSuccess && launched && tune) e = hipEventRecord(c->tuner.pend[phase].ev[1], c->stream);
+    if (e != hipSuccess || launched) return e;
+  }
   c->barrier_sweeps = true;
   const void* fn = coh ? (const void*)k_gs<D, Real, true> : (const void*)k_gs<D, Real, false>;
   e = launch_cooperative(c, fn, blocks, kGSBlock, args, 0, c->stream, &launched);
@@ -1645,6 +1734,7 @@ static hipError_t solve_dim(scx_ctx* c, uint32_t C, const uint32_t* col_off, con
   if (e != hipSuccess || C == 0) return e;
   const bool ens = c->nscenes > 0;
   c->barrier_sweeps = false;
+  bool linked = false;  // the links of this contact set have been made
   if (ens) {
     k_contact_scene<<<(C + kBlock - 1) / kBlock, kBlock, 0, s>>>(C, c->d.c64.a, c->d.sid, c->d.bscene, c->d.cscene);
     e = hipGetLastError();
@@ -1679,7 +1769,7 @@ static hipError_t solve_dim(scx_ctx* c, uint32_t C, const uint32_t* col_off, con
         A.act_part = c->d.act_part;
       }
     }
-    e = coop_gs<D, float>(c, A, c->gs_blocks, col_off);
+    e = coop_gs<D, float>(c, A, c->gs_blocks, col_off, &linked);
     if (e != hipSuccess) return e;
     timing_mark(c, "gs_fp32");
     const uint32_t nr = (3 * C + kBlock - 1) / kBlock;
@@ -1714,7 +1804,7 @@ static hipError_t solve_dim(scx_ctx* c, uint32_t C, const uint32_t* col_off, con
       B.act_part = c->d.act_part;
     }
   }
-  e = coop_gs<D, double>(c, B, c->gs_blocks, col_off);
+  e = coop_gs<D, double>(c, B, c->gs_blocks, col_off, &linked);
   if (e != hipSuccess) return e;
   return tune_after_solve(c);
 }

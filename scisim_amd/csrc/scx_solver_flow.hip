@@ -1,0 +1,729 @@
+// scx_solver_flow.hip -- the sweeps of a contact set on many workgroups without barriers
+// between the colours: a contact waits only for the contacts before it on its own two bodies.
+//
+// What bounds the sweeps of a few thousand to a few hundred thousand contacts is neither
+// arithmetic nor memory but the exchange of bodies between the colours. With a grid barrier
+// per colour an interval costs 8 to 13 us (coherent gathers, the completion of scattered
+// coherent stores, the arrival and the slowest workgroup); a 16-byte store that carries its
+// own tag is seen by a polling load on another XCD after 0.4 to 0.8 us. So every contact owns
+// an outbox slot per body: it writes the body's velocities there after its update, in 16-byte
+// pieces that each end in the sweep's tag, and the next contact on that body (the order on a
+// body is the colour order, cyclic over the sweeps) polls that slot until the tag is the one
+// it waits for. No store is waited for, nothing is read that has not been written, and the
+// stores of a wave are contiguous.
+//
+// The iterates are those of the colour passes bit for bit: the order of the contacts on
+// every body is the colour order, and a contact reads nothing but its own two bodies.
+// Progress: the launch is cooperative (every workgroup resident), a wave takes its contacts
+// in colour order, and a contact waits only for contacts of lower colours of its sweep or of
+// the sweep before; the order (sweep, colour) has no cycle. A slot is written again only by
+// the same contact one sweep later, which follows its reader on the body's cycle. Every wait
+// also ends after kSpinLimit polls: the workgroup then leaves its sweeps and the step fails.
+#pragma clang fp contract(on)
+
+#include "scx_device.h"
+#include "scx_internal.h"
+#include "scx_sweep.h"
+
+#include <algorithm>
+
+namespace scx {
+
+typedef uint32_t u32x4f __attribute__((ext_vector_type(4)));
+
+constexpr int kFlowThreads = 512;
+constexpr uint32_t kSpinLimit = 1u << 21;  // about a second of polls
+constexpr size_t kFlowLdsMax = 150 * 1024;
+constexpr int kFlowAux = 16;               // agent scope (SC1)
+
+// 16-byte pieces of a slot: three words of velocity and the tag.
+template <int D, typename Real>
+constexpr int kSlotPieces = (D == 3) ? (sizeof(Real) == 8 ? 4 : 2) : (sizeof(Real) == 8 ? 2 : 1);
+
+template <int D, typename Real>
+struct FlowPort {
+  using V = typename Vec4<Real>::type;
+  static constexpr int NP = kSlotPieces<D, Real>;
+  static constexpr int NR = (D == 3) ? 6 : 2;               // Reals of a body
+  static constexpr int NW = NR * (int)sizeof(Real) / 4;     // their words
+  __amdgpu_buffer_rsrc_t rs;
+
+  struct Raw {
+    u32x4f p[NP];
+  };
+
+  __device__ __forceinline__ void ld(uint32_t slot, Raw& x) const {
+    const uint32_t o = slot * (uint32_t)(16 * NP);
+#pragma unroll
+    for (int i = 0; i < NP; ++i) x.p[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, o + 16u * i, 0, kFlowAux);
+  }
+  __device__ __forceinline__ uint32_t tag(uint32_t slot) const {  // of its last piece
+    return __builtin_amdgcn_raw_buffer_load_b32(rs, slot * (uint32_t)(16 * NP) + 16u * (NP - 1) + 12u, 0, kFlowAux);
+  }
+  __device__ __forceinline__ static bool is(const Raw& x, uint32_t tag) {
+    bool ok = true;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) ok = ok && x.p[i][3] == tag;
+    return ok;
+  }
+  __device__ __forceinline__ static bool beyond(const Raw& x, uint32_t tag) {
+    bool b = false;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) b = b || (int32_t)(x.p[i][3] - tag) > 0;
+    return b;
+  }
+  __device__ __forceinline__ static void unpack(const Raw& x, Real im, Real ii, V& v, V& w) {
+    uint32_t u[3 * NP];
+#pragma unroll
+    for (int i = 0; i < 3 * NP; ++i) u[i] = x.p[i / 3][i % 3];
+    Real r[NR];
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      if constexpr (sizeof(Real) == 8)
+        r[i] = __longlong_as_double((long long)(((unsigned long long)u[2 * i + 1] << 32) | u[2 * i]));
+      else
+        r[i] = __uint_as_float(u[i]);
+    }
+    if constexpr (D == 3) {
+      v = V{r[0], r[1], r[2], im};
+      w = V{r[3], r[4], r[5], ii};
+    } else {
+      v = V{r[0], r[1], (Real)0, im};
+      w = V{0, 0, 0, 0};
+    }
+  }
+  __device__ __forceinline__ void st(uint32_t slot, const V& v, const V& w, uint32_t tag) const {
+    Real r[NR];
+    if constexpr (D == 3) {
+      r[0] = v.x, r[1] = v.y, r[2] = v.z, r[3] = w.x, r[4] = w.y, r[5] = w.z;
+    } else {
+      r[0] = v.x, r[1] = v.y;
+    }
+    uint32_t u[3 * NP];
+#pragma unroll
+    for (int i = 0; i < 3 * NP; ++i) u[i] = 0;
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      if constexpr (sizeof(Real) == 8) {
+        const unsigned long long b = (unsigned long long)__double_as_longlong(r[i]);
+        u[2 * i] = (uint32_t)b;
+        u[2 * i + 1] = (uint32_t)(b >> 32);
+      } else {
+        u[i] = __float_as_uint(r[i]);
+      }
+    }
+    const uint32_t o = slot * (uint32_t)(16 * NP);
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const u32x4f x = {u[3 * i], u[3 * i + 1], u[3 * i + 2], tag};
+      __builtin_amdgcn_raw_buffer_store_b128(x, rs, o + 16u * i, 0, kFlowAux);
+    }
+  }
+};
+
+// A contact ready to be updated: its record and impulse, and where its bodies come from
+// (slot << 1 | 1 when the slot is the one of the sweep before).
+template <int D, typename Real>
+struct FlowContact {
+  typename Vec4<Real>::type g[kRecGroups<D>];
+  Real r[3];
+  uint32_t from_a, from_b;  // from_b == kNoBody: a plane
+};
+
+// The solve of k_gs for one scene, step for step (phases, stopping rule, best iterate,
+// stagnation, skipped evaluations).
+template <int D, typename Real>
+__global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBufs<Real> F) {
+  using V = typename Vec4<Real>::type;
+  using V2 = typename Vec2<Real>::type;
+  using Port = FlowPort<D, Real>;
+  using Raw = typename Port::Raw;
+  constexpr int kWaves = kFlowThreads / 64;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  __shared__ uint32_t s_lo[kMaxColours], s_hi[kMaxColours];  // this workgroup's contacts of each colour
+  __shared__ uint32_t s_at[kMaxColours];  // the first one's place in the workgroup's list
+  __shared__ double s_red[kWaves];
+  __shared__ uint32_t s_flag[2], s_skip[2], s_dead;
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  const uint32_t C = A.C, G = gridDim.x;
+  const uint32_t wg = xcd_block();  // neighbouring ranges on one XCD
+  const uint32_t ncol = A.ctr->ncolours;
+  for (uint32_t c = tid; c < ncol; c += kFlowThreads) {
+    const uint32_t o = A.coloff[c], n = A.coloff[c + 1] - o;
+    s_lo[c] = o + (uint32_t)((uint64_t)n * wg / G);
+    s_hi[c] = o + (uint32_t)((uint64_t)n * (wg + 1) / G);
+  }
+  if (tid == 0) s_flag[0] = s_flag[1] = s_skip[0] = s_skip[1] = s_dead = 0;
+  __syncthreads();
+  if (tid == 0) {
+    uint32_t n = 0;
+    for (uint32_t c = 0; c < ncol; ++c) {
+      s_at[c] = n;
+      n += s_hi[c] - s_lo[c];
+    }
+  }
+  __syncthreads();
+  // The first kept contacts of the workgroup's list (its wide colours) keep their records,
+  // impulses and links in LDS.
+  const uint32_t kept = F.kept;
+  V* l_rec = reinterpret_cast<V*>(lds);
+  uint2* l_from = reinterpret_cast<uint2*>(l_rec + (size_t)kRecGroups<D> * kept);
+  Real* l_r = reinterpret_cast<Real*>(l_from + kept);
+  Port P;
+  P.rs = __builtin_amdgcn_make_buffer_rsrc(F.slots, (short)0, (int)(2u * C * (uint32_t)(16 * Port::NP)), 0x00020000);
+  const __amdgpu_buffer_rsrc_t frs = __builtin_amdgcn_make_buffer_rsrc(F.flags, (short)0, (int)(4u * kFlowMaxBlocks), 0x00020000);
+  const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(F.parts, (short)0, (int)(16u * kFlowMaxBlocks), 0x00020000);
+  uint32_t tag = F.tag0;  // of the sweep under way
+  bool dead = false;      // a wait of this wave ran out
+
+  // contact j, entry i of the workgroup's list
+  auto load = [&](uint32_t j, uint32_t i, FlowContact<D, Real>& L) {
+    if (i < kept) {
+#pragma unroll
+      for (int g = 0; g < kRecGroups<D>; ++g) L.g[g] = l_rec[(size_t)g * kept + i];
+      const uint2 f = l_from[i];
+      L.from_a = f.x;
+      L.from_b = f.y;
+#pragma unroll
+      for (int d = 0; d < D; ++d) L.r[d] = l_r[(size_t)d * kept + i];
+      if (D == 2) L.r[2] = 0;
+      return;
+    }
+    const V* rec = reinterpret_cast<const V*>(F.rec);
+#pragma unroll
+    for (int g = 0; g < kRecGroups<D>; ++g) L.g[g] = rec[(size_t)g * C + j];
+    const uint2 f = reinterpret_cast<const uint2*>(F.from)[j];
+    L.from_a = f.x;
+    L.from_b = f.y;
+    if constexpr (D == 3) {
+      const V r = reinterpret_cast<const V*>(F.r)[j];
+      L.r[0] = r.x, L.r[1] = r.y, L.r[2] = r.z;
+    } else {
+      const V2 r = reinterpret_cast<const V2*>(F.r)[j];
+      L.r[0] = r.x, L.r[1] = r.y, L.r[2] = 0;
+    }
+  };
+  auto store_r = [&](uint32_t j, uint32_t i, const Real* r) {
+    if (i < kept) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) l_r[(size_t)d * kept + i] = r[d];
+    } else if constexpr (D == 3) {
+      reinterpret_cast<V*>(F.r)[j] = V{r[0], r[1], r[2], (Real)0};
+    } else {
+      reinterpret_cast<V2*>(F.r)[j] = V2{r[0], r[1]};
+    }
+  };
+  // waits until two slots carry their tags (b only with hasb). The first look reads them
+  // whole; while one is not there, only its last piece's tag is polled, at intervals: the
+  // polls of the waiting waves would otherwise hold up the loads of those that work.
+  auto wait_two = [&](uint32_t sa, uint32_t ta, bool hasb, uint32_t sb, uint32_t tb, Raw& xa, Raw& xb) {
+    sb = hasb ? sb : sa;
+    tb = hasb ? tb : ta;
+    bool ok = false;
+    for (uint32_t n = 0; !ok && !dead;) {
+      asm volatile("" ::: "memory");  // each round reads memory again
+      P.ld(sa, xa);
+      P.ld(sb, xb);
+      ok = Port::is(xa, ta) && Port::is(xb, tb);
+      for (bool here = ok; !here && !dead;) {
+        __builtin_amdgcn_s_sleep(1);
+        asm volatile("" ::: "memory");
+        here = P.tag(sa) == ta;
+        here = P.tag(sb) == tb && here;
+        if (++n >= kSpinLimit) dead = true;
+      }
+    }
+  };
+  auto update = [&](uint32_t j, uint32_t i, const FlowContact<D, Real>& L, bool init, Real* rbest) {
+    const bool hasb = L.from_b != kNoBody;
+    Loaded<D, Real> ld;
+    Real im[4];
+    unpack_rec<D, Real>(L.g, hasb, ld.R, im);
+    ld.r[0] = L.r[0], ld.r[1] = L.r[1], ld.r[2] = L.r[2];
+    Raw xa, xb;
+    wait_two(L.from_a >> 1, tag - (L.from_a & 1u), hasb, L.from_b >> 1, tag - (L.from_b & 1u), xa, xb);
+    V b[4];
+    Port::unpack(xa, im[0], im[2], b[0], b[1]);
+    Port::unpack(xb, im[1], im[3], b[2], b[3]);
+    Real rn[3] = {0, 0, 0};
+    update_core<D, Real>(
+        ld, init, rbest, 0, 2, [&](size_t i) { return b[i]; }, [&](size_t i, const V& x) { b[i] = x; },
+        [&](int d, Real x) { rn[d] = x; });
+    P.st(j, b[0], b[1], tag);
+    if (hasb) P.st(C + j, b[2], b[3], tag);
+    if (!init) store_r(j, i, rn);
+  };
+  // squared residual of contact j on the bodies' final velocities of this sweep; false when a
+  // body has already moved on to a later sweep (only in the check of a noted contact)
+  auto residual = [&](const FlowContact<D, Real>& L, uint2 fin, bool check, double& e) {
+    const bool hasb = fin.y != kNoBody;
+    Raw xa, xb;
+    bool ok = false, late = false;
+    for (uint32_t n = 0; !ok && !late && !dead; ++n) {
+      asm volatile("" ::: "memory");
+      P.ld(fin.x, xa);
+      P.ld(hasb ? fin.y : fin.x, xb);
+      ok = Port::is(xa, tag) && (!hasb || Port::is(xb, tag));
+      if (check && !ok) late = Port::beyond(xa, tag) || (hasb && Port::beyond(xb, tag));
+      if (n >= kSpinLimit) dead = true;
+    }
+    if (!ok) return false;
+    Rec<D, Real> R;
+    Real im[4];
+    unpack_rec<D, Real>(L.g, hasb, R, im);
+    const V z = {0, 0, 0, 0};
+    V va, wa, vb = z, wb = z;
+    Port::unpack(xa, im[0], im[2], va, wa);
+    if (hasb) Port::unpack(xb, im[1], im[3], vb, wb);
+    if (A.phase == 1) {
+      float u[3];
+      rel_vel<D, float, Real>(R, va, wa, vb, wb, u);
+      const float r[3] = {(float)L.r[0], (float)L.r[1], (float)L.r[2]};
+      e = (double)fb_err<D, float>((float)R.mu, r, u);
+    } else {
+      double u[3];
+      rel_vel<D, double, Real>(R, va, wa, vb, wb, u);
+      const double r[3] = {(double)L.r[0], (double)L.r[1], (double)L.r[2]};
+      e = fb_err<D, double>((double)R.mu, r, u);
+    }
+    return true;
+  };
+  // every contact of this workgroup, in colour order: contact j, entry i of its list
+  auto for_each = [&](auto&& f) {
+    for (uint32_t c = 0; c < ncol; ++c)
+      for (uint32_t j = s_lo[c] + tid; j < s_hi[c]; j += kFlowThreads) f(j, s_at[c] + (j - s_lo[c]));
+  };
+  // the bodies' start velocities into the slots of their last contacts
+  auto start_bodies = [&](bool reset) {
+    for_each([&](uint32_t j, uint32_t) {
+      const uint2 fin = reinterpret_cast<const uint2*>(F.fin)[j];
+      for (int side = 0; side < 2; ++side) {
+        const uint32_t own = side ? C + j : j;
+        if ((side ? fin.y : fin.x) != own) continue;
+        const uint32_t sl = side ? A.c.b[j] : A.c.a[j];
+        V v, w = {0, 0, 0, 0};
+        if (reset) {
+          const uint32_t i = A.sid ? A.sid[sl] : sl;
+          v = V{(Real)A.v0[(size_t)D * i], (Real)A.v0[(size_t)D * i + 1], (Real)0, (Real)0};
+          if (D == 3) {
+            v.z = (Real)A.v0[(size_t)D * i + D - 1];
+            w = V{(Real)A.w0[3 * (size_t)i], (Real)A.w0[3 * (size_t)i + 1], (Real)A.w0[3 * (size_t)i + 2], (Real)0};
+          }
+        } else {
+          const V* rec = reinterpret_cast<const V*>(A.body) + (size_t)kBodyVecs<D> * sl;
+          v = rec[0];
+          if (D == 3) w = rec[1];
+        }
+        P.st(own, v, w, tag);
+      }
+    });
+  };
+  auto apply = [&]() {
+    for_each([&](uint32_t j, uint32_t i) {
+      FlowContact<D, Real> L;
+      load(j, i, L);
+      update(j, i, L, true, nullptr);
+    });
+  };
+  // the largest of the workgroups' values published under the current tag, the same in every
+  // thread; every workgroup has arrived when it returns
+  auto exchange = [&](double m) {
+    m = wave_reduce_max_f64(m);
+    if (lane == 0) s_red[tid >> 6] = m;
+    if (__any(dead) && lane == 0) s_dead = 1;
+    __syncthreads();
+    if (tid < 64) {
+      double b = lane < kWaves ? s_red[lane] : 0.0;
+      b = wave_reduce_max_f64(b);
+      if (lane == 0) {
+        const unsigned long long u = (unsigned long long)__double_as_longlong(b);
+        const u32x4f x = {(uint32_t)u, (uint32_t)(u >> 32), 0u, tag};
+        __builtin_amdgcn_raw_buffer_store_b128(x, prs, wg * 16u, 0, kFlowAux);
+      }
+      double all = 0.0;
+      for (uint32_t g = lane; g < G; g += 64) {
+        bool ok = false;
+        for (uint32_t n = 0; !ok && !dead; ++n) {
+          asm volatile("" ::: "memory");
+          const u32x4f x = __builtin_amdgcn_raw_buffer_load_b128(prs, g * 16u, 0, kFlowAux);
+          ok = x[3] == tag;
+          if (ok) all = fmax(all, __longlong_as_double((long long)(((unsigned long long)x[1] << 32) | x[0])));
+          if (n >= kSpinLimit) dead = true;
+        }
+      }
+      all = wave_reduce_max_f64(all);
+      if (__any(dead) && lane == 0) s_dead = 1;
+      if (lane == 0) s_red[0] = all;
+    }
+    __syncthreads();
+    const double out = s_red[0];
+    __syncthreads();
+    return out;
+  };
+  // the largest residual of the sweep just done over all workgroups, the same in every thread;
+  // a thread also notes the largest of its contacts at or above `capture` (>= 0)
+  uint32_t noted = kNoBody, noted_i = 0;
+  uint2 noted_fin = make_uint2(0, 0);
+  auto evaluate = [&](double capture) {
+    double m = 0.0;
+    noted = kNoBody;
+    for_each([&](uint32_t j, uint32_t i) {
+      FlowContact<D, Real> L;
+      load(j, i, L);
+      const uint2 fin = reinterpret_cast<const uint2*>(F.fin)[j];
+      double e = 0.0;
+      residual(L, fin, false, e);
+      if (capture >= 0.0 && e >= capture && e > m) {
+        noted = j;
+        noted_i = i;
+        noted_fin = fin;
+      }
+      m = fmax(m, e);
+    });
+    return exchange(m);
+  };
+
+  uint32_t max_iters = A.max_iters;
+  if (A.phase == 1) max_iters = max(1u, max_iters - max_iters / 4);
+  if (A.phase == 2) max_iters = (A.ctr->sweeps_fp32 < max_iters) ? max_iters - A.ctr->sweeps_fp32 : 0u;
+  const bool track_best = A.phase != 1;
+  for_each([&](uint32_t j, uint32_t i) {
+    if (i >= kept) return;
+    const V* rec = reinterpret_cast<const V*>(F.rec);
+#pragma unroll
+    for (int g = 0; g < kRecGroups<D>; ++g) l_rec[(size_t)g * kept + i] = rec[(size_t)g * C + j];
+    l_from[i] = reinterpret_cast<const uint2*>(F.from)[j];
+#pragma unroll
+    for (int d = 0; d < D; ++d) l_r[(size_t)d * kept + i] = F.r[(size_t)(D == 3 ? 4 : 2) * j + d];
+  });
+  start_bodies(false);
+  if (A.apply_init) {
+    ++tag;
+    apply();
+  }
+  const double stop = (A.phase == 1) ? 0.5 * A.tol : A.tol;
+  const bool subset = A.viol != nullptr;
+  const bool early = A.phase == 1 && F.skip_early;  // as WgBufs::skip_early
+  constexpr uint32_t kFullEvery = 256, kSkipUntil = 1024 - kFullEvery;  // as in k_gs
+  double err = evaluate(subset ? stop : -1.0);
+  uint32_t nev = 1, nskip = 0, nchecks = 0, last_full = 0;
+  double best = err, ref = best;
+  bool copy_pending = track_best;
+  uint32_t ref_it = 0, it = 0;
+  if (!(err < stop) && max_iters > 0) {
+    FlowContact<D, Real> c0, c1;
+    // lowered: the last evaluation found a new best residual below the threshold of its
+    // check; while that goes on, the next check would fail as well and is left out
+    bool copy = copy_pending, may_skip = false, eval_now = false, lowered = false;
+    double th = 0.0;
+    auto begin_sweep = [&]() {
+      ++it;
+      ++tag;
+      copy = copy_pending;
+      copy_pending = false;
+      eval_now = A.eval_every > 0 && it % A.eval_every == 0;
+      const bool stagnation_due = A.phase == 1 && it - ref_it >= 1024;
+      may_skip = subset && eval_now && it - last_full < kFullEvery && !stagnation_due &&
+                 !(lowered && last_full + A.eval_every == it);
+      th = (early && it < kSkipUntil) ? stop : fmax(stop, best);
+    };
+    // true when the solve is over
+    auto end_sweep = [&]() {
+      if (may_skip) {
+        // Is one of the contacts noted by the last full evaluation still at or above th? A
+        // workgroup that has one goes on at once; the others go on when they see its flag (or
+        // that it is past this sweep). Only when every workgroup has none is the sweep
+        // evaluated, and then none has gone on. A noted contact whose body has moved on
+        // means that another workgroup went on, so this one's answer no longer counts.
+        const uint32_t f = nchecks++ & 1u;
+        bool above = false;
+        if (noted != kNoBody) {
+          FlowContact<D, Real> L;
+          load(noted, noted_i, L);
+          double e = 0.0;
+          above = residual(L, noted_fin, true, e) && e >= th;
+        }
+        if (__any(above) && lane == 0) s_flag[f] = 1u;
+        if (__any(dead) && lane == 0) s_dead = 1u;
+        __syncthreads();
+        if (tid < 64) {
+          bool skip = s_flag[f] != 0u;
+          if (lane == 0)
+            __builtin_amdgcn_raw_buffer_store_b32(2u * tag + (skip ? 1u : 0u), frs, wg * 4u, 0, kFlowAux);
+          bool all = skip;
+          for (uint32_t n = 0; !all && !dead; ++n) {
+            asm volatile("" ::: "memory");
+            const uint32_t g = 4 * lane;
+            int32_t d[4] = {0, 0, 0, 0};
+            if (g < G) {
+              const u32x4f x = __builtin_amdgcn_raw_buffer_load_b128(frs, 4u * g, 0, kFlowAux);
+#pragma unroll
+              for (int i = 0; i < 4; ++i) d[i] = g + i < G ? (int32_t)(x[i] - 2u * tag) : 0;
+            }
+            bool any = false, here = true;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              any = any || d[i] > 0;
+              here = here && d[i] >= 0;
+            }
+            skip = __any(any);
+            all = skip || __all(here);
+            if (n >= kSpinLimit) dead = true;
+          }
+          if (lane == 0) {
+            s_skip[f] = skip ? 1u : 0u;
+            if (dead) s_dead = 1u;
+            s_flag[f ^ 1u] = 0u;
+          }
+        }
+        __syncthreads();
+        if (s_dead) return true;
+        if (s_skip[f]) {
+          ++nskip;
+          return false;
+        }
+      }
+      if (eval_now) {
+        last_full = it;
+        err = evaluate(subset ? fmax(stop, 0.1 * err) : -1.0);
+        ++nev;
+        if (s_dead) return true;
+        lowered = err < th;
+        if (err < best) {
+          best = err;
+          copy_pending = track_best;
+        }
+        if (err < stop) return true;
+        if (A.phase == 1 && it - ref_it >= 1024) {
+          if (best > 0.9999 * ref) return true;
+          ref = best;
+          ref_it = it;
+        }
+      }
+      return false;
+    };
+    // One pass: kFlowThreads contacts of a colour from position pos, held in `use`; the next
+    // pass's records are loaded into `fill` first, behind the wait and the update.
+    uint32_t col = 0, pos = s_lo[0];
+    auto pass = [&](const FlowContact<D, Real>& use, FlowContact<D, Real>& fill) {
+      dead = __any(dead);
+      const uint32_t j = pos + tid, hi = s_hi[col];
+      const bool last = pos + kFlowThreads >= hi, sweep_done = last && col + 1 == ncol;
+      const uint32_t ncol_ = sweep_done ? 0u : last ? col + 1 : col;
+      const uint32_t npos = last ? s_lo[ncol_] : pos + kFlowThreads;
+      const bool next = npos + tid < s_hi[ncol_], self = npos == pos;
+      const uint32_t i = s_at[col] + (j - s_lo[col]), ni = s_at[ncol_] + (npos + tid - s_lo[ncol_]);
+      if (next && !self) load(npos + tid, ni, fill);
+      if (j < hi) update(j, i, use, false, copy ? A.rbest + 3 * (size_t)j : nullptr);
+      if (next && self) load(npos + tid, ni, fill);  // a single pass: the impulse just stored
+      col = ncol_;
+      pos = npos;
+      if (!sweep_done) return false;
+      if (end_sweep()) return true;
+      if (it == max_iters) {
+        ++it;
+        return true;
+      }
+      begin_sweep();
+      return false;
+    };
+    begin_sweep();
+    if (s_lo[0] + tid < s_hi[0]) load(s_lo[0] + tid, tid, c0);
+    while (!pass(c0, c1) && !pass(c1, c0)) {
+    }
+    if (it > max_iters) {
+      it = max_iters;
+      if (track_best && !copy_pending) {
+        // the best iterate and its velocities: v0, then its impulses in colour order, once
+        // every workgroup is through with the last sweep's slots
+        for_each([&](uint32_t j, uint32_t i) {
+          const Real r[3] = {A.rbest[3 * (size_t)j], A.rbest[3 * (size_t)j + 1], A.rbest[3 * (size_t)j + 2]};
+          store_r(j, i, r);
+        });
+        ++tag;
+        (void)exchange(0.0);
+        ++tag;
+        start_bodies(true);
+        ++tag;
+        apply();
+      }
+    }
+  }
+  wait_stores();
+  // impulses, and the velocities of the bodies whose last contact is here
+  for_each([&](uint32_t j, uint32_t i) {
+    FlowContact<D, Real> L;
+    load(j, i, L);
+    for (int d = 0; d < D; ++d) A.c.r[3 * (size_t)j + d] = L.r[d];
+    const uint2 fin = reinterpret_cast<const uint2*>(F.fin)[j];
+    for (int side = 0; side < 2; ++side) {
+      const uint32_t own = side ? C + j : j;
+      if ((side ? fin.y : fin.x) != own) continue;
+      const uint32_t sl = side ? A.c.b[j] : A.c.a[j];
+      Raw x;
+      P.ld(own, x);
+      V v, w;
+      V* rec = reinterpret_cast<V*>(A.body) + (size_t)kBodyVecs<D> * sl;
+      Port::unpack(x, rec[0].w, (D == 3) ? rec[D == 3].w : (Real)0, v, w);
+      rec[0] = v;
+      if (D == 3) rec[1] = w;
+    }
+  });
+  if (tid == 0 && (dead || s_dead)) atomicOr(&A.ctr->overflow, 16u);
+  if (wg == 0 && tid == 0) {
+    if (A.phase == 1) {
+      A.ctr->sweeps_fp32 = it;
+      A.ctr->error_fp32 = best;
+      A.ctr->evals_fp32 = nev;
+    }
+    A.ctr->sweeps += it;
+    A.ctr->error = best;
+    A.ctr->evals += nev;
+    A.ctr->evals_skipped += nskip;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Links of the contact graph: per body its contacts in colour order (a body has at most one
+// contact of a colour, so the set of its colours orders them).
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ uint32_t colour_of(const uint32_t* off, uint32_t ncol, uint32_t k) {
+  uint32_t lo = 0, hi = ncol - 1;  // the last colour that starts at or before k
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi + 1) >> 1;
+    if (off[mid] <= k) lo = mid;
+    else hi = mid - 1;
+  }
+  return lo;
+}
+
+__global__ void __launch_bounds__(kBlock) k_flow_colours(uint32_t C, const uint32_t* __restrict__ ca,
+                                                         const uint32_t* __restrict__ cb,
+                                                         const uint32_t* __restrict__ coloff,
+                                                         const StepCounters* __restrict__ ctr,
+                                                         unsigned long long* __restrict__ mask) {
+  __shared__ uint32_t off[kMaxColours + 1];
+  const uint32_t ncol = ctr->ncolours;
+  for (uint32_t c = threadIdx.x; c <= ncol; c += kBlock) off[c] = coloff[c];
+  __syncthreads();
+  const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+  if (k >= C) return;
+  const unsigned long long m = 1ull << colour_of(off, ncol, k);
+  atomicOr(&mask[ca[k]], m);
+  if (cb[k] != kNoBody) atomicOr(&mask[cb[k]], m);
+}
+
+// Start of each body's entries in the table (any order of the bodies); mask[n] counts them.
+__global__ void __launch_bounds__(kBlock) k_flow_offsets(uint32_t n, unsigned long long* __restrict__ mask,
+                                                         uint32_t* __restrict__ start) {
+  __shared__ uint32_t s_base;
+  const uint32_t b = blockIdx.x * kBlock + threadIdx.x;
+  const uint32_t deg = b < n ? (uint32_t)__popcll(mask[b]) : 0u;
+  uint32_t total;
+  const uint32_t before = block_exclusive_scan_u32(deg, &total);
+  if (threadIdx.x == 0) s_base = total ? atomicAdd(reinterpret_cast<uint32_t*>(mask + n), total) : 0u;
+  __syncthreads();
+  if (b < n) start[b] = s_base + before;
+}
+
+// The body's contact of this colour (its outbox slot: k for side a, C + k for side b).
+__global__ void __launch_bounds__(kBlock) k_flow_table(uint32_t C, const uint32_t* __restrict__ ca,
+                                                       const uint32_t* __restrict__ cb,
+                                                       const uint32_t* __restrict__ coloff,
+                                                       const StepCounters* __restrict__ ctr,
+                                                       const unsigned long long* __restrict__ mask,
+                                                       const uint32_t* __restrict__ start,
+                                                       uint32_t* __restrict__ table) {
+  __shared__ uint32_t off[kMaxColours + 1];
+  const uint32_t ncol = ctr->ncolours;
+  for (uint32_t c = threadIdx.x; c <= ncol; c += kBlock) off[c] = coloff[c];
+  __syncthreads();
+  const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+  if (k >= C) return;
+  const unsigned long long below = (1ull << colour_of(off, ncol, k)) - 1ull;
+  const uint32_t a = ca[k], b = cb[k];
+  table[start[a] + (uint32_t)__popcll(mask[a] & below)] = k;
+  if (b != kNoBody) table[start[b] + (uint32_t)__popcll(mask[b] & below)] = C + k;
+}
+
+__global__ void __launch_bounds__(kBlock) k_flow_links(uint32_t C, const uint32_t* __restrict__ ca,
+                                                       const uint32_t* __restrict__ cb,
+                                                       const uint32_t* __restrict__ coloff,
+                                                       const StepCounters* __restrict__ ctr,
+                                                       const unsigned long long* __restrict__ mask,
+                                                       const uint32_t* __restrict__ start,
+                                                       const uint32_t* __restrict__ table, uint2* __restrict__ from,
+                                                       uint2* __restrict__ fin) {
+  __shared__ uint32_t off[kMaxColours + 1];
+  const uint32_t ncol = ctr->ncolours;
+  for (uint32_t c = threadIdx.x; c <= ncol; c += kBlock) off[c] = coloff[c];
+  __syncthreads();
+  const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+  if (k >= C) return;
+  const unsigned long long below = (1ull << colour_of(off, ncol, k)) - 1ull;
+  uint32_t fr[2] = {kNoBody, kNoBody}, fi[2] = {kNoBody, kNoBody};
+#pragma unroll
+  for (int side = 0; side < 2; ++side) {
+    const uint32_t b = side ? cb[k] : ca[k];
+    if (b == kNoBody) continue;
+    const uint32_t deg = (uint32_t)__popcll(mask[b]), rank = (uint32_t)__popcll(mask[b] & below);
+    const uint32_t* t = table + start[b];
+    fi[side] = t[deg - 1];
+    fr[side] = rank ? t[rank - 1] << 1 : (t[deg - 1] << 1 | 1u);
+  }
+  from[k] = make_uint2(fr[0], fr[1]);
+  fin[k] = make_uint2(fi[0], fi[1]);
+}
+
+// Packed records and impulses (see kRecGroups) from the colour-order arrays.
+template <int D, typename Real>
+__global__ void __launch_bounds__(kBlock) k_flow_pack(ContactSoA<Real> c, uint32_t C, const Real* __restrict__ body,
+                                                      Real* __restrict__ rec_, Real* __restrict__ r_) {
+  using V = typename Vec4<Real>::type;
+  using V2 = typename Vec2<Real>::type;
+  const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+  if (k >= C) return;
+  Rec<D, Real> R;
+  load_rec<D, Real>(c, k, R);
+  pack_rec<D, Real>(R, reinterpret_cast<const V*>(body), C, k, reinterpret_cast<V*>(rec_));
+  const Real* rp = c.r + 3 * (size_t)k;
+  if constexpr (D == 3) reinterpret_cast<V*>(r_)[k] = V{rp[0], rp[1], rp[2], (Real)0};
+  else reinterpret_cast<V2*>(r_)[k] = V2{rp[0], rp[1]};
+}
+
+hipError_t launch_flow_links(scx_ctx* c, uint32_t C, const uint32_t* ca, const uint32_t* cb, const FlowLinks& L) {
+  hipStream_t s = c->stream;
+  const uint32_t nc = (C + kBlock - 1) / kBlock, nb = (c->n + kBlock - 1) / kBlock;
+  hipError_t e = hipMemsetAsync(L.mask, 0, sizeof(unsigned long long) * ((size_t)c->n + 1), s);
+  if (e != hipSuccess) return e;
+  k_flow_colours<<<nc, kBlock, 0, s>>>(C, ca, cb, c->d.coloff, c->d.ctr, L.mask);
+  k_flow_offsets<<<nb, kBlock, 0, s>>>(c->n, L.mask, L.start);
+  k_flow_table<<<nc, kBlock, 0, s>>>(C, ca, cb, c->d.coloff, c->d.ctr, L.mask, L.start, L.table);
+  k_flow_links<<<nc, kBlock, 0, s>>>(C, ca, cb, c->d.coloff, c->d.ctr, L.mask, L.start, L.table, L.from, L.fin);
+  return hipGetLastError();
+}
+
+template <int D, typename Real>
+hipError_t launch_gs_flow(scx_ctx* c, GSArgs<Real> A, FlowBufs<Real> F, int blocks, bool* launched) {
+  const uint32_t nc = (A.C + kBlock - 1) / kBlock;
+  k_flow_pack<D, Real><<<nc, kBlock, 0, c->stream>>>(A.c, A.C, A.body, F.rec, F.r);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  // the LDS holds the records, links and impulses of as many of a workgroup's contacts as it can
+  const size_t each = sizeof(Real) * (D == 3 ? 16 + 3 : 8 + 2) + sizeof(uint2);
+  const uint32_t most = (A.C + blocks - 1) / blocks + kMaxColours;  // contacts of a workgroup
+  F.kept = std::min<uint32_t>((most + 1) / 2 * 2, (uint32_t)(kFlowLdsMax / each) / 2 * 2);
+  const size_t lds = each * F.kept;
+  const hipError_t ea = hipFuncSetAttribute((const void*)k_gs_flow<D, Real>,
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (ea != hipSuccess) return ea;
+  void* args[] = {&A, &F};
+  return launch_cooperative(c, (const void*)k_gs_flow<D, Real>, blocks, kFlowThreads, args, lds, c->stream, launched);
+}
+
+template hipError_t launch_gs_flow<2, float>(scx_ctx*, GSArgs<float>, FlowBufs<float>, int, bool*);
+template hipError_t launch_gs_flow<3, float>(scx_ctx*, GSArgs<float>, FlowBufs<float>, int, bool*);
+template hipError_t launch_gs_flow<2, double>(scx_ctx*, GSArgs<double>, FlowBufs<double>, int, bool*);
+template hipError_t launch_gs_flow<3, double>(scx_ctx*, GSArgs<double>, FlowBufs<double>, int, bool*);
+
+}  // namespace scx

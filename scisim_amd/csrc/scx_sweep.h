@@ -373,4 +373,32 @@ size_t wg_lds_bytes(uint32_t nbodies, uint32_t C);
 template <int D, typename Real>
 hipError_t launch_gs_wg(const GSArgs<Real>& A, const WgBufs<Real>& W, hipStream_t s);
 
+// Working memory of the sweeps without barriers (k_gs_flow), in colour order.
+constexpr int kFlowMaxBlocks = 256;  // one wave reads every workgroup's flag
+template <typename Real>
+struct FlowBufs {
+  Real* rec;          // packed records
+  Real* r;            // impulses: 4 (3D) or 2 (2D) Reals per contact
+  const uint32_t* from;  // per contact, 2: the slots its bodies come from (slot << 1 | sweep before)
+  const uint32_t* fin;   // per contact, 2: the slots of its bodies' last contacts
+  void* slots;        // 2 C outbox slots, in 16-byte pieces
+  uint32_t* flags;    // per workgroup: 2 * tag + whether it holds a contact above the threshold
+  void* parts;        // per workgroup: its largest residual and the tag
+  uint32_t tag0;      // first tag of this launch: above every tag in slots, flags and parts
+  int skip_early;     // as WgBufs::skip_early
+  uint32_t kept;      // contacts of a workgroup that its LDS holds
+};
+struct FlowLinks {
+  unsigned long long* mask;  // per body slot: its colours; entry n: the table's length
+  uint32_t* start;           // per body slot: start of its entries in the table
+  uint32_t* table;           // outbox slots of each body's contacts in colour order
+  uint2* from;
+  uint2* fin;
+};
+hipError_t launch_flow_links(scx_ctx* c, uint32_t C, const uint32_t* ca, const uint32_t* cb, const FlowLinks& L);
+// Packs the records and launches the sweeps on `blocks` workgroups; *launched is false when a
+// cooperative launch is not to be had (nothing ran).
+template <int D, typename Real>
+hipError_t launch_gs_flow(scx_ctx* c, GSArgs<Real> A, FlowBufs<Real> F, int blocks, bool* launched);
+
 }  // namespace scx

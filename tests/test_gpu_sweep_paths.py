@@ -1,5 +1,6 @@
-"""The sweeps of one workgroup with the bodies in LDS (k_gs_wg) against the sweeps with grid
-barriers (SCX_WG_SWEEPS=0): every contact is updated in its colour's turn with the same expressions, so steps are the
+"""The sweeps of one workgroup with the bodies in LDS (k_gs_wg) and the sweeps without barriers
+between the colours (k_gs_flow) against the sweeps with grid barriers (both switched off):
+every contact is updated in its colour's turn with the same expressions, so steps are the
 same bit for bit -- positions, velocities, impulses, sweep counts, residuals -- in FP64 and in
 FP32 with the FP64 polish, converging, ending at a sweep limit with the best iterate, through
 the FP32 stagnation test, with sparse residual checks; for contact sets around the passes of a
@@ -28,8 +29,13 @@ def _scene(kind):
     return s
 
 
-def _run(monkeypatch, s, path, prm, steps):
+def _run(monkeypatch, s, path, prm, steps, blocks=None):
     monkeypatch.setenv("SCX_WG_SWEEPS", "1" if path == "wg" else "0")
+    monkeypatch.setenv("SCX_FLOW_SWEEPS", "1" if path == "flow" else "0")
+    if blocks:
+        monkeypatch.setenv("SCX_FLOW_BLOCKS", str(blocks))
+    else:
+        monkeypatch.delenv("SCX_FLOW_BLOCKS", raising=False)
     D = s["dim"]
     ctx = scx.Context(D, s["r"].size, max_planes=8)
     try:
@@ -74,3 +80,14 @@ def test_one_workgroup(monkeypatch, kind, precision, limit):
     s = _scene(kind)
     prm = _params(s, precision, limit)
     _same(_run(monkeypatch, s, "", prm, 3), _run(monkeypatch, s, "wg", prm, 3))
+
+
+@pytest.mark.parametrize("kind,blocks", [("circles", 2), ("circles", None), ("lattice", 7), ("2500", 3), ("2500", None),
+                                         ("9000", None), ("9000", 256)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("limit", ["converged", "limit", "sparse", "stagnates"])
+def test_without_barriers(monkeypatch, kind, blocks, precision, limit):
+    print("case", kind, blocks, precision, limit, flush=True)
+    s = _scene(kind)
+    prm = _params(s, precision, limit)
+    _same(_run(monkeypatch, s, "", prm, 3), _run(monkeypatch, s, "flow", prm, 3, blocks))
