@@ -841,7 +841,7 @@ int scx_set_scenes(scx_ctx* c, uint32_t nscenes, const uint32_t* body_off, const
     HIPC(dalloc(&d.scene_shift, (size_t)3 * nscenes));
     HIPC(dalloc(&d.scene_err, nscenes));
     HIPC(dalloc(&d.scene_cnt, nscenes));
-    HIPC(dalloc(&d.scene_acc, (size_t)2 * nscenes));
+    HIPC(dalloc(&d.scene_acc, (size_t)3 * nscenes));
     HIPC(dalloc(&d.scene_sweeps, nscenes));
     c->cap_scenes = nscenes;
   }
@@ -1847,7 +1847,7 @@ int scx_load_checkpoint(scx_ctx* c, const void* buf, uint64_t len) {
       HIPC(dalloc(&d.scene_shift, (size_t)3 * h.nscenes));
       HIPC(dalloc(&d.scene_err, h.nscenes));
       HIPC(dalloc(&d.scene_cnt, h.nscenes));
-      HIPC(dalloc(&d.scene_acc, (size_t)2 * h.nscenes));
+      HIPC(dalloc(&d.scene_acc, (size_t)3 * h.nscenes));
       HIPC(dalloc(&d.scene_sweeps, h.nscenes));
       c->cap_scenes = h.nscenes;
     }

@@ -149,7 +149,7 @@ struct DeviceBuffers {
   uint32_t* scene_cnt = nullptr;   // S: per-scene contacts
   double* cmu = nullptr;           // per contact friction coefficient (cap_contacts)
   uint32_t* cscene = nullptr;      // per contact in colour order: its scene (cap_contacts)
-  unsigned long long* scene_acc = nullptr;  // 2 S: per-scene residual bits of the sweeps
+  unsigned long long* scene_acc = nullptr;  // 3 S: per-scene residual bits of the sweeps
   uint32_t* scene_sweeps = nullptr;         // S: sweep at which each scene met the tolerance
   uint32_t* act_idx = nullptr;   // 2 x cap_contacts: compacted lists of the unfrozen scenes' contacts
   uint32_t* act_part = nullptr;  // kMaxColours x gs_blocks: per-colour per-workgroup counts

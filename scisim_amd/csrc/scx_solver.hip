@@ -1525,6 +1525,15 @@ constexpr uint32_t kFlowTagMax = 1u << 30;
 // sweep on 64, 128 and 256 workgroups; 44.6 with barriers).
 constexpr uint32_t kFlowMinContacts = 1024, kFlowMaxContacts = 1u << 18;
 constexpr uint32_t kFlowContacts = 128;  // contacts of a workgroup
+// Small sets run on one XCD's CUs: every slot is then a near one (k_gs_flow), and a body's hop
+// from contact to contact costs an L2 access. From there on one XCD's 32 CUs are too few.
+// One XCD against eight, whole solves of 300 to 800 sweeps in ms: circles 3,680 contacts FP64
+// 10.1 and 11.6, 13,169 FP64 15.1 and 16.3, 24,976 FP32 5.7 and 6.4; spheres 8,495 FP64 2.8 and
+// 3.0, 10,019 FP64 11.3 and 10.9, 16,987 FP32 4.15 and 4.5, 16,987 FP64 3.35 and 2.9.
+template <int D, typename Real>
+constexpr uint32_t flow_one_xcd() {
+  return D == 2 ? 24576 : sizeof(Real) == 4 ? 16384 : 8192;
+}
 
 static hipError_t flow_arena(unsigned char** p, size_t* cap, size_t need, hipStream_t s) {
   if (need <= *cap) return hipSuccess;
@@ -1539,17 +1548,18 @@ static hipError_t flow_arena(unsigned char** p, size_t* cap, size_t need, hipStr
 }
 
 template <int D, typename Real>
-static hipError_t flow_prepare(scx_ctx* c, const GSArgs<Real>& A, bool* linked, FlowBufs<Real>& F) {
+static hipError_t flow_prepare(scx_ctx* c, const GSArgs<Real>& A, uint32_t xcds, uint32_t per_xcd, uint32_t* linked,
+                               FlowBufs<Real>& F) {
   DeviceBuffers& d = c->d;
   const size_t C = A.C, n = c->n;
   const size_t links = sizeof(unsigned long long) * (n + 2) + sizeof(uint32_t) * ((n + 1) / 2 * 2) +
                        sizeof(uint2) * 3 * C + 256;
   const size_t rec = sizeof(Real) * (D == 3 ? 16 : 8) * C, r = sizeof(Real) * (D == 3 ? 4 : 2) * C;
-  const size_t slot = (size_t)(D == 3 ? 8 : 4) * sizeof(Real) * 2 * C;  // bytes of the 2 C slots
-  const size_t sync = (size_t)kFlowMaxBlocks * (sizeof(uint32_t) + 16);
+  const size_t slot = (size_t)(D == 3 ? 8 : 4) * sizeof(Real) * 4 * flow_side(A.C);  // bytes of the slots
+  const size_t sync = (size_t)kFlowMaxBlocks * (sizeof(uint32_t) + 32);
   const unsigned char* old = d.flow_links;
   hipError_t e = flow_arena(&d.flow_links, &d.cap_flow_links, links, c->stream);
-  if (e == hipSuccess && d.flow_links != old) *linked = false;
+  if (e == hipSuccess && d.flow_links != old) *linked = 0;
   if (e == hipSuccess) e = flow_arena(&d.flow_rec, &d.cap_flow_rec, rec + r, c->stream);
   if (e == hipSuccess) e = flow_arena(&d.flow_slots, &d.cap_flow_slots, sync + slot, c->stream);
   if (e != hipSuccess) return e;
@@ -1577,13 +1587,14 @@ static hipError_t flow_prepare(scx_ctx* c, const GSArgs<Real>& A, bool* linked, 
   F.flags = reinterpret_cast<uint32_t*>(d.flow_slots);
   F.parts = d.flow_slots + sizeof(uint32_t) * kFlowMaxBlocks;
   F.slots = d.flow_slots + sync;
-  if (*linked) return hipSuccess;
-  *linked = true;
-  return launch_flow_links(c, A.C, A.c.a, A.c.b, L);
+  F.xcds = xcds;
+  if (*linked == (xcds << 16 | per_xcd)) return hipSuccess;  // the other phase's links serve
+  *linked = xcds << 16 | per_xcd;
+  return launch_flow_links(c, A.C, A.c.a, A.c.b, L, xcds, per_xcd);
 }
 
 template <int D, typename Real>
-static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint32_t* col_off, bool* linked) {
+static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint32_t* col_off, uint32_t* linked) {
   // Tail: the suffix of colours no wider than one workgroup, swept by one workgroup (no
   // grid barrier between them) when the launch has several workgroups and the suffix has
   // at least two colours.
@@ -1628,17 +1639,20 @@ static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint
                         !A.cscene;
   // bodies in one workgroup's LDS: up to kWgMaxContacts contacts
   const size_t wg_lds = wg_lds_bytes<D, Real>(A.nbodies, A.C);
-  const bool one_scene = c->force_blocks <= 0 && !A.cscene && !lds_path;
-  const bool wg = one_scene && c->wg_sweeps && A.lmap && A.C <= kWgMaxContacts && wg_lds <= kWgLdsMax;
+  const bool free_width = c->force_blocks <= 0 && !lds_path;
+  const bool wg = free_width && !A.cscene && c->wg_sweeps && A.lmap && A.C <= kWgMaxContacts && wg_lds <= kWgLdsMax;
   // no barriers between the colours: from there to kFlowMaxContacts, while the slots can be
-  // addressed and the tags last
-  const bool flow = one_scene && !wg && c->flow_sweeps && !c->coop_unavailable && max_blocks > 1 &&
-                    A.C >= kFlowMinContacts && A.C <= kFlowMaxContacts && A.max_iters < kFlowTagMax / 4 &&
-                    (uint64_t)A.C * (D == 3 ? 16 : 8) * sizeof(Real) < (1ull << 31);
+  // addressed and the tags last; ensembles of up to kFlowMaxScenes scenes
+  const bool flow = free_width && !wg && c->flow_sweeps && !c->coop_unavailable && max_blocks >= (int)kXcds &&
+                    A.C >= kFlowMinContacts && A.C <= kFlowMaxContacts && A.nscenes <= kFlowMaxScenes &&
+                    A.max_iters < kFlowTagMax / 4 && (uint64_t)A.C * (D == 3 ? 32 : 16) * sizeof(Real) < (1ull << 31) - 4096;
   // the autotuner picks among widths around the model's (not for the solves of one workgroup)
   const int phase = std::is_same<Real, double>::value ? 1 : 0;
   const bool tune = c->tuner.enabled && c->force_blocks <= 0 && !lds_path && !wg && !c->coop_unavailable;
-  const int flow_most = std::min(max_blocks, kFlowMaxBlocks);
+  // one XCD's CUs up to flow_one_xcd contacts, all beyond
+  uint32_t xcds = A.C <= flow_one_xcd<D, Real>() ? 1 : kXcds;
+  if (const char* env = getenv("SCX_FLOW_XCDS")) xcds = (uint32_t)std::max(1, std::min(atoi(env), (int)kXcds));
+  const int flow_most = std::min(max_blocks, kFlowMaxBlocks) / (int)kXcds * (int)xcds;
   const int width = flow ? std::max(2, std::min((int)((A.C + kFlowContacts - 1) / kFlowContacts), flow_most)) : model;
   const int want = tune ? tune_pick(c, phase, tune_key(D, phase, A.cscene != nullptr, A.C, nw), width,
                                     flow ? flow_most : max_blocks)
@@ -1673,13 +1687,19 @@ static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint
   bool launched = false;
   if (flow) {
     FlowBufs<Real> F;
-    e = flow_prepare<D, Real>(c, A, linked, F);
+    // SCX_FLOW_BLOCKS, SCX_FLOW_XCDS: a fixed workgroup count and spread (the results do not
+    // depend on them; for tests)
+    int fb = want;
+    if (const char* env = getenv("SCX_FLOW_BLOCKS")) fb = atoi(env);
+    const uint32_t per_xcd = ((uint32_t)std::max(1, std::min(fb, flow_most)) + xcds - 1) / xcds;
+    e = flow_prepare<D, Real>(c, A, xcds, per_xcd, linked, F);
     if (e != hipSuccess) return e;
     F.skip_early = skip_early;
-    int fb = std::max(2, std::min(want, flow_most));
-    // SCX_FLOW_BLOCKS: a fixed workgroup count (the results do not depend on it; for tests)
-    if (const char* env = getenv("SCX_FLOW_BLOCKS")) fb = std::max(2, std::min(atoi(env), flow_most));
-    e = launch_gs_flow<D, Real>(c, A, F, fb, &launched);
+    if (A.cscene) {
+      e = hipMemsetAsync(A.scene_acc, 0, sizeof(unsigned long long) * 3 * A.nscenes, c->stream);
+      if (e != hipSuccess) return e;
+    }
+    e = launch_gs_flow<D, Real>(c, A, F, per_xcd, &launched);
     if (e == hipSuccess && launched && tune) e = hipEventRecord(c->tuner.pend[phase].ev[1], c->stream);
     if (e != hipSuccess || launched) return e;
   }
@@ -1734,7 +1754,7 @@ static hipError_t solve_dim(scx_ctx* c, uint32_t C, const uint32_t* col_off, con
   if (e != hipSuccess || C == 0) return e;
   const bool ens = c->nscenes > 0;
   c->barrier_sweeps = false;
-  bool linked = false;  // the links of this contact set have been made
+  uint32_t linked = 0;  // the launch shape for which this contact set has its links
   if (ens) {
     k_contact_scene<<<(C + kBlock - 1) / kBlock, kBlock, 0, s>>>(C, c->d.c64.a, c->d.sid, c->d.bscene, c->d.cscene);
     e = hipGetLastError();

@@ -11,6 +11,8 @@
 // body is the colour order, cyclic over the sweeps) polls that slot until the tag is the one
 // it waits for. No store is waited for, nothing is read that has not been written, and the
 // stores of a wave are contiguous.
+// A slot whose readers are all on the writer's XCD is stored into its L2 (430 cycles to the
+// next load, which passes the L1 by), others go through to memory (600 to 1,000 cycles).
 //
 // The iterates are those of the colour passes bit for bit: the order of the contacts on
 // every body is the colour order, and a contact reads nothing but its own two bodies.
@@ -33,7 +35,7 @@ typedef uint32_t u32x4f __attribute__((ext_vector_type(4)));
 
 constexpr int kFlowThreads = 512;
 constexpr uint32_t kSpinLimit = 1u << 21;  // about a second of polls
-constexpr size_t kFlowLdsMax = 150 * 1024;
+constexpr size_t kFlowLdsMax = 138 * 1024;  // beside the kernel's static arrays
 constexpr int kFlowAux = 16;               // agent scope (SC1)
 
 // 16-byte pieces of a slot: three words of velocity and the tag.
@@ -92,7 +94,8 @@ struct FlowPort {
       w = V{0, 0, 0, 0};
     }
   }
-  __device__ __forceinline__ void st(uint32_t slot, const V& v, const V& w, uint32_t tag) const {
+  // near: every reader is on this XCD, so the store may stay in its L2
+  __device__ __forceinline__ void st(uint32_t slot, const V& v, const V& w, uint32_t tag, bool near) const {
     Real r[NR];
     if constexpr (D == 3) {
       r[0] = v.x, r[1] = v.y, r[2] = v.z, r[3] = w.x, r[4] = w.y, r[5] = w.z;
@@ -116,23 +119,28 @@ struct FlowPort {
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
       const u32x4f x = {u[3 * i], u[3 * i + 1], u[3 * i + 2], tag};
-      __builtin_amdgcn_raw_buffer_store_b128(x, rs, o + 16u * i, 0, kFlowAux);
+      if (near) __builtin_amdgcn_raw_buffer_store_b128(x, rs, o + 16u * i, 0, 0);
+      else __builtin_amdgcn_raw_buffer_store_b128(x, rs, o + 16u * i, 0, kFlowAux);
     }
   }
 };
 
 // A contact ready to be updated: its record and impulse, and where its bodies come from
-// (slot << 1 | 1 when the slot is the one of the sweep before).
+// (slot << 2 | whether its own slot of that body is read on this XCD alone << 1 | whether the
+// slot is the one of the sweep before).
 template <int D, typename Real>
 struct FlowContact {
   typename Vec4<Real>::type g[kRecGroups<D>];
   Real r[3];
   uint32_t from_a, from_b;  // from_b == kNoBody: a plane
+  uint32_t scene;           // ensembles
 };
 
-// The solve of k_gs for one scene, step for step (phases, stopping rule, best iterate,
-// stagnation, skipped evaluations).
-template <int D, typename Real>
+// The solve of k_gs, step for step (phases, stopping rule, best iterate, stagnation, skipped
+// evaluations). Ens: an ensemble; its scenes share no body, so they are independent parts of
+// one graph. A scene is frozen when an evaluation finds it below the tolerance: its contacts
+// are neither updated nor evaluated any more, its residual stays in frozen_max.
+template <int D, typename Real, bool Ens>
 __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBufs<Real> F) {
   using V = typename Vec4<Real>::type;
   using V2 = typename Vec2<Real>::type;
@@ -144,9 +152,15 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
   __shared__ uint32_t s_at[kMaxColours];  // the first one's place in the workgroup's list
   __shared__ double s_red[kWaves];
   __shared__ uint32_t s_flag[2], s_skip[2], s_dead;
+  __shared__ uint32_t s_frozen[Ens ? kFlowMaxScenes / 32 : 1];           // frozen scenes
+  __shared__ unsigned long long s_acc[Ens ? kFlowMaxScenes : 1];         // residuals of this workgroup's scenes
   const uint32_t tid = threadIdx.x, lane = tid & 63;
-  const uint32_t C = A.C, G = gridDim.x;
-  const uint32_t wg = xcd_block();  // neighbouring ranges on one XCD
+  // The dispatcher deals workgroups to the XCDs round-robin: the workgroups of the first
+  // F.xcds XCDs take part, neighbouring ranges of contacts on one XCD.
+  const uint32_t per_xcd = gridDim.x / kXcds;
+  if (blockIdx.x % kXcds >= F.xcds) return;
+  const uint32_t C = A.C, Cp = flow_side(C), G = F.xcds * per_xcd;
+  const uint32_t wg = blockIdx.x % kXcds * per_xcd + blockIdx.x / kXcds;
   const uint32_t ncol = A.ctr->ncolours;
   for (uint32_t c = tid; c < ncol; c += kFlowThreads) {
     const uint32_t o = A.coloff[c], n = A.coloff[c + 1] - o;
@@ -154,6 +168,8 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
     s_hi[c] = o + (uint32_t)((uint64_t)n * (wg + 1) / G);
   }
   if (tid == 0) s_flag[0] = s_flag[1] = s_skip[0] = s_skip[1] = s_dead = 0;
+  if (Ens)
+    for (uint32_t w = tid; w < kFlowMaxScenes / 32; w += kFlowThreads) s_frozen[w] = 0;
   __syncthreads();
   if (tid == 0) {
     uint32_t n = 0;
@@ -170,14 +186,19 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
   uint2* l_from = reinterpret_cast<uint2*>(l_rec + (size_t)kRecGroups<D> * kept);
   Real* l_r = reinterpret_cast<Real*>(l_from + kept);
   Port P;
-  P.rs = __builtin_amdgcn_make_buffer_rsrc(F.slots, (short)0, (int)(2u * C * (uint32_t)(16 * Port::NP)), 0x00020000);
+  P.rs = __builtin_amdgcn_make_buffer_rsrc(F.slots, (short)0, (int)(4u * Cp * (uint32_t)(16 * Port::NP)), 0x00020000);
   const __amdgpu_buffer_rsrc_t frs = __builtin_amdgcn_make_buffer_rsrc(F.flags, (short)0, (int)(4u * kFlowMaxBlocks), 0x00020000);
-  const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(F.parts, (short)0, (int)(16u * kFlowMaxBlocks), 0x00020000);
+  const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(F.parts, (short)0, (int)(32u * kFlowMaxBlocks), 0x00020000);
   uint32_t tag = F.tag0;  // of the sweep under way
   bool dead = false;      // a wait of this wave ran out
+  // Exchanges so far. Their parts lie in two buffers in turn: a workgroup that publishes for
+  // exchange n + 2 has seen every part of exchange n + 1, whose owners had read all of n.
+  uint32_t nex = 0;
+  bool one_l2 = false;    // the workgroups dealt to an XCD are on one XCD
 
   // contact j, entry i of the workgroup's list
-  auto load = [&](uint32_t j, uint32_t i, FlowContact<D, Real>& L) {
+  auto load = [&](uint32_t j, uint32_t i, FlowContact<D, Real>& L) __attribute__((always_inline)) {
+    if (Ens) L.scene = A.cscene[j];
     if (i < kept) {
 #pragma unroll
       for (int g = 0; g < kRecGroups<D>; ++g) L.g[g] = l_rec[(size_t)g * kept + i];
@@ -213,10 +234,14 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
       reinterpret_cast<V2*>(F.r)[j] = V2{r[0], r[1]};
     }
   };
+  // the slot that contact j writes for a body: near ones after the far ones
+  auto own_slot = [&](uint32_t j, uint32_t side, uint32_t from) {
+    return j + (side ? Cp : 0u) + ((from & 2u) ? 2u * Cp : 0u);
+  };
   // waits until two slots carry their tags (b only with hasb). The first look reads them
   // whole; while one is not there, only its last piece's tag is polled, at intervals: the
   // polls of the waiting waves would otherwise hold up the loads of those that work.
-  auto wait_two = [&](uint32_t sa, uint32_t ta, bool hasb, uint32_t sb, uint32_t tb, Raw& xa, Raw& xb) {
+  auto wait_two = [&](uint32_t sa, uint32_t ta, bool hasb, uint32_t sb, uint32_t tb, Raw& xa, Raw& xb) __attribute__((always_inline)) {
     sb = hasb ? sb : sa;
     tb = hasb ? tb : ta;
     bool ok = false;
@@ -234,14 +259,14 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
       }
     }
   };
-  auto update = [&](uint32_t j, uint32_t i, const FlowContact<D, Real>& L, bool init, Real* rbest) {
+  auto update = [&](uint32_t j, uint32_t i, const FlowContact<D, Real>& L, bool init, Real* rbest) __attribute__((always_inline)) {
     const bool hasb = L.from_b != kNoBody;
     Loaded<D, Real> ld;
     Real im[4];
     unpack_rec<D, Real>(L.g, hasb, ld.R, im);
     ld.r[0] = L.r[0], ld.r[1] = L.r[1], ld.r[2] = L.r[2];
     Raw xa, xb;
-    wait_two(L.from_a >> 1, tag - (L.from_a & 1u), hasb, L.from_b >> 1, tag - (L.from_b & 1u), xa, xb);
+    wait_two(L.from_a >> 2, tag - (L.from_a & 1u), hasb, L.from_b >> 2, tag - (L.from_b & 1u), xa, xb);
     V b[4];
     Port::unpack(xa, im[0], im[2], b[0], b[1]);
     Port::unpack(xb, im[1], im[3], b[2], b[3]);
@@ -249,13 +274,13 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
     update_core<D, Real>(
         ld, init, rbest, 0, 2, [&](size_t i) { return b[i]; }, [&](size_t i, const V& x) { b[i] = x; },
         [&](int d, Real x) { rn[d] = x; });
-    P.st(j, b[0], b[1], tag);
-    if (hasb) P.st(C + j, b[2], b[3], tag);
+    P.st(own_slot(j, 0, L.from_a), b[0], b[1], tag, one_l2 && (L.from_a & 2u));
+    if (hasb) P.st(own_slot(j, 1, L.from_b), b[2], b[3], tag, one_l2 && (L.from_b & 2u));
     if (!init) store_r(j, i, rn);
   };
   // squared residual of contact j on the bodies' final velocities of this sweep; false when a
   // body has already moved on to a later sweep (only in the check of a noted contact)
-  auto residual = [&](const FlowContact<D, Real>& L, uint2 fin, bool check, double& e) {
+  auto residual = [&](const FlowContact<D, Real>& L, uint2 fin, bool check, double& e) __attribute__((always_inline)) {
     const bool hasb = fin.y != kNoBody;
     Raw xa, xb;
     bool ok = false, late = false;
@@ -288,6 +313,9 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
     }
     return true;
   };
+  auto frozen = [&](const FlowContact<D, Real>& L) {
+    return Ens && ((s_frozen[L.scene >> 5] >> (L.scene & 31)) & 1u) != 0;
+  };
   // every contact of this workgroup, in colour order: contact j, entry i of its list
   auto for_each = [&](auto&& f) {
     for (uint32_t c = 0; c < ncol; ++c)
@@ -296,9 +324,9 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
   // the bodies' start velocities into the slots of their last contacts
   auto start_bodies = [&](bool reset) {
     for_each([&](uint32_t j, uint32_t) {
-      const uint2 fin = reinterpret_cast<const uint2*>(F.fin)[j];
+      const uint2 fin = reinterpret_cast<const uint2*>(F.fin)[j], fr = reinterpret_cast<const uint2*>(F.from)[j];
       for (int side = 0; side < 2; ++side) {
-        const uint32_t own = side ? C + j : j;
+        const uint32_t own = own_slot(j, side, side ? fr.y : fr.x);
         if ((side ? fin.y : fin.x) != own) continue;
         const uint32_t sl = side ? A.c.b[j] : A.c.a[j];
         V v, w = {0, 0, 0, 0};
@@ -314,7 +342,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
           v = rec[0];
           if (D == 3) w = rec[1];
         }
-        P.st(own, v, w, tag);
+        P.st(own, v, w, tag, one_l2 && ((side ? fr.y : fr.x) & 2u));
       }
     });
   };
@@ -327,10 +355,11 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
   };
   // the largest of the workgroups' values published under the current tag, the same in every
   // thread; every workgroup has arrived when it returns
-  auto exchange = [&](double m) {
+  auto exchange = [&](double m) __attribute__((always_inline)) {
     m = wave_reduce_max_f64(m);
     if (lane == 0) s_red[tid >> 6] = m;
     if (__any(dead) && lane == 0) s_dead = 1;
+    if (Ens) wait_stores();  // the scenes' residuals are in memory before the workgroup arrives
     __syncthreads();
     if (tid < 64) {
       double b = lane < kWaves ? s_red[lane] : 0.0;
@@ -338,14 +367,15 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
       if (lane == 0) {
         const unsigned long long u = (unsigned long long)__double_as_longlong(b);
         const u32x4f x = {(uint32_t)u, (uint32_t)(u >> 32), 0u, tag};
-        __builtin_amdgcn_raw_buffer_store_b128(x, prs, wg * 16u, 0, kFlowAux);
+        __builtin_amdgcn_raw_buffer_store_b128(x, prs, (nex & 1u) * 16u * kFlowMaxBlocks + wg * 16u, 0, kFlowAux);
       }
       double all = 0.0;
       for (uint32_t g = lane; g < G; g += 64) {
         bool ok = false;
         for (uint32_t n = 0; !ok && !dead; ++n) {
           asm volatile("" ::: "memory");
-          const u32x4f x = __builtin_amdgcn_raw_buffer_load_b128(prs, g * 16u, 0, kFlowAux);
+          const u32x4f x =
+              __builtin_amdgcn_raw_buffer_load_b128(prs, (nex & 1u) * 16u * kFlowMaxBlocks + g * 16u, 0, kFlowAux);
           ok = x[3] == tag;
           if (ok) all = fmax(all, __longlong_as_double((long long)(((unsigned long long)x[1] << 32) | x[0])));
           if (n >= kSpinLimit) dead = true;
@@ -357,6 +387,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
     }
     __syncthreads();
     const double out = s_red[0];
+    ++nex;
     __syncthreads();
     return out;
   };
@@ -364,15 +395,31 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
   // a thread also notes the largest of its contacts at or above `capture` (>= 0)
   uint32_t noted = kNoBody, noted_i = 0;
   uint2 noted_fin = make_uint2(0, 0);
-  auto evaluate = [&](double capture) {
+  const double stop = (A.phase == 1) ? 0.5 * A.tol : A.tol;
+  uint32_t nev = 0;  // evaluations
+  double frozen_max = 0.0;
+  auto evaluate = [&](double capture, uint32_t sweeps) __attribute__((always_inline)) {
     double m = 0.0;
     noted = kNoBody;
+    // Ensembles: three buffers of the scenes' residuals in turn. This evaluation's was cleared
+    // during the last one; the next one's, which every workgroup is through with since it
+    // arrived at the last exchange, is cleared now.
+    unsigned long long* acc = A.scene_acc + (size_t)(nev % 3) * A.nscenes;
+    if (Ens) {
+      unsigned long long* clear = A.scene_acc + (size_t)((nev + 1) % 3) * A.nscenes;
+      for (uint32_t sc = wg * kFlowThreads + tid; sc < A.nscenes; sc += G * kFlowThreads)
+        __hip_atomic_store(clear + sc, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (uint32_t sc = tid; sc < A.nscenes; sc += kFlowThreads) s_acc[sc] = 0ull;
+      __syncthreads();
+    }
     for_each([&](uint32_t j, uint32_t i) {
       FlowContact<D, Real> L;
       load(j, i, L);
+      if (frozen(L)) return;
       const uint2 fin = reinterpret_cast<const uint2*>(F.fin)[j];
       double e = 0.0;
       residual(L, fin, false, e);
+      if (Ens && e > 0.0) atomicMax(s_acc + L.scene, (unsigned long long)__double_as_longlong(e));
       if (capture >= 0.0 && e >= capture && e > m) {
         noted = j;
         noted_i = i;
@@ -380,7 +427,45 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
       }
       m = fmax(m, e);
     });
-    return exchange(m);
+    if (Ens) {
+      __syncthreads();
+      for (uint32_t sc = tid; sc < A.nscenes; sc += kFlowThreads)
+        if (s_acc[sc] != 0ull) atomicMax(acc + sc, s_acc[sc]);
+    }
+    double out = exchange(m);
+    ++nev;
+    if (Ens) {
+      out = fmax(out, frozen_max);
+      auto of_scene = [&](uint32_t sc) {
+        return __longlong_as_double(
+            (long long)__hip_atomic_load(acc + sc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+      };
+      double fm = 0.0;
+      for (uint32_t b0 = 0; b0 < A.nscenes; b0 += kFlowThreads) {
+        const uint32_t sc = b0 + tid;
+        const uint32_t w = sc >> 5;
+        const bool was = sc < A.nscenes && ((s_frozen[w] >> (sc & 31)) & 1u) != 0;
+        const double es = sc < A.nscenes && !was ? of_scene(sc) : 0.0;
+        const bool now_f = sc < A.nscenes && !was && es < stop;
+        if (now_f) fm = fmax(fm, es);
+        const unsigned long long bal = __ballot(now_f || was);
+        if ((sc & 31) == 0 && sc < A.nscenes) s_frozen[w] = (uint32_t)(bal >> (lane & 32));
+        // one thread of the grid keeps the scene's sweep count
+        if (sc < A.nscenes && !was && sc % (G * kFlowThreads) == wg * kFlowThreads + tid % kFlowThreads) {
+          if (now_f) {
+            if (A.scene_sweeps[sc] == kNoBody) A.scene_sweeps[sc] = sweeps;
+          } else if (A.phase == 2) {
+            A.scene_sweeps[sc] = kNoBody;  // an FP32 estimate below the tolerance was not confirmed
+          }
+        }
+      }
+      fm = wave_reduce_max_f64(fm);
+      if (lane == 0) s_red[tid >> 6] = fm;
+      __syncthreads();
+      for (int w = 0; w < kWaves; ++w) frozen_max = fmax(frozen_max, s_red[w]);
+      __syncthreads();
+    }
+    return out;
   };
 
   uint32_t max_iters = A.max_iters;
@@ -396,17 +481,44 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
 #pragma unroll
     for (int d = 0; d < D; ++d) l_r[(size_t)d * kept + i] = F.r[(size_t)(D == 3 ? 4 : 2) * j + d];
   });
+  {
+    // every workgroup's XCD, published and read like the residuals
+    if (tid < 64) {
+      const uint32_t xcc = __builtin_amdgcn_s_getreg(20 | (0 << 6) | (3 << 11));  // XCC_ID
+      const u32x4f mine = {xcc, 0u, 0u, tag};
+      if (lane == 0) __builtin_amdgcn_raw_buffer_store_b128(mine, prs, wg * 16u, 0, kFlowAux);
+      bool same = true;
+      for (uint32_t g = lane; g < G; g += 64) {
+        bool ok = false;
+        for (uint32_t n = 0; !ok && !dead; ++n) {
+          asm volatile("" ::: "memory");
+          const u32x4f x = __builtin_amdgcn_raw_buffer_load_b128(prs, g * 16u, 0, kFlowAux);
+          const u32x4f y = __builtin_amdgcn_raw_buffer_load_b128(prs, g / per_xcd * per_xcd * 16u, 0, kFlowAux);
+          ok = x[3] == tag && y[3] == tag;
+          same = same && (!ok || x[0] == y[0]);
+          if (n >= kSpinLimit) dead = true;
+        }
+      }
+      const bool all = __all(same && !dead);
+      if (lane == 0) s_skip[0] = all ? 1u : 0u;
+      if (__any(dead) && lane == 0) s_dead = 1;
+    }
+    __syncthreads();
+    one_l2 = s_skip[0] != 0u;
+    ++nex;
+    ++tag;
+  }
   start_bodies(false);
   if (A.apply_init) {
     ++tag;
     apply();
   }
-  const double stop = (A.phase == 1) ? 0.5 * A.tol : A.tol;
+  const uint32_t base = (A.phase == 2) ? A.ctr->sweeps_fp32 : 0u;
   const bool subset = A.viol != nullptr;
   const bool early = A.phase == 1 && F.skip_early;  // as WgBufs::skip_early
   constexpr uint32_t kFullEvery = 256, kSkipUntil = 1024 - kFullEvery;  // as in k_gs
-  double err = evaluate(subset ? stop : -1.0);
-  uint32_t nev = 1, nskip = 0, nchecks = 0, last_full = 0;
+  double err = evaluate(subset ? stop : -1.0, base);
+  uint32_t nskip = 0, nchecks = 0, last_full = 0;
   double best = err, ref = best;
   bool copy_pending = track_best;
   uint32_t ref_it = 0, it = 0;
@@ -428,7 +540,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
       th = (early && it < kSkipUntil) ? stop : fmax(stop, best);
     };
     // true when the solve is over
-    auto end_sweep = [&]() {
+    auto end_sweep = [&]() __attribute__((always_inline)) {
       if (may_skip) {
         // Is one of the contacts noted by the last full evaluation still at or above th? A
         // workgroup that has one goes on at once; the others go on when they see its flag (or
@@ -485,8 +597,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
       }
       if (eval_now) {
         last_full = it;
-        err = evaluate(subset ? fmax(stop, 0.1 * err) : -1.0);
-        ++nev;
+        err = evaluate(subset ? fmax(stop, 0.1 * err) : -1.0, base + it);
         if (s_dead) return true;
         lowered = err < th;
         if (err < best) {
@@ -505,7 +616,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
     // One pass: kFlowThreads contacts of a colour from position pos, held in `use`; the next
     // pass's records are loaded into `fill` first, behind the wait and the update.
     uint32_t col = 0, pos = s_lo[0];
-    auto pass = [&](const FlowContact<D, Real>& use, FlowContact<D, Real>& fill) {
+    auto pass = [&](const FlowContact<D, Real>& use, FlowContact<D, Real>& fill) __attribute__((always_inline)) {
       dead = __any(dead);
       const uint32_t j = pos + tid, hi = s_hi[col];
       const bool last = pos + kFlowThreads >= hi, sweep_done = last && col + 1 == ncol;
@@ -514,11 +625,20 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
       const bool next = npos + tid < s_hi[ncol_], self = npos == pos;
       const uint32_t i = s_at[col] + (j - s_lo[col]), ni = s_at[ncol_] + (npos + tid - s_lo[ncol_]);
       if (next && !self) load(npos + tid, ni, fill);
-      if (j < hi) update(j, i, use, false, copy ? A.rbest + 3 * (size_t)j : nullptr);
+      if (j < hi) {
+        Real* rb = copy ? A.rbest + 3 * (size_t)j : nullptr;
+        if (!frozen(use)) {
+          update(j, i, use, false, rb);
+        } else if (rb) {
+          for (int d = 0; d < 3; ++d) rb[d] = use.r[d];
+        }
+      }
       if (next && self) load(npos + tid, ni, fill);  // a single pass: the impulse just stored
       col = ncol_;
       pos = npos;
-      if (!sweep_done) return false;
+      return sweep_done;
+    };
+    auto sweep_over = [&]() __attribute__((always_inline)) {
       if (end_sweep()) return true;
       if (it == max_iters) {
         ++it;
@@ -529,7 +649,14 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
     };
     begin_sweep();
     if (s_lo[0] + tid < s_hi[0]) load(s_lo[0] + tid, tid, c0);
-    while (!pass(c0, c1) && !pass(c1, c0)) {
+    if constexpr (Ens) {  // one copy of the larger evaluation
+      for (bool odd = false;; odd = !odd)
+        if ((odd ? pass(c1, c0) : pass(c0, c1)) && sweep_over()) break;
+    } else {
+      for (;;) {
+        if (pass(c0, c1) && sweep_over()) break;
+        if (pass(c1, c0) && sweep_over()) break;
+      }
     }
     if (it > max_iters) {
       it = max_iters;
@@ -537,6 +664,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
         // the best iterate and its velocities: v0, then its impulses in colour order, once
         // every workgroup is through with the last sweep's slots
         for_each([&](uint32_t j, uint32_t i) {
+          if (Ens && ((s_frozen[A.cscene[j] >> 5] >> (A.cscene[j] & 31)) & 1u)) return;  // keeps its impulses
           const Real r[3] = {A.rbest[3 * (size_t)j], A.rbest[3 * (size_t)j + 1], A.rbest[3 * (size_t)j + 2]};
           store_r(j, i, r);
         });
@@ -557,7 +685,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
     for (int d = 0; d < D; ++d) A.c.r[3 * (size_t)j + d] = L.r[d];
     const uint2 fin = reinterpret_cast<const uint2*>(F.fin)[j];
     for (int side = 0; side < 2; ++side) {
-      const uint32_t own = side ? C + j : j;
+      const uint32_t own = own_slot(j, side, side ? L.from_b : L.from_a);
       if ((side ? fin.y : fin.x) != own) continue;
       const uint32_t sl = side ? A.c.b[j] : A.c.a[j];
       Raw x;
@@ -626,7 +754,7 @@ __global__ void __launch_bounds__(kBlock) k_flow_offsets(uint32_t n, unsigned lo
   if (b < n) start[b] = s_base + before;
 }
 
-// The body's contact of this colour (its outbox slot: k for side a, C + k for side b).
+// The body's contact of this colour (its outbox slot: k for side a, flow_side(C) + k for side b).
 __global__ void __launch_bounds__(kBlock) k_flow_table(uint32_t C, const uint32_t* __restrict__ ca,
                                                        const uint32_t* __restrict__ cb,
                                                        const uint32_t* __restrict__ coloff,
@@ -643,7 +771,7 @@ __global__ void __launch_bounds__(kBlock) k_flow_table(uint32_t C, const uint32_
   const unsigned long long below = (1ull << colour_of(off, ncol, k)) - 1ull;
   const uint32_t a = ca[k], b = cb[k];
   table[start[a] + (uint32_t)__popcll(mask[a] & below)] = k;
-  if (b != kNoBody) table[start[b] + (uint32_t)__popcll(mask[b] & below)] = C + k;
+  if (b != kNoBody) table[start[b] + (uint32_t)__popcll(mask[b] & below)] = flow_side(C) + k;
 }
 
 __global__ void __launch_bounds__(kBlock) k_flow_links(uint32_t C, const uint32_t* __restrict__ ca,
@@ -652,7 +780,8 @@ __global__ void __launch_bounds__(kBlock) k_flow_links(uint32_t C, const uint32_
                                                        const StepCounters* __restrict__ ctr,
                                                        const unsigned long long* __restrict__ mask,
                                                        const uint32_t* __restrict__ start,
-                                                       const uint32_t* __restrict__ table, uint2* __restrict__ from,
+                                                       const uint32_t* __restrict__ table, uint32_t xcds,
+                                                       uint32_t per_xcd, uint2* __restrict__ from,
                                                        uint2* __restrict__ fin) {
   __shared__ uint32_t off[kMaxColours + 1];
   const uint32_t ncol = ctr->ncolours;
@@ -661,15 +790,42 @@ __global__ void __launch_bounds__(kBlock) k_flow_links(uint32_t C, const uint32_
   const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
   if (k >= C) return;
   const unsigned long long below = (1ull << colour_of(off, ncol, k)) - 1ull;
+  // the XCD of the workgroup that updates contact i of colour c
+  auto xcd_of = [&](uint32_t c, uint32_t i) {
+    const uint64_t n = off[c + 1] - off[c], G = (uint64_t)xcds * per_xcd;
+    return (uint32_t)((((uint64_t)(i - off[c]) + 1) * G - 1) / n) / per_xcd;
+  };
+  // A slot may stay in its XCD's L2 when every contact of the body is updated there (they are
+  // its readers) and the slots that share its lines are written there too: a line that is dirty
+  // in one L2 must not hold another XCD's slots.
+  const uint32_t col = colour_of(off, ncol, k), x = xcd_of(col, k);
+  auto line = [&](uint32_t c, uint32_t i) {
+    const uint32_t i0 = i / kFlowLine * kFlowLine, i1 = min(i0 + kFlowLine, C) - 1;
+    return off[c] <= i0 && i1 < off[c + 1] && xcd_of(c, i0) == xcd_of(c, i1);
+  };
+  const uint32_t Cp = flow_side(C);
   uint32_t fr[2] = {kNoBody, kNoBody}, fi[2] = {kNoBody, kNoBody};
 #pragma unroll
   for (int side = 0; side < 2; ++side) {
     const uint32_t b = side ? cb[k] : ca[k];
     if (b == kNoBody) continue;
-    const uint32_t deg = (uint32_t)__popcll(mask[b]), rank = (uint32_t)__popcll(mask[b] & below);
+    const unsigned long long m = mask[b];
+    const uint32_t deg = (uint32_t)__popcll(m), rank = (uint32_t)__popcll(m & below);
     const uint32_t* t = table + start[b];
-    fi[side] = t[deg - 1];
-    fr[side] = rank ? t[rank - 1] << 1 : (t[deg - 1] << 1 | 1u);
+    bool here = true;  // every contact of the body is updated on XCD x
+    uint32_t cpred = 0, clast = 0;
+    unsigned long long left = m;
+    for (uint32_t q = 0; q < deg; ++q) {
+      const uint32_t c = (uint32_t)__ffsll((long long)left) - 1;
+      left &= left - 1;
+      here = here && xcd_of(c, t[q] < Cp ? t[q] : t[q] - Cp) == x;
+      if (q + 1 == (rank ? rank : deg)) cpred = c;
+      clast = c;
+    }
+    // slot of the body's contact `e` (colour c): after the far slots when it is near
+    auto slot = [&](uint32_t c, uint32_t e) { return e + (here && line(c, e < Cp ? e : e - Cp) ? 2u * Cp : 0u); };
+    fi[side] = slot(clast, t[deg - 1]);
+    fr[side] = slot(cpred, t[rank ? rank - 1 : deg - 1]) << 2 | (here && line(col, k) ? 2u : 0u) | (rank ? 0u : 1u);
   }
   from[k] = make_uint2(fr[0], fr[1]);
   fin[k] = make_uint2(fi[0], fi[1]);
@@ -691,7 +847,8 @@ __global__ void __launch_bounds__(kBlock) k_flow_pack(ContactSoA<Real> c, uint32
   else reinterpret_cast<V2*>(r_)[k] = V2{rp[0], rp[1]};
 }
 
-hipError_t launch_flow_links(scx_ctx* c, uint32_t C, const uint32_t* ca, const uint32_t* cb, const FlowLinks& L) {
+hipError_t launch_flow_links(scx_ctx* c, uint32_t C, const uint32_t* ca, const uint32_t* cb, const FlowLinks& L,
+                             uint32_t xcds, uint32_t per_xcd) {
   hipStream_t s = c->stream;
   const uint32_t nc = (C + kBlock - 1) / kBlock, nb = (c->n + kBlock - 1) / kBlock;
   hipError_t e = hipMemsetAsync(L.mask, 0, sizeof(unsigned long long) * ((size_t)c->n + 1), s);
@@ -699,31 +856,39 @@ hipError_t launch_flow_links(scx_ctx* c, uint32_t C, const uint32_t* ca, const u
   k_flow_colours<<<nc, kBlock, 0, s>>>(C, ca, cb, c->d.coloff, c->d.ctr, L.mask);
   k_flow_offsets<<<nb, kBlock, 0, s>>>(c->n, L.mask, L.start);
   k_flow_table<<<nc, kBlock, 0, s>>>(C, ca, cb, c->d.coloff, c->d.ctr, L.mask, L.start, L.table);
-  k_flow_links<<<nc, kBlock, 0, s>>>(C, ca, cb, c->d.coloff, c->d.ctr, L.mask, L.start, L.table, L.from, L.fin);
+  k_flow_links<<<nc, kBlock, 0, s>>>(C, ca, cb, c->d.coloff, c->d.ctr, L.mask, L.start, L.table, xcds, per_xcd, L.from,
+                                      L.fin);
   return hipGetLastError();
 }
 
-template <int D, typename Real>
-hipError_t launch_gs_flow(scx_ctx* c, GSArgs<Real> A, FlowBufs<Real> F, int blocks, bool* launched) {
+template <int D, typename Real, bool Ens>
+static hipError_t launch_flow_of(scx_ctx* c, GSArgs<Real> A, FlowBufs<Real> F, uint32_t per_xcd, bool* launched) {
   const uint32_t nc = (A.C + kBlock - 1) / kBlock;
   k_flow_pack<D, Real><<<nc, kBlock, 0, c->stream>>>(A.c, A.C, A.body, F.rec, F.r);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   // the LDS holds the records, links and impulses of as many of a workgroup's contacts as it can
   const size_t each = sizeof(Real) * (D == 3 ? 16 + 3 : 8 + 2) + sizeof(uint2);
-  const uint32_t most = (A.C + blocks - 1) / blocks + kMaxColours;  // contacts of a workgroup
+  const uint32_t most = A.C / (F.xcds * per_xcd) + 1 + kMaxColours;  // contacts of a workgroup
   F.kept = std::min<uint32_t>((most + 1) / 2 * 2, (uint32_t)(kFlowLdsMax / each) / 2 * 2);
   const size_t lds = each * F.kept;
-  const hipError_t ea = hipFuncSetAttribute((const void*)k_gs_flow<D, Real>,
+  const hipError_t ea = hipFuncSetAttribute((const void*)k_gs_flow<D, Real, Ens>,
                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (ea != hipSuccess) return ea;
   void* args[] = {&A, &F};
-  return launch_cooperative(c, (const void*)k_gs_flow<D, Real>, blocks, kFlowThreads, args, lds, c->stream, launched);
+  return launch_cooperative(c, (const void*)k_gs_flow<D, Real, Ens>, (int)(kXcds * per_xcd), kFlowThreads, args, lds,
+                            c->stream, launched);
 }
 
-template hipError_t launch_gs_flow<2, float>(scx_ctx*, GSArgs<float>, FlowBufs<float>, int, bool*);
-template hipError_t launch_gs_flow<3, float>(scx_ctx*, GSArgs<float>, FlowBufs<float>, int, bool*);
-template hipError_t launch_gs_flow<2, double>(scx_ctx*, GSArgs<double>, FlowBufs<double>, int, bool*);
-template hipError_t launch_gs_flow<3, double>(scx_ctx*, GSArgs<double>, FlowBufs<double>, int, bool*);
+template <int D, typename Real>
+hipError_t launch_gs_flow(scx_ctx* c, GSArgs<Real> A, FlowBufs<Real> F, uint32_t per_xcd, bool* launched) {
+  return A.cscene ? launch_flow_of<D, Real, true>(c, A, F, per_xcd, launched)
+                  : launch_flow_of<D, Real, false>(c, A, F, per_xcd, launched);
+}
+
+template hipError_t launch_gs_flow<2, float>(scx_ctx*, GSArgs<float>, FlowBufs<float>, uint32_t, bool*);
+template hipError_t launch_gs_flow<3, float>(scx_ctx*, GSArgs<float>, FlowBufs<float>, uint32_t, bool*);
+template hipError_t launch_gs_flow<2, double>(scx_ctx*, GSArgs<double>, FlowBufs<double>, uint32_t, bool*);
+template hipError_t launch_gs_flow<3, double>(scx_ctx*, GSArgs<double>, FlowBufs<double>, uint32_t, bool*);
 
 }  // namespace scx

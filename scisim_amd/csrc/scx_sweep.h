@@ -374,14 +374,20 @@ template <int D, typename Real>
 hipError_t launch_gs_wg(const GSArgs<Real>& A, const WgBufs<Real>& W, hipStream_t s);
 
 // Working memory of the sweeps without barriers (k_gs_flow), in colour order.
+constexpr uint32_t kFlowMaxScenes = 2048;  // an ensemble's residuals, in every workgroup's LDS
 constexpr int kFlowMaxBlocks = 256;  // one wave reads every workgroup's flag
+// Slots of side b follow those of side a, the near ones (read on one XCD alone) of both follow
+// the far ones, so that no line holds both kinds; kFlowLine consecutive ones fill at least two lines.
+constexpr uint32_t kFlowLine = 16;
+__host__ __device__ inline uint32_t flow_side(uint32_t C) { return (C + kFlowLine - 1) / kFlowLine * kFlowLine; }
 template <typename Real>
 struct FlowBufs {
   Real* rec;          // packed records
   Real* r;            // impulses: 4 (3D) or 2 (2D) Reals per contact
-  const uint32_t* from;  // per contact, 2: the slots its bodies come from (slot << 1 | sweep before)
+  const uint32_t* from;  // per contact, 2: the slots its bodies come from (slot << 2 | flags)
   const uint32_t* fin;   // per contact, 2: the slots of its bodies' last contacts
-  void* slots;        // 2 C outbox slots, in 16-byte pieces
+  void* slots;        // outbox slots, in 16-byte pieces
+  uint32_t xcds;      // XCDs that take part
   uint32_t* flags;    // per workgroup: 2 * tag + whether it holds a contact above the threshold
   void* parts;        // per workgroup: its largest residual and the tag
   uint32_t tag0;      // first tag of this launch: above every tag in slots, flags and parts
@@ -395,10 +401,11 @@ struct FlowLinks {
   uint2* from;
   uint2* fin;
 };
-hipError_t launch_flow_links(scx_ctx* c, uint32_t C, const uint32_t* ca, const uint32_t* cb, const FlowLinks& L);
-// Packs the records and launches the sweeps on `blocks` workgroups; *launched is false when a
+hipError_t launch_flow_links(scx_ctx* c, uint32_t C, const uint32_t* ca, const uint32_t* cb, const FlowLinks& L,
+                             uint32_t xcds, uint32_t per_xcd);
+// Packs the records and launches the sweeps on per_xcd workgroups of each of F.xcds XCDs; *launched is false when a
 // cooperative launch is not to be had (nothing ran).
 template <int D, typename Real>
-hipError_t launch_gs_flow(scx_ctx* c, GSArgs<Real> A, FlowBufs<Real> F, int blocks, bool* launched);
+hipError_t launch_gs_flow(scx_ctx* c, GSArgs<Real> A, FlowBufs<Real> F, uint32_t per_xcd, bool* launched);
 
 }  // namespace scx

@@ -91,3 +91,47 @@ def test_without_barriers(monkeypatch, kind, blocks, precision, limit):
     s = _scene(kind)
     prm = _params(s, precision, limit)
     _same(_run(monkeypatch, s, "", prm, 3), _run(monkeypatch, s, "flow", prm, 3, blocks))
+
+
+@pytest.mark.parametrize("kind", ["circles", "2500"])
+@pytest.mark.parametrize("xcds,blocks", [(1, 1), (1, 32), (2, 2), (8, 8), (8, 256)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_without_barriers_spread(monkeypatch, kind, xcds, blocks, precision):
+    """The slots of bodies that one XCD holds stay in its L2, the others go through to memory."""
+    print("case", kind, xcds, blocks, precision, flush=True)
+    s = _scene(kind)
+    prm = _params(s, precision, "converged")
+    ref = _run(monkeypatch, s, "", prm, 3)
+    monkeypatch.setenv("SCX_FLOW_XCDS", str(xcds))
+    _same(ref, _run(monkeypatch, s, "flow", prm, 3, blocks))
+
+
+@pytest.mark.parametrize("blocks", [None, 3, 256])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("limit", ["converged", "limit", "sparse", "stagnates"])
+def test_ensemble_without_barriers(monkeypatch, blocks, precision, limit):
+    """70 piles (more than two words of the frozen mask), most of which freeze on the way."""
+    print("case", blocks, precision, limit, flush=True)
+    cat, body_off, plane_off, mus, _ = scenes.ensemble_piles(nscenes=70, nmin=20, nmax=200, seed=4, workers=4)
+    prm = _params(cat, precision, limit)
+
+    def run(path):
+        monkeypatch.setenv("SCX_FLOW_SWEEPS", "1" if path else "0")
+        monkeypatch.delenv("SCX_FLOW_BLOCKS", raising=False)
+        if path and blocks:
+            monkeypatch.setenv("SCX_FLOW_BLOCKS", str(blocks))
+        ctx = scx.Context(3, cat["r"].size, max_planes=350)
+        try:
+            ctx.set_planes(cat["px"], cat["pn"])
+            ctx.set_bodies(cat["q"], cat["v"], cat["r"], cat["m"], inertia=cat["inertia"])
+            ctx.set_scenes(body_off, plane_off, mus)
+            out = []
+            for _ in range(3):
+                st = ctx.step(scx.step_params(**prm))
+                con = ctx.contacts()
+                out.append((st, *ctx.get_state(), con["alpha"], con["beta"], *ctx.scene_stats()))
+            return out
+        finally:
+            ctx.close()
+
+    _same(run(False), run(True))
