@@ -1526,9 +1526,7 @@ int scx_train_warm_model(scx_ctx* c, uint32_t n, const float* features, const fl
     }
     HIPC(hipMemcpyAsync(c->d.mlp_idx, idx.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice, c->stream));
     for (uint32_t b0 = 0; b0 + batch <= n; b0 += batch) {
-      HIPC(launch_mlp_gradients(c, batch, c->d.mlp_idx, b0, c->d.mlp_pool_x, c->d.mlp_pool_t));
-      HIPC(launch_mlp_adam(c, lr, ++c->d.mlp_step));
-      HIPC(launch_mlp_pack(c));
+      HIPC(launch_mlp_train(c, batch, c->d.mlp_idx, b0, c->d.mlp_pool_x, c->d.mlp_pool_t, lr, ++c->d.mlp_step));
     }
     // idx is reused by the next epoch's upload only after these launches (same stream)
     HIPC(hipStreamSynchronize(c->stream));

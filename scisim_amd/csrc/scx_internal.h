@@ -365,7 +365,8 @@ hipError_t launch_mlp_pack(scx_ctx* c);
 hipError_t launch_mlp_infer(scx_ctx* c, uint32_t n, const float* X, float* Y);
 hipError_t launch_mlp_gradients(scx_ctx* c, uint32_t nb, const uint32_t* idx, uint32_t b0, const float* X,
                                 const float* Tgt);
-hipError_t launch_mlp_adam(scx_ctx* c, float lr, uint32_t step);
+hipError_t launch_mlp_train(scx_ctx* c, uint32_t nb, const uint32_t* idx, uint32_t b0, const float* X,
+                            const float* Tgt, float lr, uint32_t step);
 int solver_max_blocks(scx_ctx* c);
 int colour_max_blocks(scx_ctx* c);
 }  // namespace scx

@@ -165,3 +165,50 @@ def test_learned_prediction_beats_the_transported_impulse_on_held_out_steps():
     assert new.sum() >= 100
     assert got_all < base_all
     assert got_new < 0.8 * base_new
+
+
+def _shuffled(n, seed, epochs):
+    """The training's sample order: one Fisher-Yates shuffle (splitmix64) per epoch."""
+    mask, state, out = (1 << 64) - 1, seed, []
+    for _ in range(epochs):
+        idx = list(range(n))
+        for i in range(n, 1, -1):
+            state = (state + 0x9E3779B97F4A7C15) & mask
+            z = ((state ^ (state >> 30)) * 0xBF58476D1CE4E5B9) & mask
+            z = ((z ^ (z >> 27)) * 0x94D049BB133111EB) & mask
+            z ^= z >> 31
+            idx[i - 1], idx[z % i] = idx[z % i], idx[i - 1]
+        out.append(idx)
+    return out
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 255, 257, 512, 513, 1030])
+def test_training_steps_are_adam_on_the_device_gradients(ctx, n):
+    """Two steps of one batch (tiles of 16 samples, 16 of them loaded ahead, twice): each is
+    Adam in FP64 on the gradients the device reports for the same samples in the same order,
+    to the rounding of a dozen FP32 operations on a step of at most the rate."""
+    rng = np.random.default_rng(n)
+    p = mlp.init(seed=n)
+    X = rng.normal(size=(n, 16)).astype(np.float32)
+    T = rng.normal(size=(n, 3)).astype(np.float32)
+    lr, b1, b2, eps = np.float32(1e-3), float(np.float32(0.9)), float(np.float32(0.999)), float(np.float32(1e-8))
+    fresh = scx.Context(3, 10, max_planes=8)
+    m = v = np.zeros(p.size)
+    want = p.astype(np.float64)
+    for step, idx in enumerate(_shuffled(n, 9, 2), 1):
+        fresh.set_warm_model(want.astype(np.float32) if step == 1 else got1)
+        g = fresh.warm_model_gradients(X[idx], T[idx])[0].astype(np.float64)
+        m, v = b1 * m + (1 - b1) * g, b2 * v + (1 - b2) * g * g
+        want = want - float(lr) * (m / (1 - b1 ** step)) / (np.sqrt(v / (1 - b2 ** step)) + eps)
+        ctx.set_warm_model(p)
+        ctx.train_warm_model(X, T, epochs=step, batch=n, lr=float(lr), seed=9)
+        got = ctx.warm_model()
+        if step == 1:
+            got1 = got
+        # 1 - b2^step keeps 24 - 10 bits of b2's rounding in FP32, half of it under the root
+        np.testing.assert_allclose(got, want, rtol=2e-7 * step, atol=float(lr) * 1e-4 * step)
+    # the weights the next pass reads are those of the parameters reported
+    fresh.set_warm_model(got)
+    a, b = fresh.warm_model_gradients(X, T), ctx.warm_model_gradients(X, T)
+    fresh.close()
+    assert np.array_equal(a[0], b[0]) and a[1] == b[1]
