@@ -219,7 +219,7 @@ int alloc_contacts(scx_ctx* c, uint32_t C) {
   HIPC(dalloc(&d.cstate, C));
   c->cap_perm = std::max<uint32_t>(C, c->cap_bodies);
   HIPC(dalloc(&d.perm, c->cap_perm));
-  HIPC(dalloc(&d.rbest, 3 * (size_t)C));
+  HIPC(dalloc(&d.rbest, 3 * ((size_t)C + 256)));
   HIPC(dalloc(&d.act_idx, 2 * (size_t)C));
   if (alloc_soa(c, d.c64, C) != SCX_OK) return SCX_E_HIP;
   if (alloc_soa(c, d.c32, C) != SCX_OK) return SCX_E_HIP;

@@ -338,11 +338,28 @@ __device__ __forceinline__ uint32_t cell_key(const GridParams& g, uint32_t x, ui
   return x + g.dims[0] * (y + g.dims[1] * z);
 }
 
+// Place of a cell in the home-cell order: tiles of 1 << tile cells a side, one after the other, and
+// row by row within a tile, so that a range of bodies is a block in space rather than a layer.
+// (The sweeps give each workgroup the contacts of such a range: 76 % of the contacts' bodies of a
+// pile of 262,144 spheres then lie in one of 256 workgroups, 42 % with rows over the whole grid.)
+template <int D>
+__device__ __forceinline__ uint32_t home_key(const GridParams& g, const uint32_t* x, uint32_t tile) {
+  uint32_t t[3], w[3];  // the tile's lower corner, its sides (the last ones of an axis are cut)
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    t[a] = a < D ? x[a] >> tile << tile : 0u;
+    w[a] = a < D ? min(1u << tile, g.dims[a] - t[a]) : 1u;
+  }
+  const uint32_t before = t[2] * g.dims[0] * g.dims[1] + w[2] * (t[1] * g.dims[0] + w[1] * t[0]);
+  return before + ((x[2] - t[2]) * w[1] + (x[1] - t[1])) * w[0] + (x[0] - t[0]);
+}
+
 // Counts over sweep positions: home cells (one per body) and covered cells (one per entry).
 template <int D>
 __global__ void __launch_bounds__(kBlock) k_cells_count(uint32_t n, const float4* __restrict__ tbox,
                                                         const GridParams* __restrict__ gp, uint32_t* __restrict__ ccnt,
-                                                        uint32_t* __restrict__ hcnt, StepCounters* __restrict__ ctr) {
+                                                        uint32_t* __restrict__ hcnt, uint32_t tile,
+                                                        StepCounters* __restrict__ ctr) {
   const uint32_t t = xcd_block() * kBlock + threadIdx.x;
   const GridParams g = *gp;
   uint32_t cnt = 0;
@@ -351,7 +368,7 @@ __global__ void __launch_bounds__(kBlock) k_cells_count(uint32_t n, const float4
     load_box32<D>(tbox, t, bl, bh);
     uint32_t lo[3], hi[3];
     cell_range_f<D>(bl, bh, g, lo, hi);
-    if (hcnt) atomicAdd(&hcnt[cell_key(g, lo[0], lo[1], lo[2])], 1u);
+    if (hcnt) atomicAdd(&hcnt[home_key<D>(g, lo, tile)], 1u);
     if (ccnt)
       for (uint32_t z = lo[2]; z <= hi[2]; ++z)
         for (uint32_t y = lo[1]; y <= hi[1]; ++y)
@@ -374,7 +391,7 @@ __global__ void __launch_bounds__(kBlock) k_entries_scatter(uint32_t n, const fl
                                                             uint32_t* __restrict__ ccnt,
                                                             const uint32_t* __restrict__ cstart,
                                                             uint32_t* __restrict__ hcnt,
-                                                            const uint32_t* __restrict__ hstart,
+                                                            const uint32_t* __restrict__ hstart, uint32_t tile,
                                                             const uint32_t* __restrict__ order_in,
                                                             uint32_t* __restrict__ order_out, uint32_t* __restrict__ ent,
                                                             uint32_t cap, StepCounters* __restrict__ ctr) {
@@ -385,9 +402,11 @@ __global__ void __launch_bounds__(kBlock) k_entries_scatter(uint32_t n, const fl
   load_box32<D>(tbox, t, bl, bh);
   uint32_t lo[3], hi[3];
   cell_range_f<D>(bl, bh, g, lo, hi);
-  const uint32_t home = cell_key(g, lo[0], lo[1], lo[2]);
-  const uint32_t k = hstart[home] + atomicSub(&hcnt[home], 1u) - 1u;
-  order_out[k] = order_in ? order_in[t] : t;
+  if (hcnt) {
+    const uint32_t home = home_key<D>(g, lo, tile);
+    const uint32_t k = hstart[home] + atomicSub(&hcnt[home], 1u) - 1u;
+    order_out[k] = order_in ? order_in[t] : t;
+  }
   if (!ccnt) return;
   for (uint32_t z = lo[2]; z <= hi[2]; ++z)
     for (uint32_t y = lo[1]; y <= hi[1]; ++y)
@@ -676,29 +695,35 @@ hipError_t launch_slots(scx_ctx* c, uint32_t n) {
 }
 
 // Home-cell sort (home_only) or full binning of the sweep-order boxes in d.tbox.
-// order_in == nullptr: the sweep order is the identity.
+// order_in == nullptr: the sweep order is the identity; order_out == nullptr: no home-cell order.
 template <int D>
 static hipError_t bin_sweep_boxes(scx_ctx* c, uint32_t n, bool home_only, const uint32_t* order_in,
-                                  uint32_t* order_out) {
+                                  uint32_t* order_out, uint32_t tile) {
   hipStream_t s = c->stream;
   DeviceBuffers& d = c->d;
   const uint32_t nblk = (n + kBlock - 1) / kBlock;
   const uint32_t cap = c->cap_cells;
   uint32_t* ccnt = home_only ? nullptr : d.cells;
   uint32_t* cstart = d.cells + (cap + 1);
-  uint32_t* hcnt = d.cells + 2 * (size_t)(cap + 1);
+  uint32_t* hcnt = order_out ? d.cells + 2 * (size_t)(cap + 1) : nullptr;
   uint32_t* hstart = d.cells + 3 * (size_t)(cap + 1);
-  hipError_t e = hipMemsetAsync(hcnt, 0, sizeof(uint32_t) * (cap + 1), s);
+  hipError_t e = hipSuccess;
+  if (hcnt) e = hipMemsetAsync(hcnt, 0, sizeof(uint32_t) * (cap + 1), s);
   if (e == hipSuccess && ccnt) e = hipMemsetAsync(ccnt, 0, sizeof(uint32_t) * (cap + 1), s);
   if (e != hipSuccess) return e;
-  k_cells_count<D><<<nblk, kBlock, 0, s>>>(n, d.tbox, d.grid, ccnt, hcnt, d.ctr);
+  k_cells_count<D><<<nblk, kBlock, 0, s>>>(n, d.tbox, d.grid, ccnt, hcnt, tile, d.ctr);
   if (ccnt) e = launch_exclusive_scan(ccnt, cstart, cap, d.scan_tmp, s);
-  if (e == hipSuccess) e = launch_exclusive_scan(hcnt, hstart, cap, d.scan_tmp, s);
+  if (e == hipSuccess && hcnt) e = launch_exclusive_scan(hcnt, hstart, cap, d.scan_tmp, s);
   if (e != hipSuccess) return e;
-  k_entries_scatter<D><<<nblk, kBlock, 0, s>>>(n, d.tbox, d.grid, ccnt, cstart, hcnt, hstart, order_in, order_out,
+  k_entries_scatter<D><<<nblk, kBlock, 0, s>>>(n, d.tbox, d.grid, ccnt, cstart, hcnt, hstart, tile, order_in, order_out,
                                                 d.ent, c->cap_entries, d.ctr);
   return hipGetLastError();
 }
+
+// Log2 of the tiles' sides in the home-cell order. Bodies of a simulation: for the sweeps (see
+// home_key). Given boxes, which have no sweeps: rows over the whole grid, in whose order the
+// neighbour search is 3 % faster.
+constexpr uint32_t kTile = 3, kRows = 31;
 
 template <int D>
 static hipError_t grid_build_dim(scx_ctx* c, uint32_t n, bool given_boxes) {
@@ -712,13 +737,13 @@ static hipError_t grid_build_dim(scx_ctx* c, uint32_t n, bool given_boxes) {
     k_bounds_partials<D><<<nblk, kBlock, 0, s>>>(n, d.aabb_min, d.aabb_max, d.red);
     k_grid_params<D><<<1, kBlock, 0, s>>>(d.red, nblk, n, c->cap_cells, d.grid, d.ctr);
     k_boxes_to_sweep<D><<<nblk, kBlock, 0, s>>>(n, nullptr, d.aabb_min, d.aabb_max, d.tbox, d.tnar);
-    e = bin_sweep_boxes<D>(c, n, true, nullptr, d.order);
+    e = bin_sweep_boxes<D>(c, n, true, nullptr, d.order, kRows);
     if (e != hipSuccess) return e;
     k_boxes_to_sweep<D><<<nblk, kBlock, 0, s>>>(n, d.order, d.aabb_min, d.aabb_max, d.tbox, d.tnar);
   } else {
     k_grid_params<D><<<1, kBlock, 0, s>>>(d.red, nblk, n, c->cap_cells, d.grid, d.ctr);
   }
-  e = bin_sweep_boxes<D>(c, n, false, d.order, d.order_next);
+  e = bin_sweep_boxes<D>(c, n, false, d.order, given_boxes ? nullptr : d.order_next, kTile);
   if (e != hipSuccess) return e;
   return hipGetLastError();
 }

@@ -197,7 +197,7 @@ struct DeviceBuffers {
   // sweep records
   ContactSoA<double> c64{};
   ContactSoA<float> c32{};
-  double* rbest = nullptr;     // 3 per contact
+  double* rbest = nullptr;     // 3 per contact, and for the 256 more places of flow_places at most
   double* partial = nullptr;   // per-block residual partials
   uint32_t* viol = nullptr;    // FP32 phase: 2 counts, 512 listed contacts, a flag (k_gs)
   uint32_t* comp_parent = nullptr;  // N: union-find parents of the component phase (k_gs)

@@ -1518,22 +1518,17 @@ static hipError_t wg_buffers(scx_ctx* c, uint32_t C, uint32_t nbodies, WgBufs<Re
 // arenas (grown when a larger contact set takes the path), and the links of this contact set
 // (shared by the two phases of a solve).
 constexpr uint32_t kFlowTagMax = 1u << 30;
-// Above kFlowMaxContacts the scattered 16-byte gathers of the slots fill the L2s' request
-// rate, and the sweeps with barriers, whose late colours stay in LDS, are as fast (420,000
-// sphere contacts: 50 against 58 us per FP32 sweep, but 200 against 125 us in FP64). Workgroups:
-// 128 contacts each up to the whole chip (34,257 sphere contacts: 21.0, 20.0 and 19.8 us per FP32
-// sweep on 64, 128 and 256 workgroups; 44.6 with barriers).
-constexpr uint32_t kFlowMinContacts = 1024, kFlowMaxContacts = 1u << 18;
+// Ahead of the sweeps with barriers at every size measured (whole solves, ms, with barriers and
+// without): spheres 16,987 contacts 15.3 and 6.2, 34,176 20.5 and 9.4, 99,626 17.1 and 8.5,
+// 423,718 30.1 and 14.9, 848,458 18.9 and 8.7, 1,283,826 18.6 and 11.8. kFlowMaxContacts bounds
+// the buffers (0.5 GB per million contacts). Workgroups: 128 contacts each, up to the CUs in use.
+constexpr uint32_t kFlowMinContacts = 1024, kFlowMaxContacts = 1u << 21;
 constexpr uint32_t kFlowContacts = 128;  // contacts of a workgroup
-// Small sets run on one XCD's CUs: every slot is then a near one (k_gs_flow), and a body's hop
-// from contact to contact costs an L2 access. From there on one XCD's 32 CUs are too few.
-// One XCD against eight, whole solves of 300 to 800 sweeps in ms: circles 3,680 contacts FP64
-// 10.1 and 11.6, 13,169 FP64 15.1 and 16.3, 24,976 FP32 5.7 and 6.4; spheres 8,495 FP64 2.8 and
-// 3.0, 10,019 FP64 11.3 and 10.9, 16,987 FP32 4.15 and 4.5, 16,987 FP64 3.35 and 2.9.
-template <int D, typename Real>
-constexpr uint32_t flow_one_xcd() {
-  return D == 2 ? 24576 : sizeof(Real) == 4 ? 16384 : 8192;
-}
+// Up to kFlowOneXcd contacts one XCD's CUs do better than all: every slot is then a near one
+// (k_gs_flow), and more bodies live in LDS. One XCD against eight, whole solves of 300 to 2,000
+// sweeps in ms: circles 13,169 contacts 20.2 and 24.8, 24,976 8.6 and 10.1; spheres 16,987 6.2
+// and 7.4, 34,176 9.4 and 11.0, 67,457 8.7 and 8.6, 99,626 11.4 and 8.5.
+constexpr uint32_t kFlowOneXcd = 1u << 16;
 
 static hipError_t flow_arena(unsigned char** p, size_t* cap, size_t need, hipStream_t s) {
   if (need <= *cap) return hipSuccess;
@@ -1552,10 +1547,11 @@ static hipError_t flow_prepare(scx_ctx* c, const GSArgs<Real>& A, uint32_t xcds,
                                FlowBufs<Real>& F) {
   DeviceBuffers& d = c->d;
   const size_t C = A.C, n = c->n;
-  const size_t links = sizeof(unsigned long long) * (n + 2) + sizeof(uint32_t) * ((n + 1) / 2 * 2) +
-                       sizeof(uint2) * 3 * C + 256;
-  const size_t rec = sizeof(Real) * (D == 3 ? 16 : 8) * C, r = sizeof(Real) * (D == 3 ? 4 : 2) * C;
-  const size_t slot = (size_t)(D == 3 ? 8 : 4) * sizeof(Real) * 4 * flow_side(A.C);  // bytes of the slots
+  const size_t N = flow_places(A.C), W = (size_t)(kFlowMaxBlocks + 1) * (kMaxColours + 1);
+  const size_t links = sizeof(unsigned long long) * (n + 2) + sizeof(uint2) * 2 * N +
+                       sizeof(uint32_t) * (2 * n + 2 * C + 2 * C + 2 * N + 2 * W + kFlowMaxBlocks);
+  const size_t rec = sizeof(Real) * (D == 3 ? 16 : 8) * N, r = sizeof(Real) * (D == 3 ? 4 : 2) * N;
+  const size_t slot = (size_t)(D == 3 ? 8 : 4) * sizeof(Real) * 4 * N;  // bytes of the slots
   const size_t sync = (size_t)kFlowMaxBlocks * (sizeof(uint32_t) + 32);
   const unsigned char* old = d.flow_links;
   hipError_t e = flow_arena(&d.flow_links, &d.cap_flow_links, links, c->stream);
@@ -1573,24 +1569,43 @@ static hipError_t flow_prepare(scx_ctx* c, const GSArgs<Real>& A, uint32_t xcds,
   F.tag0 = c->flow_tag;
   c->flow_tag += tags;
   FlowLinks L;
-  unsigned char* p = d.flow_links;
-  L.mask = reinterpret_cast<unsigned long long*>(p);
-  p += sizeof(unsigned long long) * (n + 2);
-  L.from = reinterpret_cast<uint2*>(p);
-  L.fin = L.from + C;
-  L.table = reinterpret_cast<uint32_t*>(L.fin + C);
-  L.start = L.table + 2 * C;
+  L.mask = reinterpret_cast<unsigned long long*>(d.flow_links);
+  L.from = reinterpret_cast<uint2*>(L.mask + n + 2);
+  L.fin = L.from + N;
+  uint32_t* p = reinterpret_cast<uint32_t*>(L.fin + N);
+  auto take = [&](size_t count) {
+    uint32_t* q = p;
+    p += count;
+    return q;
+  };
+  L.start = take(n);
+  L.where = take(n);
+  L.table = take(2 * C);
+  L.own = take(C);
+  L.place = take(C);
+  L.who = take(N);
+  L.scene = take(N);
+  L.lo = take(W);
+  L.beg = take(W);
+  L.homes = take(kFlowMaxBlocks);
   F.from = reinterpret_cast<const uint32_t*>(L.from);
   F.fin = reinterpret_cast<const uint32_t*>(L.fin);
+  F.beg = L.beg;
+  F.place = L.place;
+  F.who = L.who;
+  F.scene = L.scene;
   F.rec = reinterpret_cast<Real*>(d.flow_rec);
   F.r = reinterpret_cast<Real*>(d.flow_rec + rec);
   F.flags = reinterpret_cast<uint32_t*>(d.flow_slots);
   F.parts = d.flow_slots + sizeof(uint32_t) * kFlowMaxBlocks;
   F.slots = d.flow_slots + sync;
   F.xcds = xcds;
+  // A body needs about 1.5 contacts of its workgroup; the rest of the LDS serves their records.
+  F.home = std::min<uint32_t>((A.C / (xcds * per_xcd) * 3 / 4 + 64) / 16 * 16, D == 3 ? 1280 : 2560);
   if (*linked == (xcds << 16 | per_xcd)) return hipSuccess;  // the other phase's links serve
   *linked = xcds << 16 | per_xcd;
-  return launch_flow_links(c, A.C, A.c.a, A.c.b, L, xcds, per_xcd);
+  // (the contacts before those of each slot: launch_colour_sort)
+  return launch_flow_links(c, A.C, A.c.a, A.c.b, d.slot_map ? d.deg + n + 1 : nullptr, L, xcds, per_xcd, F.home);
 }
 
 template <int D, typename Real>
@@ -1645,12 +1660,12 @@ static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint
   // addressed and the tags last; ensembles of up to kFlowMaxScenes scenes
   const bool flow = free_width && !wg && c->flow_sweeps && !c->coop_unavailable && max_blocks >= (int)kXcds &&
                     A.C >= kFlowMinContacts && A.C <= kFlowMaxContacts && A.nscenes <= kFlowMaxScenes &&
-                    A.max_iters < kFlowTagMax / 4 && (uint64_t)A.C * (D == 3 ? 32 : 16) * sizeof(Real) < (1ull << 31) - 4096;
+                    A.max_iters < kFlowTagMax / 4 && (uint64_t)flow_places(A.C) * (D == 3 ? 32 : 16) * sizeof(Real) < (1ull << 31);
   // the autotuner picks among widths around the model's (not for the solves of one workgroup)
   const int phase = std::is_same<Real, double>::value ? 1 : 0;
   const bool tune = c->tuner.enabled && c->force_blocks <= 0 && !lds_path && !wg && !c->coop_unavailable;
   // one XCD's CUs up to flow_one_xcd contacts, all beyond
-  uint32_t xcds = A.C <= flow_one_xcd<D, Real>() ? 1 : kXcds;
+  uint32_t xcds = A.C <= kFlowOneXcd ? 1 : kXcds;
   if (const char* env = getenv("SCX_FLOW_XCDS")) xcds = (uint32_t)std::max(1, std::min(atoi(env), (int)kXcds));
   const int flow_most = std::min(max_blocks, kFlowMaxBlocks) / (int)kXcds * (int)xcds;
   const int width = flow ? std::max(2, std::min((int)((A.C + kFlowContacts - 1) / kFlowContacts), flow_most)) : model;
@@ -1693,15 +1708,16 @@ static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint
     if (const char* env = getenv("SCX_FLOW_BLOCKS")) fb = atoi(env);
     const uint32_t per_xcd = ((uint32_t)std::max(1, std::min(fb, flow_most)) + xcds - 1) / xcds;
     e = flow_prepare<D, Real>(c, A, xcds, per_xcd, linked, F);
-    if (e != hipSuccess) return e;
-    F.skip_early = skip_early;
-    if (A.cscene) {
-      e = hipMemsetAsync(A.scene_acc, 0, sizeof(unsigned long long) * 3 * A.nscenes, c->stream);
-      if (e != hipSuccess) return e;
+    if (e != hipSuccess && e != hipErrorOutOfMemory) return e;
+    if (e == hipSuccess) {
+      F.skip_early = skip_early;
+      if (A.cscene) e = hipMemsetAsync(A.scene_acc, 0, sizeof(unsigned long long) * 3 * A.nscenes, c->stream);
+      if (e == hipSuccess) e = launch_gs_flow<D, Real>(c, A, F, per_xcd, &launched);
+      if (e == hipSuccess && launched && tune) e = hipEventRecord(c->tuner.pend[phase].ev[1], c->stream);
+      if (e != hipSuccess || launched) return e;
+    } else {
+      (void)hipGetLastError();  // the sweeps with barriers need no such buffers
     }
-    e = launch_gs_flow<D, Real>(c, A, F, per_xcd, &launched);
-    if (e == hipSuccess && launched && tune) e = hipEventRecord(c->tuner.pend[phase].ev[1], c->stream);
-    if (e != hipSuccess || launched) return e;
   }
   c->barrier_sweeps = true;
   const void* fn = coh ? (const void*)k_gs<D, Real, true> : (const void*)k_gs<D, Real, false>;

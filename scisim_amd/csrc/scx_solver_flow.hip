@@ -1,18 +1,23 @@
 // scx_solver_flow.hip -- the sweeps of a contact set on many workgroups without barriers
 // between the colours: a contact waits only for the contacts before it on its own two bodies.
 //
-// What bounds the sweeps of a few thousand to a few hundred thousand contacts is neither
-// arithmetic nor memory but the exchange of bodies between the colours. With a grid barrier
-// per colour an interval costs 8 to 13 us (coherent gathers, the completion of scattered
-// coherent stores, the arrival and the slowest workgroup); a 16-byte store that carries its
-// own tag is seen by a polling load on another XCD after 0.4 to 0.8 us. So every contact owns
-// an outbox slot per body: it writes the body's velocities there after its update, in 16-byte
-// pieces that each end in the sweep's tag, and the next contact on that body (the order on a
-// body is the colour order, cyclic over the sweeps) polls that slot until the tag is the one
-// it waits for. No store is waited for, nothing is read that has not been written, and the
-// stores of a wave are contiguous.
-// A slot whose readers are all on the writer's XCD is stored into its L2 (430 cycles to the
-// next load, which passes the L1 by), others go through to memory (600 to 1,000 cycles).
+// What bounds the sweeps of a few thousand to a million contacts is neither arithmetic nor
+// memory but the exchange of bodies between the colours. With a grid barrier per colour an
+// interval costs 8 to 13 us (coherent gathers, the completion of scattered coherent stores,
+// the arrival and the slowest workgroup). Here a contact's successors on its two bodies wait
+// for it alone, and the way between them is as short as the split of the contacts allows:
+//   - A workgroup owns the contacts of a range of bodies that lie together, so most bodies
+//     have all their contacts in one workgroup (75 to 85 % of the contacts' bodies on a pile
+//     of 262,144 spheres over 256 workgroups). Their velocities stay in its LDS, each with the
+//     sweep and colour of its last update, for which the next contact waits.
+//   - For the other bodies every contact owns an outbox slot per body: it writes the body's
+//     velocities there after its update, in 16-byte pieces that each end in the sweep's tag,
+//     and the next contact on that body (the order on a body is the colour order, cyclic over
+//     the sweeps) polls that slot until the tag is the one it waits for. A slot whose readers
+//     are all on the writer's XCD is stored into its L2 (430 cycles to the next load, which
+//     passes the L1 by), others go through to memory (600 to 1,000 cycles).
+// No store is waited for, nothing is read that has not been written, and the stores of a wave
+// are contiguous.
 //
 // The iterates are those of the colour passes bit for bit: the order of the contacts on
 // every body is the colour order, and a contact reads nothing but its own two bodies.
@@ -68,30 +73,16 @@ struct FlowPort {
     for (int i = 0; i < NP; ++i) ok = ok && x.p[i][3] == tag;
     return ok;
   }
-  __device__ __forceinline__ static bool beyond(const Raw& x, uint32_t tag) {
-    bool b = false;
-#pragma unroll
-    for (int i = 0; i < NP; ++i) b = b || (int32_t)(x.p[i][3] - tag) > 0;
-    return b;
-  }
-  __device__ __forceinline__ static void unpack(const Raw& x, Real im, Real ii, V& v, V& w) {
+  __device__ __forceinline__ static void unpack(const Raw& x, Real* r) {
     uint32_t u[3 * NP];
 #pragma unroll
     for (int i = 0; i < 3 * NP; ++i) u[i] = x.p[i / 3][i % 3];
-    Real r[NR];
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
       if constexpr (sizeof(Real) == 8)
         r[i] = __longlong_as_double((long long)(((unsigned long long)u[2 * i + 1] << 32) | u[2 * i]));
       else
         r[i] = __uint_as_float(u[i]);
-    }
-    if constexpr (D == 3) {
-      v = V{r[0], r[1], r[2], im};
-      w = V{r[3], r[4], r[5], ii};
-    } else {
-      v = V{r[0], r[1], (Real)0, im};
-      w = V{0, 0, 0, 0};
     }
   }
   // near: every reader is on this XCD, so the store may stay in its L2
@@ -126,8 +117,9 @@ struct FlowPort {
 };
 
 // A contact ready to be updated: its record and impulse, and where its bodies come from
-// (slot << 2 | whether its own slot of that body is read on this XCD alone << 1 | whether the
-// slot is the one of the sweep before).
+// (kFlowHome: LDS entry << 9 | colour of the contact before it << 3; else: slot << 3 | whether
+// its own slot of that body is read on this XCD alone (kFlowNear); kFlowWrap: the contact before
+// it is one of the sweep before).
 template <int D, typename Real>
 struct FlowContact {
   typename Vec4<Real>::type g[kRecGroups<D>];
@@ -140,7 +132,9 @@ struct FlowContact {
 // evaluations). Ens: an ensemble; its scenes share no body, so they are independent parts of
 // one graph. A scene is frozen when an evaluation finds it below the tolerance: its contacts
 // are neither updated nor evaluated any more, its residual stays in frozen_max.
-template <int D, typename Real, bool Ens>
+// All: the LDS holds all contacts of every workgroup (no loads of records from memory, which
+// would be waited for behind the stores to the slots).
+template <int D, typename Real, bool Ens, bool All>
 __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBufs<Real> F) {
   using V = typename Vec4<Real>::type;
   using V2 = typename Vec2<Real>::type;
@@ -148,10 +142,9 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
   using Raw = typename Port::Raw;
   constexpr int kWaves = kFlowThreads / 64;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  __shared__ uint32_t s_lo[kMaxColours], s_hi[kMaxColours];  // this workgroup's contacts of each colour
-  __shared__ uint32_t s_at[kMaxColours];  // the first one's place in the workgroup's list
   __shared__ double s_red[kWaves];
   __shared__ uint32_t s_flag[2], s_skip[2], s_dead;
+  __shared__ uint32_t s_beg[kMaxColours + 1], s_rows;
   __shared__ uint32_t s_frozen[Ens ? kFlowMaxScenes / 32 : 1];           // frozen scenes
   __shared__ unsigned long long s_acc[Ens ? kFlowMaxScenes : 1];         // residuals of this workgroup's scenes
   const uint32_t tid = threadIdx.x, lane = tid & 63;
@@ -159,34 +152,27 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
   // F.xcds XCDs take part, neighbouring ranges of contacts on one XCD.
   const uint32_t per_xcd = gridDim.x / kXcds;
   if (blockIdx.x % kXcds >= F.xcds) return;
-  const uint32_t C = A.C, Cp = flow_side(C), G = F.xcds * per_xcd;
+  const uint32_t N = flow_places(A.C), G = F.xcds * per_xcd;
   const uint32_t wg = blockIdx.x % kXcds * per_xcd + blockIdx.x / kXcds;
   const uint32_t ncol = A.ctr->ncolours;
-  for (uint32_t c = tid; c < ncol; c += kFlowThreads) {
-    const uint32_t o = A.coloff[c], n = A.coloff[c + 1] - o;
-    s_lo[c] = o + (uint32_t)((uint64_t)n * wg / G);
-    s_hi[c] = o + (uint32_t)((uint64_t)n * (wg + 1) / G);
-  }
+  const uint32_t* beg = F.beg + (size_t)wg * (kMaxColours + 1);
+  const uint32_t first = beg[0];
+  for (uint32_t c = tid; c <= ncol; c += kFlowThreads) s_beg[c] = beg[c];
   if (tid == 0) s_flag[0] = s_flag[1] = s_skip[0] = s_skip[1] = s_dead = 0;
   if (Ens)
     for (uint32_t w = tid; w < kFlowMaxScenes / 32; w += kFlowThreads) s_frozen[w] = 0;
-  __syncthreads();
-  if (tid == 0) {
-    uint32_t n = 0;
-    for (uint32_t c = 0; c < ncol; ++c) {
-      s_at[c] = n;
-      n += s_hi[c] - s_lo[c];
-    }
-  }
-  __syncthreads();
   // The first kept contacts of the workgroup's list (its wide colours) keep their records,
   // impulses and links in LDS.
   const uint32_t kept = F.kept;
-  V* l_rec = reinterpret_cast<V*>(lds);
+  Real* l_body = reinterpret_cast<Real*>(lds);
+  uint32_t* l_tag = reinterpret_cast<uint32_t*>(l_body + (size_t)Port::NR * F.home);
+  // rows of up to 64 contacts of a colour, in colour order: first place, contacts << 8 | colour
+  uint2* l_row = reinterpret_cast<uint2*>(l_tag + F.home);
+  V* l_rec = reinterpret_cast<V*>(l_row + F.rows);
   uint2* l_from = reinterpret_cast<uint2*>(l_rec + (size_t)kRecGroups<D> * kept);
   Real* l_r = reinterpret_cast<Real*>(l_from + kept);
   Port P;
-  P.rs = __builtin_amdgcn_make_buffer_rsrc(F.slots, (short)0, (int)(4u * Cp * (uint32_t)(16 * Port::NP)), 0x00020000);
+  P.rs = __builtin_amdgcn_make_buffer_rsrc(F.slots, (short)0, (int)(4u * N * (uint32_t)(16 * Port::NP)), 0x00020000);
   const __amdgpu_buffer_rsrc_t frs = __builtin_amdgcn_make_buffer_rsrc(F.flags, (short)0, (int)(4u * kFlowMaxBlocks), 0x00020000);
   const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(F.parts, (short)0, (int)(32u * kFlowMaxBlocks), 0x00020000);
   uint32_t tag = F.tag0;  // of the sweep under way
@@ -196,10 +182,33 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
   uint32_t nex = 0;
   bool one_l2 = false;    // the workgroups dealt to an XCD are on one XCD
 
-  // contact j, entry i of the workgroup's list
-  auto load = [&](uint32_t j, uint32_t i, FlowContact<D, Real>& L) __attribute__((always_inline)) {
-    if (Ens) L.scene = A.cscene[j];
-    if (i < kept) {
+  for (uint32_t i = tid; i < F.home; i += kFlowThreads) l_tag[i] = (tag - 2u) << kFlowColourBits;  // no contact waits for it
+  __syncthreads();
+  if (tid < 64) {
+    const uint32_t n = lane < ncol ? s_beg[lane + 1] - s_beg[lane] : 0u, rows = (n + 63) / 64;
+    uint32_t upto = rows;
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t y = (uint32_t)__shfl_up((int)upto, d, 64);
+      if ((int)lane >= d) upto += y;
+    }
+    for (uint32_t r = 0; r < rows; ++r)
+      l_row[upto - rows + r] = make_uint2(s_beg[lane] + 64 * r, min(64u, n - 64 * r) << 8 | lane);
+    // every wave has as many rows, some of them empty
+    const uint32_t all = (uint32_t)__shfl((int)upto, 63, 64), padded = max(1u, (all + kWaves - 1) / kWaves) * kWaves;
+    if (all + lane < padded) l_row[all + lane] = make_uint2(first, 0u);
+    if (lane == 0) s_rows = padded;
+  }
+  __syncthreads();
+  const uint32_t nrows = s_rows, wave = tid >> 6;
+  auto row = [&](uint32_t r) {
+    const uint2 d = l_row[r];
+    return make_uint2((uint32_t)__builtin_amdgcn_readfirstlane((int)d.x), (uint32_t)__builtin_amdgcn_readfirstlane((int)d.y));
+  };
+  // the contact at place j
+  auto load = [&](uint32_t j, FlowContact<D, Real>& L) __attribute__((always_inline)) {
+    const uint32_t i = j - first;
+    if (Ens) L.scene = F.scene[j];
+    if (All || i < kept) {
 #pragma unroll
       for (int g = 0; g < kRecGroups<D>; ++g) L.g[g] = l_rec[(size_t)g * kept + i];
       const uint2 f = l_from[i];
@@ -212,7 +221,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
     }
     const V* rec = reinterpret_cast<const V*>(F.rec);
 #pragma unroll
-    for (int g = 0; g < kRecGroups<D>; ++g) L.g[g] = rec[(size_t)g * C + j];
+    for (int g = 0; g < kRecGroups<D>; ++g) L.g[g] = rec[(size_t)g * N + j];
     const uint2 f = reinterpret_cast<const uint2*>(F.from)[j];
     L.from_a = f.x;
     L.from_b = f.y;
@@ -224,8 +233,9 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
       L.r[0] = r.x, L.r[1] = r.y, L.r[2] = 0;
     }
   };
-  auto store_r = [&](uint32_t j, uint32_t i, const Real* r) {
-    if (i < kept) {
+  auto store_r = [&](uint32_t j, const Real* r) {
+    const uint32_t i = j - first;
+    if (All || i < kept) {
 #pragma unroll
       for (int d = 0; d < D; ++d) l_r[(size_t)d * kept + i] = r[d];
     } else if constexpr (D == 3) {
@@ -234,62 +244,117 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
       reinterpret_cast<V2*>(F.r)[j] = V2{r[0], r[1]};
     }
   };
-  // the slot that contact j writes for a body: near ones after the far ones
+  // the slot that the contact at place j writes for a body: near ones after the far ones
   auto own_slot = [&](uint32_t j, uint32_t side, uint32_t from) {
-    return j + (side ? Cp : 0u) + ((from & 2u) ? 2u * Cp : 0u);
+    return j + (side ? N : 0u) + ((from & kFlowNear) ? 2u * N : 0u);
   };
-  // waits until two slots carry their tags (b only with hasb). The first look reads them
-  // whole; while one is not there, only its last piece's tag is polled, at intervals: the
-  // polls of the waiting waves would otherwise hold up the loads of those that work.
-  auto wait_two = [&](uint32_t sa, uint32_t ta, bool hasb, uint32_t sb, uint32_t tb, Raw& xa, Raw& xb) __attribute__((always_inline)) {
-    sb = hasb ? sb : sa;
-    tb = hasb ? tb : ta;
-    bool ok = false;
-    for (uint32_t n = 0; !ok && !dead;) {
-      asm volatile("" ::: "memory");  // each round reads memory again
-      P.ld(sa, xa);
-      P.ld(sb, xb);
-      ok = Port::is(xa, ta) && Port::is(xb, tb);
-      for (bool here = ok; !here && !dead;) {
-        __builtin_amdgcn_s_sleep(1);
-        asm volatile("" ::: "memory");
-        here = P.tag(sa) == ta;
-        here = P.tag(sb) == tb && here;
-        if (++n >= kSpinLimit) dead = true;
-      }
+  // Bodies in LDS. A wave's LDS accesses are carried out in their order: a writer stores the
+  // velocities before the tag, a reader loads the tag before the velocities.
+  auto home_tag = [&](uint32_t word, uint32_t t) { return t << kFlowColourBits | ((word >> 3) & (kMaxColours - 1)); };
+  auto home_ld = [&](uint32_t word, Real* x) __attribute__((always_inline)) {
+    const uint32_t e = word >> (3 + kFlowColourBits);
+    const uint32_t t = l_tag[e];
+    asm volatile("" ::: "memory");
+    const V2* p = reinterpret_cast<const V2*>(l_body + (size_t)Port::NR * e);
+#pragma unroll
+    for (int i = 0; i < Port::NR / 2; ++i) {
+      const V2 y = p[i];
+      x[2 * i] = y.x, x[2 * i + 1] = y.y;
+    }
+    return t;
+  };
+  auto home_st = [&](uint32_t word, const V& v, const V& w, uint32_t col) __attribute__((always_inline)) {
+    const uint32_t e = word >> (3 + kFlowColourBits);
+    V2* p = reinterpret_cast<V2*>(l_body + (size_t)Port::NR * e);
+    p[0] = V2{v.x, v.y};
+    if constexpr (D == 3) {
+      p[1] = V2{v.z, w.x};
+      p[2] = V2{w.y, w.z};
+    }
+    asm volatile("" ::: "memory");
+    l_tag[e] = tag << kFlowColourBits | col;
+  };
+  auto as_body = [&](const Real* x, Real im, Real ii, V& v, V& w) __attribute__((always_inline)) {
+    if constexpr (D == 3) {
+      v = V{x[0], x[1], x[2], im};
+      w = V{x[3], x[4], x[5], ii};
+    } else {
+      v = V{x[0], x[1], (Real)0, im};
+      w = V{0, 0, 0, 0};
     }
   };
-  auto update = [&](uint32_t j, uint32_t i, const FlowContact<D, Real>& L, bool init, Real* rbest) __attribute__((always_inline)) {
+  // Looks at two bodies under the tags ta and tb; pa, pb: whether they are still to come. Only
+  // what is still to come is read (and the slots whole: a poll that finds the tag has the body).
+  auto look = [&](uint32_t wa, uint32_t ta, bool& pa, uint32_t wb, uint32_t tb, bool& pb, Real* xa, Real* xb) __attribute__((always_inline)) {
+    const bool ha = pa && (wa & kFlowHome), hb = pb && (wb & kFlowHome), sa = pa && !ha, sb = pb && !hb;
+    asm volatile("" ::: "memory");  // each look reads memory again
+    if (__any(sa || sb)) {  // (a wave with all its bodies in LDS does not wait for its stores to slots)
+      Raw ra, rb;
+      if (sa) P.ld(wa >> 3, ra);
+      if (sb) P.ld(wb >> 3, rb);
+      if (ha) pa = home_ld(wa, xa) != home_tag(wa, ta);
+      if (hb) pb = home_ld(wb, xb) != home_tag(wb, tb);
+      if (sa) {
+        pa = !Port::is(ra, ta);
+        Port::unpack(ra, xa);
+      }
+      if (sb) {
+        pb = !Port::is(rb, tb);
+        Port::unpack(rb, xb);
+      }
+      return;
+    }
+    if (ha) pa = home_ld(wa, xa) != home_tag(wa, ta);
+    if (hb) pb = home_ld(wb, xb) != home_tag(wb, tb);
+  };
+  auto wait_two = [&](uint32_t wa, uint32_t ta, bool hasb, uint32_t wb, uint32_t tb, Real* xa, Real* xb) __attribute__((always_inline)) {
+    bool pa = true, pb = hasb;
+    for (uint32_t n = 0; (pa || pb) && !dead;) {
+      look(wa, ta, pa, wb, tb, pb, xa, xb);
+      if (++n >= kSpinLimit) dead = true;
+    }
+  };
+  auto update = [&](uint32_t j, uint32_t col, const FlowContact<D, Real>& L, bool init, Real* rbest) __attribute__((always_inline)) {
     const bool hasb = L.from_b != kNoBody;
     Loaded<D, Real> ld;
     Real im[4];
     unpack_rec<D, Real>(L.g, hasb, ld.R, im);
     ld.r[0] = L.r[0], ld.r[1] = L.r[1], ld.r[2] = L.r[2];
-    Raw xa, xb;
-    wait_two(L.from_a >> 2, tag - (L.from_a & 1u), hasb, L.from_b >> 2, tag - (L.from_b & 1u), xa, xb);
+    Real xa[Port::NR], xb[Port::NR];
+#pragma unroll
+    for (int i = 0; i < Port::NR; ++i) xb[i] = 0;
+    wait_two(L.from_a, tag - (L.from_a & kFlowWrap), hasb, L.from_b, tag - (L.from_b & kFlowWrap), xa, xb);
     V b[4];
-    Port::unpack(xa, im[0], im[2], b[0], b[1]);
-    Port::unpack(xb, im[1], im[3], b[2], b[3]);
+    as_body(xa, im[0], im[2], b[0], b[1]);
+    as_body(xb, im[1], im[3], b[2], b[3]);
     Real rn[3] = {0, 0, 0};
     update_core<D, Real>(
         ld, init, rbest, 0, 2, [&](size_t i) { return b[i]; }, [&](size_t i, const V& x) { b[i] = x; },
         [&](int d, Real x) { rn[d] = x; });
-    P.st(own_slot(j, 0, L.from_a), b[0], b[1], tag, one_l2 && (L.from_a & 2u));
-    if (hasb) P.st(own_slot(j, 1, L.from_b), b[2], b[3], tag, one_l2 && (L.from_b & 2u));
-    if (!init) store_r(j, i, rn);
+    if (L.from_a & kFlowHome) home_st(L.from_a, b[0], b[1], col);
+    else P.st(own_slot(j, 0, L.from_a), b[0], b[1], tag, one_l2 && (L.from_a & kFlowNear));
+    if (hasb) {
+      if (L.from_b & kFlowHome) home_st(L.from_b, b[2], b[3], col);
+      else P.st(own_slot(j, 1, L.from_b), b[2], b[3], tag, one_l2 && (L.from_b & kFlowNear));
+    }
+    if (!init) store_r(j, rn);
   };
   // squared residual of contact j on the bodies' final velocities of this sweep; false when a
   // body has already moved on to a later sweep (only in the check of a noted contact)
   auto residual = [&](const FlowContact<D, Real>& L, uint2 fin, bool check, double& e) __attribute__((always_inline)) {
     const bool hasb = fin.y != kNoBody;
-    Raw xa, xb;
-    bool ok = false, late = false;
+    Real xa[Port::NR], xb[Port::NR];
+#pragma unroll
+    for (int i = 0; i < Port::NR; ++i) xb[i] = 0;
+    bool ok = false, late = false, pa = true, pb = hasb;
     for (uint32_t n = 0; !ok && !late && !dead; ++n) {
-      asm volatile("" ::: "memory");
-      P.ld(fin.x, xa);
-      P.ld(hasb ? fin.y : fin.x, xb);
-      ok = Port::is(xa, tag) && (!hasb || Port::is(xb, tag));
-      if (check && !ok) late = Port::beyond(xa, tag) || (hasb && Port::beyond(xb, tag));
+      look(fin.x, tag, pa, fin.y, tag, pb, xa, xb);
+      ok = !pa && !pb;
+      if (check && !ok) {
+        // (a body in LDS moves on with this workgroup only)
+        if (!(fin.x & kFlowHome)) late = pa && (int32_t)(P.tag(fin.x >> 3) - tag) > 0;
+        if (hasb && !(fin.y & kFlowHome)) late = late || (pb && (int32_t)(P.tag(fin.y >> 3) - tag) > 0);
+      }
       if (n >= kSpinLimit) dead = true;
     }
     if (!ok) return false;
@@ -298,8 +363,8 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
     unpack_rec<D, Real>(L.g, hasb, R, im);
     const V z = {0, 0, 0, 0};
     V va, wa, vb = z, wb = z;
-    Port::unpack(xa, im[0], im[2], va, wa);
-    if (hasb) Port::unpack(xb, im[1], im[3], vb, wb);
+    as_body(xa, im[0], im[2], va, wa);
+    if (hasb) as_body(xb, im[1], im[3], vb, wb);
     if (A.phase == 1) {
       float u[3];
       rel_vel<D, float, Real>(R, va, wa, vb, wb, u);
@@ -316,19 +381,28 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
   auto frozen = [&](const FlowContact<D, Real>& L) {
     return Ens && ((s_frozen[L.scene >> 5] >> (L.scene & 31)) & 1u) != 0;
   };
-  // every contact of this workgroup, in colour order: contact j, entry i of its list
+  // every contact of this wave, in colour order: place j, colour c
   auto for_each = [&](auto&& f) {
-    for (uint32_t c = 0; c < ncol; ++c)
-      for (uint32_t j = s_lo[c] + tid; j < s_hi[c]; j += kFlowThreads) f(j, s_at[c] + (j - s_lo[c]));
+    for (uint32_t r = wave; r < nrows; r += kWaves) {
+      const uint2 d = row(r);
+      if (lane < d.y >> 8) f(d.x + lane, d.y & 0xFFu);
+    }
   };
-  // the bodies' start velocities into the slots of their last contacts
+  // whether the contact (place j, colour c) is the last on its body of a side
+  auto is_last = [&](uint32_t j, uint32_t c, uint32_t side, uint32_t from, uint32_t fin) {
+    if (fin == kNoBody) return false;
+    if (fin & kFlowHome) return ((fin >> 3) & (kMaxColours - 1)) == c;
+    return fin >> 3 == own_slot(j, side, from);
+  };
+  // the bodies' start velocities, as their last contacts of the sweep before leave them
   auto start_bodies = [&](bool reset) {
-    for_each([&](uint32_t j, uint32_t) {
+    for_each([&](uint32_t j, uint32_t c) {
       const uint2 fin = reinterpret_cast<const uint2*>(F.fin)[j], fr = reinterpret_cast<const uint2*>(F.from)[j];
+      const uint32_t k = F.who[j];
       for (int side = 0; side < 2; ++side) {
-        const uint32_t own = own_slot(j, side, side ? fr.y : fr.x);
-        if ((side ? fin.y : fin.x) != own) continue;
-        const uint32_t sl = side ? A.c.b[j] : A.c.a[j];
+        const uint32_t word = side ? fr.y : fr.x;
+        if (!is_last(j, c, side, word, side ? fin.y : fin.x)) continue;
+        const uint32_t sl = side ? A.c.b[k] : A.c.a[k];
         V v, w = {0, 0, 0, 0};
         if (reset) {
           const uint32_t i = A.sid ? A.sid[sl] : sl;
@@ -342,15 +416,16 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
           v = rec[0];
           if (D == 3) w = rec[1];
         }
-        P.st(own, v, w, tag, one_l2 && ((side ? fr.y : fr.x) & 2u));
+        if (word & kFlowHome) home_st(word, v, w, c);
+        else P.st(own_slot(j, side, word), v, w, tag, one_l2 && (word & kFlowNear));
       }
     });
   };
   auto apply = [&]() {
-    for_each([&](uint32_t j, uint32_t i) {
+    for_each([&](uint32_t j, uint32_t c) {
       FlowContact<D, Real> L;
-      load(j, i, L);
-      update(j, i, L, true, nullptr);
+      load(j, L);
+      update(j, c, L, true, nullptr);
     });
   };
   // the largest of the workgroups' values published under the current tag, the same in every
@@ -393,7 +468,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
   };
   // the largest residual of the sweep just done over all workgroups, the same in every thread;
   // a thread also notes the largest of its contacts at or above `capture` (>= 0)
-  uint32_t noted = kNoBody, noted_i = 0;
+  uint32_t noted = kNoBody;
   uint2 noted_fin = make_uint2(0, 0);
   const double stop = (A.phase == 1) ? 0.5 * A.tol : A.tol;
   uint32_t nev = 0;  // evaluations
@@ -412,9 +487,9 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
       for (uint32_t sc = tid; sc < A.nscenes; sc += kFlowThreads) s_acc[sc] = 0ull;
       __syncthreads();
     }
-    for_each([&](uint32_t j, uint32_t i) {
+    for_each([&](uint32_t j, uint32_t) {
       FlowContact<D, Real> L;
-      load(j, i, L);
+      load(j, L);
       if (frozen(L)) return;
       const uint2 fin = reinterpret_cast<const uint2*>(F.fin)[j];
       double e = 0.0;
@@ -422,7 +497,6 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
       if (Ens && e > 0.0) atomicMax(s_acc + L.scene, (unsigned long long)__double_as_longlong(e));
       if (capture >= 0.0 && e >= capture && e > m) {
         noted = j;
-        noted_i = i;
         noted_fin = fin;
       }
       m = fmax(m, e);
@@ -472,11 +546,12 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
   if (A.phase == 1) max_iters = max(1u, max_iters - max_iters / 4);
   if (A.phase == 2) max_iters = (A.ctr->sweeps_fp32 < max_iters) ? max_iters - A.ctr->sweeps_fp32 : 0u;
   const bool track_best = A.phase != 1;
-  for_each([&](uint32_t j, uint32_t i) {
+  for_each([&](uint32_t j, uint32_t) {
+    const uint32_t i = j - first;
     if (i >= kept) return;
     const V* rec = reinterpret_cast<const V*>(F.rec);
 #pragma unroll
-    for (int g = 0; g < kRecGroups<D>; ++g) l_rec[(size_t)g * kept + i] = rec[(size_t)g * C + j];
+    for (int g = 0; g < kRecGroups<D>; ++g) l_rec[(size_t)g * kept + i] = rec[(size_t)g * N + j];
     l_from[i] = reinterpret_cast<const uint2*>(F.from)[j];
 #pragma unroll
     for (int d = 0; d < D; ++d) l_r[(size_t)d * kept + i] = F.r[(size_t)(D == 3 ? 4 : 2) * j + d];
@@ -551,7 +626,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
         bool above = false;
         if (noted != kNoBody) {
           FlowContact<D, Real> L;
-          load(noted, noted_i, L);
+          load(noted, L);
           double e = 0.0;
           above = residual(L, noted_fin, true, e) && e >= th;
         }
@@ -613,29 +688,29 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
       }
       return false;
     };
-    // One pass: kFlowThreads contacts of a colour from position pos, held in `use`; the next
-    // pass's records are loaded into `fill` first, behind the wait and the update.
-    uint32_t col = 0, pos = s_lo[0];
+    // One pass: a row, held in `use`; the records of the wave's next row are loaded into `fill`
+    // first, behind the wait and the update. The rows are dealt to the waves in turn, so the
+    // late colours, of a row or less, don't all fall to one wave.
+    uint32_t r = wave;
+    uint2 cur = row(wave);
     auto pass = [&](const FlowContact<D, Real>& use, FlowContact<D, Real>& fill) __attribute__((always_inline)) {
       dead = __any(dead);
-      const uint32_t j = pos + tid, hi = s_hi[col];
-      const bool last = pos + kFlowThreads >= hi, sweep_done = last && col + 1 == ncol;
-      const uint32_t ncol_ = sweep_done ? 0u : last ? col + 1 : col;
-      const uint32_t npos = last ? s_lo[ncol_] : pos + kFlowThreads;
-      const bool next = npos + tid < s_hi[ncol_], self = npos == pos;
-      const uint32_t i = s_at[col] + (j - s_lo[col]), ni = s_at[ncol_] + (npos + tid - s_lo[ncol_]);
-      if (next && !self) load(npos + tid, ni, fill);
-      if (j < hi) {
+      const bool sweep_done = r + kWaves >= nrows, self = nrows == kWaves;
+      r = sweep_done ? wave : r + kWaves;
+      const uint2 nxt = row(r);
+      const uint32_t j = cur.x + lane;
+      const bool next = lane < nxt.y >> 8;
+      if (next && !self) load(nxt.x + lane, fill);
+      if (lane < cur.y >> 8) {
         Real* rb = copy ? A.rbest + 3 * (size_t)j : nullptr;
         if (!frozen(use)) {
-          update(j, i, use, false, rb);
+          update(j, cur.y & 0xFFu, use, false, rb);
         } else if (rb) {
           for (int d = 0; d < 3; ++d) rb[d] = use.r[d];
         }
       }
-      if (next && self) load(npos + tid, ni, fill);  // a single pass: the impulse just stored
-      col = ncol_;
-      pos = npos;
+      if (next && self) load(nxt.x + lane, fill);  // a single row: the impulse just stored
+      cur = nxt;
       return sweep_done;
     };
     auto sweep_over = [&]() __attribute__((always_inline)) {
@@ -648,7 +723,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
       return false;
     };
     begin_sweep();
-    if (s_lo[0] + tid < s_hi[0]) load(s_lo[0] + tid, tid, c0);
+    if (lane < cur.y >> 8) load(cur.x + lane, c0);
     if constexpr (Ens) {  // one copy of the larger evaluation
       for (bool odd = false;; odd = !odd)
         if ((odd ? pass(c1, c0) : pass(c0, c1)) && sweep_over()) break;
@@ -663,10 +738,10 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
       if (track_best && !copy_pending) {
         // the best iterate and its velocities: v0, then its impulses in colour order, once
         // every workgroup is through with the last sweep's slots
-        for_each([&](uint32_t j, uint32_t i) {
-          if (Ens && ((s_frozen[A.cscene[j] >> 5] >> (A.cscene[j] & 31)) & 1u)) return;  // keeps its impulses
+        for_each([&](uint32_t j, uint32_t) {
+          if (Ens && ((s_frozen[F.scene[j] >> 5] >> (F.scene[j] & 31)) & 1u)) return;  // keeps its impulses
           const Real r[3] = {A.rbest[3 * (size_t)j], A.rbest[3 * (size_t)j + 1], A.rbest[3 * (size_t)j + 2]};
-          store_r(j, i, r);
+          store_r(j, r);
         });
         ++tag;
         (void)exchange(0.0);
@@ -679,20 +754,27 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
   }
   wait_stores();
   // impulses, and the velocities of the bodies whose last contact is here
-  for_each([&](uint32_t j, uint32_t i) {
+  for_each([&](uint32_t j, uint32_t c) {
     FlowContact<D, Real> L;
-    load(j, i, L);
-    for (int d = 0; d < D; ++d) A.c.r[3 * (size_t)j + d] = L.r[d];
+    load(j, L);
+    const uint32_t k = F.who[j];
+    for (int d = 0; d < D; ++d) A.c.r[3 * (size_t)k + d] = L.r[d];
     const uint2 fin = reinterpret_cast<const uint2*>(F.fin)[j];
     for (int side = 0; side < 2; ++side) {
-      const uint32_t own = own_slot(j, side, side ? L.from_b : L.from_a);
-      if ((side ? fin.y : fin.x) != own) continue;
-      const uint32_t sl = side ? A.c.b[j] : A.c.a[j];
-      Raw x;
-      P.ld(own, x);
+      const uint32_t word = side ? L.from_b : L.from_a;
+      if (!is_last(j, c, side, word, side ? fin.y : fin.x)) continue;
+      const uint32_t sl = side ? A.c.b[k] : A.c.a[k];
+      Real x[Port::NR];
+      if (word & kFlowHome) {
+        (void)home_ld(word, x);
+      } else {
+        Raw raw;
+        P.ld(own_slot(j, side, word), raw);
+        Port::unpack(raw, x);
+      }
       V v, w;
       V* rec = reinterpret_cast<V*>(A.body) + (size_t)kBodyVecs<D> * sl;
-      Port::unpack(x, rec[0].w, (D == 3) ? rec[D == 3].w : (Real)0, v, w);
+      as_body(x, rec[0].w, (D == 3) ? rec[D == 3].w : (Real)0, v, w);
       rec[0] = v;
       if (D == 3) rec[1] = w;
     }
@@ -725,20 +807,77 @@ __device__ __forceinline__ uint32_t colour_of(const uint32_t* off, uint32_t ncol
   return lo;
 }
 
+// The workgroup of contact k (colour c): with first, the number of contacts before those of
+// each first body in the order of the bodies (neighbours are near each other in it, and the
+// contacts of a colour are sorted by it), the contacts of an equal share of them; else equal
+// shares of each colour. Either way it does not fall within a colour.
+__device__ __forceinline__ uint32_t flow_owner(uint32_t k, uint32_t a, uint32_t C, uint32_t o0, uint32_t o1,
+                                               const uint32_t* first, uint32_t G) {
+  if (first) return (uint32_t)((uint64_t)first[a] * G / C);
+  return (uint32_t)((((uint64_t)(k - o0) + 1) * G - 1) / (o1 - o0));
+}
+
 __global__ void __launch_bounds__(kBlock) k_flow_colours(uint32_t C, const uint32_t* __restrict__ ca,
                                                          const uint32_t* __restrict__ cb,
                                                          const uint32_t* __restrict__ coloff,
                                                          const StepCounters* __restrict__ ctr,
-                                                         unsigned long long* __restrict__ mask) {
+                                                         const uint32_t* __restrict__ first, uint32_t G,
+                                                         unsigned long long* __restrict__ mask,
+                                                         uint32_t* __restrict__ own) {
   __shared__ uint32_t off[kMaxColours + 1];
   const uint32_t ncol = ctr->ncolours;
   for (uint32_t c = threadIdx.x; c <= ncol; c += kBlock) off[c] = coloff[c];
   __syncthreads();
   const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
   if (k >= C) return;
-  const unsigned long long m = 1ull << colour_of(off, ncol, k);
+  const uint32_t c = colour_of(off, ncol, k);
+  const unsigned long long m = 1ull << c;
   atomicOr(&mask[ca[k]], m);
   if (cb[k] != kNoBody) atomicOr(&mask[cb[k]], m);
+  own[k] = flow_owner(k, ca[k], C, off[c], off[c + 1], first, G);
+}
+
+// lo[w][c]: the first contact of colour c that belongs to workgroup w or a later one.
+__global__ void __launch_bounds__(kBlock) k_flow_ranges(uint32_t G, const uint32_t* __restrict__ coloff,
+                                                        const StepCounters* __restrict__ ctr,
+                                                        const uint32_t* __restrict__ own, uint32_t* __restrict__ lo) {
+  const uint32_t c = blockIdx.x;
+  if (c >= ctr->ncolours) return;
+  const uint32_t o0 = coloff[c], o1 = coloff[c + 1];
+  for (uint32_t w = threadIdx.x; w <= G; w += kBlock) {
+    uint32_t a = o0, b = o1;
+    while (a < b) {
+      const uint32_t mid = (a + b) >> 1;
+      if (own[mid] < w) a = mid + 1;
+      else b = mid;
+    }
+    lo[(size_t)w * (kMaxColours + 1) + c] = a;
+  }
+}
+
+// beg[w][c]: the place of workgroup w's first contact of colour c (c = ncolours: the end).
+// Workgroup after workgroup, a line's worth of places free between the XCDs.
+__global__ void __launch_bounds__(kMaxColours) k_flow_places(uint32_t per_xcd, const uint32_t* __restrict__ coloff,
+                                                             const StepCounters* __restrict__ ctr,
+                                                             const uint32_t* __restrict__ lo,
+                                                             uint32_t* __restrict__ beg,
+                                                             uint32_t* __restrict__ homes) {
+  static_assert(kMaxColours == 64, "one wave, a lane per colour");
+  const uint32_t w = blockIdx.x, c = threadIdx.x, ncol = ctr->ncolours;
+  const uint32_t* l = lo + (size_t)w * (kMaxColours + 1);
+  uint32_t before = c < ncol ? l[c] - coloff[c] : 0u;  // contacts of earlier workgroups
+  const uint32_t mine = c < ncol ? l[kMaxColours + 1 + c] - l[c] : 0u;
+  uint32_t upto = mine;
+  for (int d = 1; d < 64; d <<= 1) {
+    before += (uint32_t)__shfl_xor((int)before, d, 64);
+    const uint32_t y = (uint32_t)__shfl_up((int)upto, d, 64);
+    if ((int)c >= d) upto += y;
+  }
+  uint32_t* o = beg + (size_t)w * (kMaxColours + 1);
+  const uint32_t base = before + w / per_xcd * kFlowLine;
+  o[c] = base + upto - mine;
+  if (c == 63) o[64] = base + upto;
+  if (c == 0) homes[w] = 0;
 }
 
 // Start of each body's entries in the table (any order of the bodies); mask[n] counts them.
@@ -754,24 +893,59 @@ __global__ void __launch_bounds__(kBlock) k_flow_offsets(uint32_t n, unsigned lo
   if (b < n) start[b] = s_base + before;
 }
 
-// The body's contact of this colour (its outbox slot: k for side a, flow_side(C) + k for side b).
+// The body's contact of each of its colours (contact, its side in the top bit), and the
+// contacts' places.
 __global__ void __launch_bounds__(kBlock) k_flow_table(uint32_t C, const uint32_t* __restrict__ ca,
                                                        const uint32_t* __restrict__ cb,
                                                        const uint32_t* __restrict__ coloff,
                                                        const StepCounters* __restrict__ ctr,
                                                        const unsigned long long* __restrict__ mask,
                                                        const uint32_t* __restrict__ start,
-                                                       uint32_t* __restrict__ table) {
+                                                       const uint32_t* __restrict__ own,
+                                                       const uint32_t* __restrict__ lo,
+                                                       const uint32_t* __restrict__ beg,
+                                                       uint32_t* __restrict__ table, uint32_t* __restrict__ place,
+                                                       uint32_t* __restrict__ who) {
   __shared__ uint32_t off[kMaxColours + 1];
   const uint32_t ncol = ctr->ncolours;
   for (uint32_t c = threadIdx.x; c <= ncol; c += kBlock) off[c] = coloff[c];
   __syncthreads();
   const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
   if (k >= C) return;
-  const unsigned long long below = (1ull << colour_of(off, ncol, k)) - 1ull;
+  const uint32_t c = colour_of(off, ncol, k);
+  const unsigned long long below = (1ull << c) - 1ull;
   const uint32_t a = ca[k], b = cb[k];
   table[start[a] + (uint32_t)__popcll(mask[a] & below)] = k;
-  if (b != kNoBody) table[start[b] + (uint32_t)__popcll(mask[b] & below)] = flow_side(C) + k;
+  if (b != kNoBody) table[start[b] + (uint32_t)__popcll(mask[b] & below)] = 0x80000000u | k;
+  const size_t q = (size_t)own[k] * (kMaxColours + 1) + c;
+  const uint32_t j = beg[q] + (k - lo[q]);
+  place[k] = j;
+  who[j] = k;
+}
+
+// Where each body lives: entry of its workgroup's LDS << 2 | 1, while there are entries (most);
+// else whether all its contacts are on one XCD << 1.
+__global__ void __launch_bounds__(kBlock) k_flow_homes(uint32_t n, const unsigned long long* __restrict__ mask,
+                                                       const uint32_t* __restrict__ start,
+                                                       const uint32_t* __restrict__ table,
+                                                       const uint32_t* __restrict__ own, uint32_t per_xcd,
+                                                       uint32_t most, uint32_t* __restrict__ homes,
+                                                       uint32_t* __restrict__ where) {
+  const uint32_t b = blockIdx.x * kBlock + threadIdx.x;
+  if (b >= n) return;
+  const uint32_t deg = (uint32_t)__popcll(mask[b]);
+  if (deg == 0) return;
+  const uint32_t* t = table + start[b];
+  const uint32_t w = own[t[0] & 0x7FFFFFFFu];
+  bool one = true, near = true;
+  for (uint32_t q = 1; q < deg; ++q) {
+    const uint32_t v = own[t[q] & 0x7FFFFFFFu];
+    one = one && v == w;
+    near = near && v / per_xcd == w / per_xcd;
+  }
+  uint32_t e = most;
+  if (one) e = atomicAdd(&homes[w], 1u);
+  where[b] = e < most ? e << 2 | 1u : near ? 2u : 0u;
 }
 
 __global__ void __launch_bounds__(kBlock) k_flow_links(uint32_t C, const uint32_t* __restrict__ ca,
@@ -780,8 +954,9 @@ __global__ void __launch_bounds__(kBlock) k_flow_links(uint32_t C, const uint32_
                                                        const StepCounters* __restrict__ ctr,
                                                        const unsigned long long* __restrict__ mask,
                                                        const uint32_t* __restrict__ start,
-                                                       const uint32_t* __restrict__ table, uint32_t xcds,
-                                                       uint32_t per_xcd, uint2* __restrict__ from,
+                                                       const uint32_t* __restrict__ table,
+                                                       const uint32_t* __restrict__ place,
+                                                       const uint32_t* __restrict__ where, uint2* __restrict__ from,
                                                        uint2* __restrict__ fin) {
   __shared__ uint32_t off[kMaxColours + 1];
   const uint32_t ncol = ctr->ncolours;
@@ -789,95 +964,103 @@ __global__ void __launch_bounds__(kBlock) k_flow_links(uint32_t C, const uint32_
   __syncthreads();
   const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
   if (k >= C) return;
+  const uint32_t N = flow_places(C);
   const unsigned long long below = (1ull << colour_of(off, ncol, k)) - 1ull;
-  // the XCD of the workgroup that updates contact i of colour c
-  auto xcd_of = [&](uint32_t c, uint32_t i) {
-    const uint64_t n = off[c + 1] - off[c], G = (uint64_t)xcds * per_xcd;
-    return (uint32_t)((((uint64_t)(i - off[c]) + 1) * G - 1) / n) / per_xcd;
-  };
-  // A slot may stay in its XCD's L2 when every contact of the body is updated there (they are
-  // its readers) and the slots that share its lines are written there too: a line that is dirty
-  // in one L2 must not hold another XCD's slots.
-  const uint32_t col = colour_of(off, ncol, k), x = xcd_of(col, k);
-  auto line = [&](uint32_t c, uint32_t i) {
-    const uint32_t i0 = i / kFlowLine * kFlowLine, i1 = min(i0 + kFlowLine, C) - 1;
-    return off[c] <= i0 && i1 < off[c + 1] && xcd_of(c, i0) == xcd_of(c, i1);
-  };
-  const uint32_t Cp = flow_side(C);
   uint32_t fr[2] = {kNoBody, kNoBody}, fi[2] = {kNoBody, kNoBody};
 #pragma unroll
   for (int side = 0; side < 2; ++side) {
     const uint32_t b = side ? cb[k] : ca[k];
     if (b == kNoBody) continue;
     const unsigned long long m = mask[b];
-    const uint32_t deg = (uint32_t)__popcll(m), rank = (uint32_t)__popcll(m & below);
-    const uint32_t* t = table + start[b];
-    bool here = true;  // every contact of the body is updated on XCD x
-    uint32_t cpred = 0, clast = 0;
-    unsigned long long left = m;
-    for (uint32_t q = 0; q < deg; ++q) {
-      const uint32_t c = (uint32_t)__ffsll((long long)left) - 1;
-      left &= left - 1;
-      here = here && xcd_of(c, t[q] < Cp ? t[q] : t[q] - Cp) == x;
-      if (q + 1 == (rank ? rank : deg)) cpred = c;
-      clast = c;
+    const uint32_t wrap = (m & below) ? 0u : kFlowWrap, h = where[b];
+    // colours of the contact before this one, cyclic, and of the last
+    const uint32_t last = 63u - (uint32_t)__clzll((long long)m);
+    const uint32_t pred = wrap ? last : 63u - (uint32_t)__clzll((long long)(m & below));
+    if (h & 1u) {
+      const uint32_t e = h >> 2 << (3 + kFlowColourBits) | kFlowHome;
+      fr[side] = e | pred << 3 | wrap;
+      fi[side] = e | last << 3;
+      continue;
     }
-    // slot of the body's contact `e` (colour c): after the far slots when it is near
-    auto slot = [&](uint32_t c, uint32_t e) { return e + (here && line(c, e < Cp ? e : e - Cp) ? 2u * Cp : 0u); };
-    fi[side] = slot(clast, t[deg - 1]);
-    fr[side] = slot(cpred, t[rank ? rank - 1 : deg - 1]) << 2 | (here && line(col, k) ? 2u : 0u) | (rank ? 0u : 1u);
+    const uint32_t* t = table + start[b];
+    const uint32_t deg = (uint32_t)__popcll(m), rank = (uint32_t)__popcll(m & below);
+    auto slot = [&](uint32_t e) {
+      return place[e & 0x7FFFFFFFu] + ((e >> 31) ? N : 0u) + ((h & 2u) ? 2u * N : 0u);
+    };
+    fr[side] = slot(t[rank ? rank - 1 : deg - 1]) << 3 | ((h & 2u) ? kFlowNear : 0u) | wrap;
+    fi[side] = slot(t[deg - 1]) << 3;
   }
-  from[k] = make_uint2(fr[0], fr[1]);
-  fin[k] = make_uint2(fi[0], fi[1]);
+  from[place[k]] = make_uint2(fr[0], fr[1]);
+  fin[place[k]] = make_uint2(fi[0], fi[1]);
 }
 
-// Packed records and impulses (see kRecGroups) from the colour-order arrays.
+// Packed records and impulses (see kRecGroups), and the scenes of an ensemble's contacts, at
+// the contacts' places.
 template <int D, typename Real>
 __global__ void __launch_bounds__(kBlock) k_flow_pack(ContactSoA<Real> c, uint32_t C, const Real* __restrict__ body,
-                                                      Real* __restrict__ rec_, Real* __restrict__ r_) {
+                                                      const uint32_t* __restrict__ place,
+                                                      const uint32_t* __restrict__ cscene, Real* __restrict__ rec_,
+                                                      Real* __restrict__ r_, uint32_t* __restrict__ scene) {
   using V = typename Vec4<Real>::type;
   using V2 = typename Vec2<Real>::type;
   const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
   if (k >= C) return;
+  const uint32_t j = place[k];
   Rec<D, Real> R;
   load_rec<D, Real>(c, k, R);
-  pack_rec<D, Real>(R, reinterpret_cast<const V*>(body), C, k, reinterpret_cast<V*>(rec_));
+  pack_rec<D, Real>(R, reinterpret_cast<const V*>(body), flow_places(C), j, reinterpret_cast<V*>(rec_));
   const Real* rp = c.r + 3 * (size_t)k;
-  if constexpr (D == 3) reinterpret_cast<V*>(r_)[k] = V{rp[0], rp[1], rp[2], (Real)0};
-  else reinterpret_cast<V2*>(r_)[k] = V2{rp[0], rp[1]};
+  if constexpr (D == 3) reinterpret_cast<V*>(r_)[j] = V{rp[0], rp[1], rp[2], (Real)0};
+  else reinterpret_cast<V2*>(r_)[j] = V2{rp[0], rp[1]};
+  if (cscene) scene[j] = cscene[k];
 }
 
-hipError_t launch_flow_links(scx_ctx* c, uint32_t C, const uint32_t* ca, const uint32_t* cb, const FlowLinks& L,
-                             uint32_t xcds, uint32_t per_xcd) {
+hipError_t launch_flow_links(scx_ctx* c, uint32_t C, const uint32_t* ca, const uint32_t* cb, const uint32_t* first,
+                             const FlowLinks& L, uint32_t xcds, uint32_t per_xcd, uint32_t home) {
   hipStream_t s = c->stream;
-  const uint32_t nc = (C + kBlock - 1) / kBlock, nb = (c->n + kBlock - 1) / kBlock;
+  const uint32_t nc = (C + kBlock - 1) / kBlock, nb = (c->n + kBlock - 1) / kBlock, G = xcds * per_xcd;
   hipError_t e = hipMemsetAsync(L.mask, 0, sizeof(unsigned long long) * ((size_t)c->n + 1), s);
   if (e != hipSuccess) return e;
-  k_flow_colours<<<nc, kBlock, 0, s>>>(C, ca, cb, c->d.coloff, c->d.ctr, L.mask);
+  k_flow_colours<<<nc, kBlock, 0, s>>>(C, ca, cb, c->d.coloff, c->d.ctr, first, G, L.mask, L.own);
+  k_flow_ranges<<<kMaxColours, kBlock, 0, s>>>(G, c->d.coloff, c->d.ctr, L.own, L.lo);
+  k_flow_places<<<G, kMaxColours, 0, s>>>(per_xcd, c->d.coloff, c->d.ctr, L.lo, L.beg, L.homes);
   k_flow_offsets<<<nb, kBlock, 0, s>>>(c->n, L.mask, L.start);
-  k_flow_table<<<nc, kBlock, 0, s>>>(C, ca, cb, c->d.coloff, c->d.ctr, L.mask, L.start, L.table);
-  k_flow_links<<<nc, kBlock, 0, s>>>(C, ca, cb, c->d.coloff, c->d.ctr, L.mask, L.start, L.table, xcds, per_xcd, L.from,
-                                      L.fin);
+  k_flow_table<<<nc, kBlock, 0, s>>>(C, ca, cb, c->d.coloff, c->d.ctr, L.mask, L.start, L.own, L.lo, L.beg, L.table,
+                                      L.place, L.who);
+  k_flow_homes<<<nb, kBlock, 0, s>>>(c->n, L.mask, L.start, L.table, L.own, per_xcd, home, L.homes, L.where);
+  k_flow_links<<<nc, kBlock, 0, s>>>(C, ca, cb, c->d.coloff, c->d.ctr, L.mask, L.start, L.table, L.place, L.where,
+                                      L.from, L.fin);
   return hipGetLastError();
+}
+
+template <int D, typename Real, bool Ens, bool All>
+static hipError_t launch_flow_as(scx_ctx* c, GSArgs<Real> A, FlowBufs<Real> F, uint32_t per_xcd, size_t lds,
+                                 bool* launched) {
+  const void* fn = (const void*)k_gs_flow<D, Real, Ens, All>;
+  const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (e != hipSuccess) return e;
+  void* args[] = {&A, &F};
+  return launch_cooperative(c, fn, (int)(kXcds * per_xcd), kFlowThreads, args, lds, c->stream, launched);
 }
 
 template <int D, typename Real, bool Ens>
 static hipError_t launch_flow_of(scx_ctx* c, GSArgs<Real> A, FlowBufs<Real> F, uint32_t per_xcd, bool* launched) {
   const uint32_t nc = (A.C + kBlock - 1) / kBlock;
-  k_flow_pack<D, Real><<<nc, kBlock, 0, c->stream>>>(A.c, A.C, A.body, F.rec, F.r);
+  k_flow_pack<D, Real><<<nc, kBlock, 0, c->stream>>>(A.c, A.C, A.body, F.place, A.cscene, F.rec, F.r, F.scene);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  // the LDS holds the records, links and impulses of as many of a workgroup's contacts as it can
+  // the LDS holds the bodies that live there, and the records, links and impulses of as many
+  // of a workgroup's contacts as it can
+  const size_t bodies = (sizeof(Real) * FlowPort<D, Real>::NR + sizeof(uint32_t)) * F.home;
   const size_t each = sizeof(Real) * (D == 3 ? 16 + 3 : 8 + 2) + sizeof(uint2);
-  const uint32_t most = A.C / (F.xcds * per_xcd) + 1 + kMaxColours;  // contacts of a workgroup
-  F.kept = std::min<uint32_t>((most + 1) / 2 * 2, (uint32_t)(kFlowLdsMax / each) / 2 * 2);
-  const size_t lds = each * F.kept;
-  const hipError_t ea = hipFuncSetAttribute((const void*)k_gs_flow<D, Real, Ens>,
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (ea != hipSuccess) return ea;
-  void* args[] = {&A, &F};
-  return launch_cooperative(c, (const void*)k_gs_flow<D, Real, Ens>, (int)(kXcds * per_xcd), kFlowThreads, args, lds,
-                            c->stream, launched);
+  // contacts of a workgroup: an equal share, and up to those of one body or one of each colour
+  const uint32_t most = A.C / (F.xcds * per_xcd) + 1 + kMaxColours;
+  F.rows = (most / 64 + kMaxColours + kFlowThreads / 64 + 1) / 2 * 2;
+  const size_t rows = sizeof(uint2) * F.rows;
+  F.kept = std::min<uint32_t>((most + 1) / 2 * 2, (uint32_t)((kFlowLdsMax - bodies - rows) / each) / 2 * 2);
+  const size_t lds = bodies + rows + each * F.kept;
+  return F.kept >= most ? launch_flow_as<D, Real, Ens, true>(c, A, F, per_xcd, lds, launched)
+                        : launch_flow_as<D, Real, Ens, false>(c, A, F, per_xcd, lds, launched);
 }
 
 template <int D, typename Real>

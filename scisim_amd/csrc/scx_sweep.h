@@ -379,30 +379,52 @@ constexpr int kFlowMaxBlocks = 256;  // one wave reads every workgroup's flag
 // Slots of side b follow those of side a, the near ones (read on one XCD alone) of both follow
 // the far ones, so that no line holds both kinds; kFlowLine consecutive ones fill at least two lines.
 constexpr uint32_t kFlowLine = 16;
-__host__ __device__ inline uint32_t flow_side(uint32_t C) { return (C + kFlowLine - 1) / kFlowLine * kFlowLine; }
+// Places of C contacts: a line's worth free behind each XCD's.
+__host__ __device__ inline uint32_t flow_places(uint32_t C) {
+  return (C + kFlowLine - 1) / kFlowLine * kFlowLine + kXcds * kFlowLine;
+}
+// Where a contact finds a body (FlowBufs::from, fin)
+constexpr uint32_t kFlowWrap = 1, kFlowNear = 2, kFlowHome = 4, kFlowColourBits = 6;
+static_assert(kMaxColours <= 1 << kFlowColourBits, "a colour's bits");
 template <typename Real>
 struct FlowBufs {
-  Real* rec;          // packed records
-  Real* r;            // impulses: 4 (3D) or 2 (2D) Reals per contact
-  const uint32_t* from;  // per contact, 2: the slots its bodies come from (slot << 2 | flags)
-  const uint32_t* fin;   // per contact, 2: the slots of its bodies' last contacts
+  Real* rec;          // packed records, by place
+  Real* r;            // impulses: 4 (3D) or 2 (2D) Reals per place
+  const uint32_t* from;  // per place, 2: where its bodies come from (as k_gs_flow's FlowContact)
+  const uint32_t* fin;   // per place, 2: where its bodies are after their last contacts
+  const uint32_t* beg;   // per workgroup, kMaxColours + 1: the first place of each colour
+  const uint32_t* place;  // of each contact
+  const uint32_t* who;   // the contact at each place
+  uint32_t* scene;    // per place (ensembles)
   void* slots;        // outbox slots, in 16-byte pieces
   uint32_t xcds;      // XCDs that take part
   uint32_t* flags;    // per workgroup: 2 * tag + whether it holds a contact above the threshold
   void* parts;        // per workgroup: its largest residual and the tag
   uint32_t tag0;      // first tag of this launch: above every tag in slots, flags and parts
   int skip_early;     // as WgBufs::skip_early
+  uint32_t home;      // bodies of a workgroup that its LDS holds
+  uint32_t rows;      // rows of a workgroup's contacts, at most
   uint32_t kept;      // contacts of a workgroup that its LDS holds
 };
 struct FlowLinks {
-  unsigned long long* mask;  // per body slot: its colours; entry n: the table's length
-  uint32_t* start;           // per body slot: start of its entries in the table
-  uint32_t* table;           // outbox slots of each body's contacts in colour order
+  unsigned long long* mask;  // per body: its colours; entry n: the table's length
+  uint32_t* start;           // per body: start of its entries in the table
+  uint32_t* where;           // per body: see k_flow_homes
+  uint32_t* table;           // each body's contacts in colour order
+  uint32_t* own;             // per contact: its workgroup
+  uint32_t* place;
+  uint32_t* who;
+  uint32_t* scene;
+  uint32_t* lo;              // per workgroup, kMaxColours + 1: see k_flow_ranges
+  uint32_t* beg;
+  uint32_t* homes;           // per workgroup: bodies that may live in its LDS
   uint2* from;
   uint2* fin;
 };
-hipError_t launch_flow_links(scx_ctx* c, uint32_t C, const uint32_t* ca, const uint32_t* cb, const FlowLinks& L,
-                             uint32_t xcds, uint32_t per_xcd);
+// first: contacts before those of each first body in the order of the bodies, or null; home:
+// bodies of a workgroup that its LDS holds.
+hipError_t launch_flow_links(scx_ctx* c, uint32_t C, const uint32_t* ca, const uint32_t* cb, const uint32_t* first,
+                             const FlowLinks& L, uint32_t xcds, uint32_t per_xcd, uint32_t home);
 // Packs the records and launches the sweeps on per_xcd workgroups of each of F.xcds XCDs; *launched is false when a
 // cooperative launch is not to be had (nothing ran).
 template <int D, typename Real>
