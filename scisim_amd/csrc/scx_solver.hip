@@ -1601,7 +1601,7 @@ static hipError_t flow_prepare(scx_ctx* c, const GSArgs<Real>& A, uint32_t xcds,
   F.slots = d.flow_slots + sync;
   F.xcds = xcds;
   // A body needs about 1.5 contacts of its workgroup; the rest of the LDS serves their records.
-  F.home = std::min<uint32_t>((A.C / (xcds * per_xcd) * 3 / 4 + 64) / 16 * 16, D == 3 ? 1280 : 2560);
+  F.home = std::min<uint32_t>((A.C / (xcds * per_xcd) * 3 / 4 + 128) / 16 * 16, D == 3 ? 1344 : 2624);
   if (*linked == (xcds << 16 | per_xcd)) return hipSuccess;  // the other phase's links serve
   *linked = xcds << 16 | per_xcd;
   // (the contacts before those of each slot: launch_colour_sort)

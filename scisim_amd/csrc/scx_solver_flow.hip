@@ -59,19 +59,27 @@ struct FlowPort {
     u32x4f p[NP];
   };
 
-  __device__ __forceinline__ void ld(uint32_t slot, Raw& x) const {
-    const uint32_t o = slot * (uint32_t)(16 * NP);
+  // byte offset of a slot; kNowhere: loads read 0, stores go nowhere (beyond the buffer's end)
+  static constexpr uint32_t kNowhere = 1u << 31;
+  __device__ __forceinline__ static uint32_t at(uint32_t slot) { return slot * (uint32_t)(16 * NP); }
+  __device__ __forceinline__ void ld(uint32_t o, Raw& x) const {
 #pragma unroll
     for (int i = 0; i < NP; ++i) x.p[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, o + 16u * i, 0, kFlowAux);
   }
   __device__ __forceinline__ uint32_t tag(uint32_t slot) const {  // of its last piece
-    return __builtin_amdgcn_raw_buffer_load_b32(rs, slot * (uint32_t)(16 * NP) + 16u * (NP - 1) + 12u, 0, kFlowAux);
+    return __builtin_amdgcn_raw_buffer_load_b32(rs, at(slot) + 16u * (NP - 1) + 12u, 0, kFlowAux);
   }
   __device__ __forceinline__ static bool is(const Raw& x, uint32_t tag) {
     bool ok = true;
 #pragma unroll
     for (int i = 0; i < NP; ++i) ok = ok && x.p[i][3] == tag;
     return ok;
+  }
+  __device__ __forceinline__ static bool beyond(const Raw& x, uint32_t tag) {
+    bool b = false;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) b = b || (int32_t)(x.p[i][3] - tag) > 0;
+    return b;
   }
   __device__ __forceinline__ static void unpack(const Raw& x, Real* r) {
     uint32_t u[3 * NP];
@@ -85,8 +93,7 @@ struct FlowPort {
         r[i] = __uint_as_float(u[i]);
     }
   }
-  // near: every reader is on this XCD, so the store may stay in its L2
-  __device__ __forceinline__ void st(uint32_t slot, const V& v, const V& w, uint32_t tag, bool near) const {
+  __device__ __forceinline__ static void pack(const V& v, const V& w, uint32_t tag, Raw& x) {
     Real r[NR];
     if constexpr (D == 3) {
       r[0] = v.x, r[1] = v.y, r[2] = v.z, r[3] = w.x, r[4] = w.y, r[5] = w.z;
@@ -106,13 +113,14 @@ struct FlowPort {
         u[i] = __float_as_uint(r[i]);
       }
     }
-    const uint32_t o = slot * (uint32_t)(16 * NP);
 #pragma unroll
-    for (int i = 0; i < NP; ++i) {
-      const u32x4f x = {u[3 * i], u[3 * i + 1], u[3 * i + 2], tag};
-      if (near) __builtin_amdgcn_raw_buffer_store_b128(x, rs, o + 16u * i, 0, 0);
-      else __builtin_amdgcn_raw_buffer_store_b128(x, rs, o + 16u * i, 0, kFlowAux);
-    }
+    for (int i = 0; i < NP; ++i) x.p[i] = u32x4f{u[3 * i], u[3 * i + 1], u[3 * i + 2], tag};
+  }
+  // Aux 0: every reader is on this XCD, so the store may stay in its L2
+  template <int Aux>
+  __device__ __forceinline__ void st(uint32_t o, const Raw& x) const {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) __builtin_amdgcn_raw_buffer_store_b128(x.p[i], rs, o + 16u * i, 0, Aux);
   }
 };
 
@@ -249,30 +257,28 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
     return j + (side ? N : 0u) + ((from & kFlowNear) ? 2u * N : 0u);
   };
   // Bodies in LDS. A wave's LDS accesses are carried out in their order: a writer stores the
-  // velocities before the tag, a reader loads the tag before the velocities.
+  // velocities before the tag, a reader loads the tag before the velocities. The last 64
+  // entries are nobody's: a lane with a body in a slot reads and writes its own of them, so that
+  // a wave goes through with few branches (a contact's successors wait for each instruction
+  // between).
+  const uint32_t nobody = F.home - 64 + lane;
+  auto home_of = [&](uint32_t word, bool home) { return home ? word >> (3 + kFlowColourBits) : nobody; };
   auto home_tag = [&](uint32_t word, uint32_t t) { return t << kFlowColourBits | ((word >> 3) & (kMaxColours - 1)); };
-  auto home_ld = [&](uint32_t word, Real* x) __attribute__((always_inline)) {
-    const uint32_t e = word >> (3 + kFlowColourBits);
-    const uint32_t t = l_tag[e];
-    asm volatile("" ::: "memory");
+  auto home_ld = [&](uint32_t e, Real* x) __attribute__((always_inline)) {
     const V2* p = reinterpret_cast<const V2*>(l_body + (size_t)Port::NR * e);
 #pragma unroll
     for (int i = 0; i < Port::NR / 2; ++i) {
       const V2 y = p[i];
       x[2 * i] = y.x, x[2 * i + 1] = y.y;
     }
-    return t;
   };
-  auto home_st = [&](uint32_t word, const V& v, const V& w, uint32_t col) __attribute__((always_inline)) {
-    const uint32_t e = word >> (3 + kFlowColourBits);
+  auto home_st = [&](uint32_t e, const V& v, const V& w) __attribute__((always_inline)) {
     V2* p = reinterpret_cast<V2*>(l_body + (size_t)Port::NR * e);
     p[0] = V2{v.x, v.y};
     if constexpr (D == 3) {
       p[1] = V2{v.z, w.x};
       p[2] = V2{w.y, w.z};
     }
-    asm volatile("" ::: "memory");
-    l_tag[e] = tag << kFlowColourBits | col;
   };
   auto as_body = [&](const Real* x, Real im, Real ii, V& v, V& w) __attribute__((always_inline)) {
     if constexpr (D == 3) {
@@ -283,35 +289,69 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
       w = V{0, 0, 0, 0};
     }
   };
-  // Looks at two bodies under the tags ta and tb; pa, pb: whether they are still to come. Only
-  // what is still to come is read (and the slots whole: a poll that finds the tag has the body).
-  auto look = [&](uint32_t wa, uint32_t ta, bool& pa, uint32_t wb, uint32_t tb, bool& pb, Real* xa, Real* xb) __attribute__((always_inline)) {
-    const bool ha = pa && (wa & kFlowHome), hb = pb && (wb & kFlowHome), sa = pa && !ha, sb = pb && !hb;
-    asm volatile("" ::: "memory");  // each look reads memory again
-    if (__any(sa || sb)) {  // (a wave with all its bodies in LDS does not wait for its stores to slots)
+  auto is_home = [&](uint32_t word, bool has) { return has && (word & kFlowHome); };
+  // Waits for two bodies under the tags ta and tb (b only with hasb). check: gives up (false)
+  // when a body in a slot has already moved on to a later sweep (one in LDS moves on with this
+  // workgroup only).
+  auto gather = [&](uint32_t wa, uint32_t ta, bool hasb, uint32_t wb, uint32_t tb, bool check, Real* xa, Real* xb) __attribute__((always_inline)) {
+    const bool ha = is_home(wa, true), hb = is_home(wb, hasb), sa = !ha, sb = hasb && !hb;
+    const uint32_t ia = home_of(wa, ha), ib = home_of(wb, hb), ea = home_tag(wa, ta), eb = home_tag(wb, tb);
+    const uint32_t oa = sa ? Port::at(wa >> 3) : Port::kNowhere, ob = sb ? Port::at(wb >> 3) : Port::kNowhere;
+    const bool slots = __any(sa || sb);  // (a wave without does not wait for its stores to slots)
+    bool ok = false, late = false;
+    for (uint32_t n = 0; !ok && !late && !dead;) {
+      asm volatile("" ::: "memory");  // each look reads memory again
       Raw ra, rb;
-      if (sa) P.ld(wa >> 3, ra);
-      if (sb) P.ld(wb >> 3, rb);
-      if (ha) pa = home_ld(wa, xa) != home_tag(wa, ta);
-      if (hb) pb = home_ld(wb, xb) != home_tag(wb, tb);
-      if (sa) {
-        pa = !Port::is(ra, ta);
-        Port::unpack(ra, xa);
+      if (slots) {
+        P.ld(oa, ra);
+        P.ld(ob, rb);
       }
-      if (sb) {
-        pb = !Port::is(rb, tb);
-        Port::unpack(rb, xb);
+      const uint32_t la = l_tag[ia], lb = l_tag[ib];
+      asm volatile("" ::: "memory");
+      home_ld(ia, xa);
+      home_ld(ib, xb);
+      bool oka = la == ea, okb = lb == eb;
+      if (slots) {
+        Real ya[Port::NR], yb[Port::NR];
+        Port::unpack(ra, ya);
+        Port::unpack(rb, yb);
+#pragma unroll
+        for (int i = 0; i < Port::NR; ++i) {
+          xa[i] = sa ? ya[i] : xa[i];
+          xb[i] = sb ? yb[i] : xb[i];
+        }
+        oka = sa ? Port::is(ra, ta) : oka;
+        okb = sb ? Port::is(rb, tb) : okb;
+        if (check) late = (sa && Port::beyond(ra, ta)) || (sb && Port::beyond(rb, tb));
       }
-      return;
-    }
-    if (ha) pa = home_ld(wa, xa) != home_tag(wa, ta);
-    if (hb) pb = home_ld(wb, xb) != home_tag(wb, tb);
-  };
-  auto wait_two = [&](uint32_t wa, uint32_t ta, bool hasb, uint32_t wb, uint32_t tb, Real* xa, Real* xb) __attribute__((always_inline)) {
-    bool pa = true, pb = hasb;
-    for (uint32_t n = 0; (pa || pb) && !dead;) {
-      look(wa, ta, pa, wb, tb, pb, xa, xb);
+      ok = oka && (okb || !hasb);
       if (++n >= kSpinLimit) dead = true;
+    }
+    return ok;
+  };
+  // Stores the bodies of the contact at place j, of colour col, under the sweep's tag.
+  auto scatter = [&](uint32_t j, uint32_t col, uint32_t wa, bool hasa, uint32_t wb, bool hasb, const V* b) __attribute__((always_inline)) {
+    const bool ha = is_home(wa, hasa), hb = is_home(wb, hasb), sa = hasa && !ha, sb = hasb && !hb;
+    const uint32_t ia = home_of(wa, ha), ib = home_of(wb, hb);
+    home_st(ia, b[0], b[1]);
+    home_st(ib, b[2], b[3]);
+    asm volatile("" ::: "memory");
+    l_tag[ia] = tag << kFlowColourBits | col;
+    l_tag[ib] = tag << kFlowColourBits | col;
+    if (__any(sa || sb)) {
+      Raw ra, rb;
+      Port::pack(b[0], b[1], tag, ra);
+      Port::pack(b[2], b[3], tag, rb);
+      const bool na = one_l2 && (wa & kFlowNear), nb = one_l2 && (wb & kFlowNear);
+      const uint32_t oa = Port::at(own_slot(j, 0, wa)), ob = Port::at(own_slot(j, 1, wb));
+      if (__any((sa && na) || (sb && nb))) {
+        P.template st<0>(sa && na ? oa : Port::kNowhere, ra);
+        P.template st<0>(sb && nb ? ob : Port::kNowhere, rb);
+      }
+      if (__any((sa && !na) || (sb && !nb))) {
+        P.template st<kFlowAux>(sa && !na ? oa : Port::kNowhere, ra);
+        P.template st<kFlowAux>(sb && !nb ? ob : Port::kNowhere, rb);
+      }
     }
   };
   auto update = [&](uint32_t j, uint32_t col, const FlowContact<D, Real>& L, bool init, Real* rbest) __attribute__((always_inline)) {
@@ -321,9 +361,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
     unpack_rec<D, Real>(L.g, hasb, ld.R, im);
     ld.r[0] = L.r[0], ld.r[1] = L.r[1], ld.r[2] = L.r[2];
     Real xa[Port::NR], xb[Port::NR];
-#pragma unroll
-    for (int i = 0; i < Port::NR; ++i) xb[i] = 0;
-    wait_two(L.from_a, tag - (L.from_a & kFlowWrap), hasb, L.from_b, tag - (L.from_b & kFlowWrap), xa, xb);
+    (void)gather(L.from_a, tag - (L.from_a & kFlowWrap), hasb, L.from_b, tag - (L.from_b & kFlowWrap), false, xa, xb);
     V b[4];
     as_body(xa, im[0], im[2], b[0], b[1]);
     as_body(xb, im[1], im[3], b[2], b[3]);
@@ -331,12 +369,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
     update_core<D, Real>(
         ld, init, rbest, 0, 2, [&](size_t i) { return b[i]; }, [&](size_t i, const V& x) { b[i] = x; },
         [&](int d, Real x) { rn[d] = x; });
-    if (L.from_a & kFlowHome) home_st(L.from_a, b[0], b[1], col);
-    else P.st(own_slot(j, 0, L.from_a), b[0], b[1], tag, one_l2 && (L.from_a & kFlowNear));
-    if (hasb) {
-      if (L.from_b & kFlowHome) home_st(L.from_b, b[2], b[3], col);
-      else P.st(own_slot(j, 1, L.from_b), b[2], b[3], tag, one_l2 && (L.from_b & kFlowNear));
-    }
+    scatter(j, col, L.from_a, true, L.from_b, hasb, b);
     if (!init) store_r(j, rn);
   };
   // squared residual of contact j on the bodies' final velocities of this sweep; false when a
@@ -344,20 +377,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
   auto residual = [&](const FlowContact<D, Real>& L, uint2 fin, bool check, double& e) __attribute__((always_inline)) {
     const bool hasb = fin.y != kNoBody;
     Real xa[Port::NR], xb[Port::NR];
-#pragma unroll
-    for (int i = 0; i < Port::NR; ++i) xb[i] = 0;
-    bool ok = false, late = false, pa = true, pb = hasb;
-    for (uint32_t n = 0; !ok && !late && !dead; ++n) {
-      look(fin.x, tag, pa, fin.y, tag, pb, xa, xb);
-      ok = !pa && !pb;
-      if (check && !ok) {
-        // (a body in LDS moves on with this workgroup only)
-        if (!(fin.x & kFlowHome)) late = pa && (int32_t)(P.tag(fin.x >> 3) - tag) > 0;
-        if (hasb && !(fin.y & kFlowHome)) late = late || (pb && (int32_t)(P.tag(fin.y >> 3) - tag) > 0);
-      }
-      if (n >= kSpinLimit) dead = true;
-    }
-    if (!ok) return false;
+    if (!gather(fin.x, tag, hasb, fin.y, tag, check, xa, xb)) return false;
     Rec<D, Real> R;
     Real im[4];
     unpack_rec<D, Real>(L.g, hasb, R, im);
@@ -416,8 +436,8 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
           v = rec[0];
           if (D == 3) w = rec[1];
         }
-        if (word & kFlowHome) home_st(word, v, w, c);
-        else P.st(own_slot(j, side, word), v, w, tag, one_l2 && (word & kFlowNear));
+        const V b[4] = {v, w, v, w};
+        scatter(j, c, word, side == 0, word, side == 1, b);
       }
     });
   };
@@ -766,10 +786,10 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
       const uint32_t sl = side ? A.c.b[k] : A.c.a[k];
       Real x[Port::NR];
       if (word & kFlowHome) {
-        (void)home_ld(word, x);
+        home_ld(home_of(word, true), x);
       } else {
         Raw raw;
-        P.ld(own_slot(j, side, word), raw);
+        P.ld(Port::at(own_slot(j, side, word)), raw);
         Port::unpack(raw, x);
       }
       V v, w;
@@ -1027,7 +1047,7 @@ hipError_t launch_flow_links(scx_ctx* c, uint32_t C, const uint32_t* ca, const u
   k_flow_offsets<<<nb, kBlock, 0, s>>>(c->n, L.mask, L.start);
   k_flow_table<<<nc, kBlock, 0, s>>>(C, ca, cb, c->d.coloff, c->d.ctr, L.mask, L.start, L.own, L.lo, L.beg, L.table,
                                       L.place, L.who);
-  k_flow_homes<<<nb, kBlock, 0, s>>>(c->n, L.mask, L.start, L.table, L.own, per_xcd, home, L.homes, L.where);
+  k_flow_homes<<<nb, kBlock, 0, s>>>(c->n, L.mask, L.start, L.table, L.own, per_xcd, home - 64, L.homes, L.where);
   k_flow_links<<<nc, kBlock, 0, s>>>(C, ca, cb, c->d.coloff, c->d.ctr, L.mask, L.start, L.table, L.place, L.where,
                                       L.from, L.fin);
   return hipGetLastError();

@@ -402,7 +402,7 @@ struct FlowBufs {
   void* parts;        // per workgroup: its largest residual and the tag
   uint32_t tag0;      // first tag of this launch: above every tag in slots, flags and parts
   int skip_early;     // as WgBufs::skip_early
-  uint32_t home;      // bodies of a workgroup that its LDS holds
+  uint32_t home;      // bodies of a workgroup that its LDS holds, and 64 more
   uint32_t rows;      // rows of a workgroup's contacts, at most
   uint32_t kept;      // contacts of a workgroup that its LDS holds
 };
@@ -421,8 +421,8 @@ struct FlowLinks {
   uint2* from;
   uint2* fin;
 };
-// first: contacts before those of each first body in the order of the bodies, or null; home:
-// bodies of a workgroup that its LDS holds.
+// first: contacts before those of each first body in the order of the bodies, or null; home: as
+// FlowBufs::home.
 hipError_t launch_flow_links(scx_ctx* c, uint32_t C, const uint32_t* ca, const uint32_t* cb, const uint32_t* first,
                              const FlowLinks& L, uint32_t xcds, uint32_t per_xcd, uint32_t home);
 // Packs the records and launches the sweeps on per_xcd workgroups of each of F.xcds XCDs; *launched is false when a
