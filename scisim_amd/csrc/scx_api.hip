@@ -260,7 +260,6 @@ void free_all(scx_ctx* c) {
   dfree(&d.comp_parent);
   dfree(&d.comp_cnt);
   dfree(&d.comp_list);
-  dfree(&d.wg_arena);
   dfree(&d.flow_links);
   dfree(&d.flow_rec);
   dfree(&d.flow_slots);
@@ -619,13 +618,11 @@ int scx_create(const scx_config* cfg, scx_ctx** out) {
       c->comp_share = std::min(100.0, std::max(1.0, atof(env)));
       c->comp_adapt = false;
     }
-    // SCX_WG_SWEEPS=0: contact sets whose bodies one workgroup's LDS holds are swept on several
-    // workgroups all the same; SCX_FLOW_SWEEPS=0: larger ones with grid barriers between the
-    // colours (the same iterates bit for bit; for A/B measurements and tests). The switches of
-    // the sweeps with barriers above keep a context on them unless these two say otherwise.
+    // SCX_FLOW_SWEEPS=0: sweeps with grid barriers between the colours (the same iterates bit
+    // for bit; for A/B measurements and tests). The switches of those sweeps above keep a
+    // context on them unless it says otherwise.
     if (getenv("SCX_COMPONENT_SWEEPS") || getenv("SCX_COMPONENT_PERCENT") || getenv("SCX_COHERENT_SWEEPS"))
-      c->wg_sweeps = c->flow_sweeps = false;
-    if (const char* env = getenv("SCX_WG_SWEEPS")) c->wg_sweeps = atoi(env) != 0;
+      c->flow_sweeps = false;
     if (const char* env = getenv("SCX_FLOW_SWEEPS")) c->flow_sweeps = atoi(env) != 0;
     if ((e = dalloc(&d.partial, (size_t)std::max(c->gs_blocks, 1) + 1)) != hipSuccess ||
         (e = dalloc(&d.viol, (size_t)3 + kViolCap)) != hipSuccess ||

@@ -203,8 +203,6 @@ struct DeviceBuffers {
   uint32_t* comp_parent = nullptr;  // N: union-find parents of the component phase (k_gs)
   uint32_t* comp_cnt = nullptr;     // 1 + gs_blocks: overflow flag, per-workgroup counts
   uint32_t* comp_list = nullptr;    // gs_blocks x kCompCap: per-workgroup contacts
-  unsigned char* wg_arena = nullptr;  // working memory of the one-workgroup sweeps (cap_wg bytes)
-  size_t cap_wg = 0;
   // sweeps without barriers: links, packed records and impulses, sync words and outbox slots
   unsigned char* flow_links = nullptr;
   unsigned char* flow_rec = nullptr;
@@ -287,9 +285,8 @@ struct scx_ctx {
   double comp_ceiling = 100.0;  // below the last share that overflowed (drifts back up)
   bool comp_adapt = true;
   bool barrier_sweeps = false;  // the last solve swept with grid barriers (k_gs)
-  bool flow_sweeps = true;      // one scene: sweep without barriers between the colours (k_gs_flow)
+  bool flow_sweeps = true;      // sweep without barriers between the colours (k_gs_flow)
   uint32_t flow_tag = 1;        // next unused tag of those sweeps' slots
-  bool wg_sweeps = true;        // one scene: sweep in one workgroup when its LDS holds the bodies
   // The device's cooperative queues are limited in number (HSA_QUEUE_TYPE_COOPERATIVE,
   // hsa/hsa.h: "Queues of this type may be limited in number"); while another process holds
   // them a cooperative launch fails with hipErrorIllegalState. The persistent kernels need

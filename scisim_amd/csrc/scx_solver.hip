@@ -1482,38 +1482,6 @@ static hipError_t tune_after_solve(scx_ctx* c) {
   return e;
 }
 
-// One-workgroup sweeps with the bodies in LDS (k_gs_wg). Their time per sweep grows with the
-// contacts (one CU), that of the sweeps without barriers (k_gs_flow) with the colours: FP64
-// sweeps of 2,600 sphere contacts with their residuals take 24 us in one workgroup and 31 us
-// on 32 to 256 workgroups, of 3,347 sphere contacts 18.7 and 17.7 to 19.4 us, of 6,857 circle
-// contacts 26 and 18 us. The LDS limit leaves room for the kernel's static arrays.
-constexpr size_t kWgLdsMax = 152 * 1024;
-constexpr uint32_t kWgMaxContacts = 3072;
-
-// Their buffers, in the context's arena (grown when a larger contact set takes the path).
-template <int D, typename Real>
-static hipError_t wg_buffers(scx_ctx* c, uint32_t C, uint32_t nbodies, WgBufs<Real>& W) {
-  const size_t rec = sizeof(Real) * (D == 3 ? 16 : 8) * (size_t)C, r = sizeof(Real) * (D == 3 ? 4 : 2) * (size_t)C;
-  const size_t ids = sizeof(uint32_t) * (size_t)((C + 3) / 4 * 4), slot = sizeof(uint32_t) * (size_t)nbodies;
-  const size_t need = rec + r + ids + slot;
-  DeviceBuffers& d = c->d;
-  if (need > d.cap_wg) {
-    // the buffer may still be in use by an earlier launch on the stream; hipFree waits for it
-    if (d.wg_arena) (void)hipFree(d.wg_arena);
-    d.wg_arena = nullptr;
-    d.cap_wg = 0;
-    const hipError_t e = hipMalloc((void**)&d.wg_arena, need + need / 4);
-    if (e != hipSuccess) return e;
-    d.cap_wg = need + need / 4;
-  }
-  unsigned char* p = d.wg_arena;
-  W.rec = reinterpret_cast<Real*>(p);
-  W.r = reinterpret_cast<Real*>(p + rec);
-  W.ids = reinterpret_cast<uint32_t*>(p + rec + r);
-  W.slot = reinterpret_cast<uint32_t*>(p + rec + r + ids);
-  return hipSuccess;
-}
-
 // Sweeps without barriers between the colours (k_gs_flow): their buffers, in the context's
 // arenas (grown when a larger contact set takes the path), and the links of this contact set
 // (shared by the two phases of a solve).
@@ -1522,13 +1490,18 @@ constexpr uint32_t kFlowTagMax = 1u << 30;
 // without): spheres 16,987 contacts 15.3 and 6.2, 34,176 20.5 and 9.4, 99,626 17.1 and 8.5,
 // 423,718 30.1 and 14.9, 848,458 18.9 and 8.7, 1,283,826 18.6 and 11.8. kFlowMaxContacts bounds
 // the buffers (0.5 GB per million contacts). Workgroups: 128 contacts each, up to the CUs in use.
-constexpr uint32_t kFlowMinContacts = 1024, kFlowMaxContacts = 1u << 21;
+constexpr uint32_t kFlowMaxContacts = 1u << 21;
 constexpr uint32_t kFlowContacts = 128;  // contacts of a workgroup
 // Up to kFlowOneXcd contacts one XCD's CUs do better than all: every slot is then a near one
 // (k_gs_flow), and more bodies live in LDS. One XCD against eight, whole solves of 300 to 2,000
 // sweeps in ms: circles 13,169 contacts 20.2 and 24.8, 24,976 8.6 and 10.1; spheres 16,987 6.2
 // and 7.4, 34,176 9.4 and 11.0, 67,457 8.7 and 8.6, 99,626 11.4 and 8.5.
 constexpr uint32_t kFlowOneXcd = 1u << 16;
+// Up to kFlowOneGroup contacts one workgroup does better than several: all its bodies live in its
+// LDS. One workgroup, two and eight, FP64 solves in ms: spheres 522 contacts 3.5, 4.9 and 5.1,
+// 1,377 6.1, 6.8 and 7.6, 2,454 10.7, 7.2 and 7.2; a stand-alone solve of 2,600 sphere contacts,
+// whose bodies come in no order, 11.6, 13.8 and 14.2 (32 workgroups: 12.3).
+constexpr uint32_t kFlowOneGroup = 1536, kFlowOneGroupUnsorted = 3072;
 
 static hipError_t flow_arena(unsigned char** p, size_t* cap, size_t need, hipStream_t s) {
   if (need <= *cap) return hipSuccess;
@@ -1652,23 +1625,24 @@ static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint
   const size_t lds = LdsLayout<D, Real>::bytes(A.C);
   const bool lds_path = std::min(max_blocks, model) <= 1 && c->force_blocks <= 0 && lds <= kGSLdsMax && A.lmap &&
                         !A.cscene;
-  // bodies in one workgroup's LDS: up to kWgMaxContacts contacts
-  const size_t wg_lds = wg_lds_bytes<D, Real>(A.nbodies, A.C);
   const bool free_width = c->force_blocks <= 0 && !lds_path;
-  const bool wg = free_width && !A.cscene && c->wg_sweeps && A.lmap && A.C <= kWgMaxContacts && wg_lds <= kWgLdsMax;
-  // no barriers between the colours: from there to kFlowMaxContacts, while the slots can be
-  // addressed and the tags last; ensembles of up to kFlowMaxScenes scenes
-  const bool flow = free_width && !wg && c->flow_sweeps && !c->coop_unavailable && max_blocks >= (int)kXcds &&
-                    A.C >= kFlowMinContacts && A.C <= kFlowMaxContacts && A.nscenes <= kFlowMaxScenes &&
-                    A.max_iters < kFlowTagMax / 4 && (uint64_t)flow_places(A.C) * (D == 3 ? 32 : 16) * sizeof(Real) < (1ull << 31);
+  // no barriers between the colours: up to kFlowMaxContacts, while the slots can be addressed
+  // and the tags last; ensembles of up to kFlowMaxScenes scenes. One workgroup for small sets,
+  // larger ones where nothing is known of the bodies' neighbours (a range of contacts then
+  // shares its bodies with all others).
+  const bool one = A.C <= (c->d.slot_map ? kFlowOneGroup : kFlowOneGroupUnsorted);
+  const bool flow = free_width && c->flow_sweeps && (one || !c->coop_unavailable) && max_blocks >= (int)kXcds &&
+                    A.C <= kFlowMaxContacts && A.nscenes <= kFlowMaxScenes && A.max_iters < kFlowTagMax / 4 &&
+                    (uint64_t)flow_places(A.C) * (D == 3 ? 32 : 16) * sizeof(Real) < (1ull << 31);
   // the autotuner picks among widths around the model's (not for the solves of one workgroup)
   const int phase = std::is_same<Real, double>::value ? 1 : 0;
-  const bool tune = c->tuner.enabled && c->force_blocks <= 0 && !lds_path && !wg && !c->coop_unavailable;
+  const bool tune = c->tuner.enabled && c->force_blocks <= 0 && !lds_path && !(flow && one) && !c->coop_unavailable;
   // one XCD's CUs up to flow_one_xcd contacts, all beyond
   uint32_t xcds = A.C <= kFlowOneXcd ? 1 : kXcds;
   if (const char* env = getenv("SCX_FLOW_XCDS")) xcds = (uint32_t)std::max(1, std::min(atoi(env), (int)kXcds));
   const int flow_most = std::min(max_blocks, kFlowMaxBlocks) / (int)kXcds * (int)xcds;
-  const int width = flow ? std::max(2, std::min((int)((A.C + kFlowContacts - 1) / kFlowContacts), flow_most)) : model;
+  const int width =
+      !flow ? model : one ? 1 : std::max(2, std::min((int)((A.C + kFlowContacts - 1) / kFlowContacts), flow_most));
   const int want = tune ? tune_pick(c, phase, tune_key(D, phase, A.cscene != nullptr, A.C, nw), width,
                                     flow ? flow_most : max_blocks)
                         : width;
@@ -1681,13 +1655,6 @@ static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint
   if (blocks > 1 && comp < ncol && comp_contacts <= (uint64_t)blocks * kCompCap / 2) A.comp_col = (uint32_t)comp;
   else A.comp_parent = nullptr;
   const int skip_early = blocks > 1 && (tail < ncol || A.comp_parent) ? 1 : 0;
-  if (wg) {
-    WgBufs<Real> W;
-    hipError_t e = wg_buffers<D, Real>(c, A.C, (uint32_t)std::min<uint64_t>(A.nbodies, 2ull * A.C), W);
-    if (e != hipSuccess) return e;
-    W.skip_early = skip_early;
-    return launch_gs_wg<D, Real>(A, W, c->stream);
-  }
   if (lds_path) {
     // the whole solve in one workgroup's LDS
     hipError_t e = hipFuncSetAttribute((const void*)k_gs_lds<D, Real>, hipFuncAttributeMaxDynamicSharedMemorySize,

@@ -610,7 +610,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
   }
   const uint32_t base = (A.phase == 2) ? A.ctr->sweeps_fp32 : 0u;
   const bool subset = A.viol != nullptr;
-  const bool early = A.phase == 1 && F.skip_early;  // as WgBufs::skip_early
+  const bool early = A.phase == 1 && F.skip_early;
   constexpr uint32_t kFullEvery = 256, kSkipUntil = 1024 - kFullEvery;  // as in k_gs
   double err = evaluate(subset ? stop : -1.0, base);
   uint32_t nskip = 0, nchecks = 0, last_full = 0;
@@ -1060,6 +1060,10 @@ static hipError_t launch_flow_as(scx_ctx* c, GSArgs<Real> A, FlowBufs<Real> F, u
   const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
   void* args[] = {&A, &F};
+  if (F.xcds * per_xcd == 1) {  // one workgroup waits for no other
+    *launched = true;
+    return hipLaunchKernel(fn, dim3(kXcds), dim3(kFlowThreads), args, lds, c->stream);
+  }
   return launch_cooperative(c, fn, (int)(kXcds * per_xcd), kFlowThreads, args, lds, c->stream, launched);
 }
 

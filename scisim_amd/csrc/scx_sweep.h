@@ -351,28 +351,6 @@ __device__ __forceinline__ void pack_rec(const Rec<D, Real>& R, const typename V
   }
 }
 
-// Working memory of the one-workgroup sweeps (k_gs_wg), in colour order.
-template <int D, typename Real>
-constexpr uint32_t kWgThreadsOf = (D == 3 && sizeof(Real) == 8) ? 512u : 1024u;
-template <typename Real>
-struct WgBufs {
-  Real* rec;       // packed records: 16 (3D) or 8 (2D) Reals per contact, in groups of 4
-  Real* r;         // impulses: 4 (3D) or 2 (2D) Reals per contact
-  uint32_t* ids;   // per contact: its two LDS bodies
-  uint32_t* slot;  // per LDS body: its slot
-  // The FP32 phase's first sweeps skip evaluations by the stopping value, as k_gs does on
-  // several workgroups with a tail or a component phase. Elsewhere k_gs evaluates every sweep,
-  // so that its stagnation test knows the best residual of those sweeps too, and the
-  // threshold here is the best residual from the start.
-  int skip_early;
-};
-
-// LDS bytes of the one-workgroup solve of C contacts of nbodies bodies.
-template <int D, typename Real>
-size_t wg_lds_bytes(uint32_t nbodies, uint32_t C);
-template <int D, typename Real>
-hipError_t launch_gs_wg(const GSArgs<Real>& A, const WgBufs<Real>& W, hipStream_t s);
-
 // Working memory of the sweeps without barriers (k_gs_flow), in colour order.
 constexpr uint32_t kFlowMaxScenes = 2048;  // an ensemble's residuals, in every workgroup's LDS
 constexpr int kFlowMaxBlocks = 256;  // one wave reads every workgroup's flag
@@ -401,7 +379,11 @@ struct FlowBufs {
   uint32_t* flags;    // per workgroup: 2 * tag + whether it holds a contact above the threshold
   void* parts;        // per workgroup: its largest residual and the tag
   uint32_t tag0;      // first tag of this launch: above every tag in slots, flags and parts
-  int skip_early;     // as WgBufs::skip_early
+  // The FP32 phase's first sweeps skip evaluations by the stopping value, as k_gs does on
+  // several workgroups with a tail or a component phase. Elsewhere k_gs evaluates every sweep,
+  // so that its stagnation test knows the best residual of those sweeps too, and the
+  // threshold here is the best residual from the start.
+  int skip_early;
   uint32_t home;      // bodies of a workgroup that its LDS holds, and 64 more
   uint32_t rows;      // rows of a workgroup's contacts, at most
   uint32_t kept;      // contacts of a workgroup that its LDS holds

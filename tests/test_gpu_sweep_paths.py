@@ -1,5 +1,5 @@
-"""The sweeps of one workgroup with the bodies in LDS (k_gs_wg) and the sweeps without barriers
-between the colours (k_gs_flow) against the sweeps with grid barriers (both switched off):
+"""The sweeps without barriers between the colours (k_gs_flow), on one workgroup and on several,
+against the sweeps with grid barriers (the others switched off):
 every contact is updated in its colour's turn with the same expressions, so steps are the
 same bit for bit -- positions, velocities, impulses, sweep counts, residuals -- in FP64 and in
 FP32 with the FP64 polish, converging, ending at a sweep limit with the best iterate, through
@@ -30,7 +30,6 @@ def _scene(kind):
 
 
 def _run(monkeypatch, s, path, prm, steps, blocks=None):
-    monkeypatch.setenv("SCX_WG_SWEEPS", "1" if path == "wg" else "0")
     monkeypatch.setenv("SCX_FLOW_SWEEPS", "1" if path == "flow" else "0")
     if blocks:
         monkeypatch.setenv("SCX_FLOW_BLOCKS", str(blocks))
@@ -79,7 +78,7 @@ def test_one_workgroup(monkeypatch, kind, precision, limit):
     print("case", kind, precision, limit, flush=True)
     s = _scene(kind)
     prm = _params(s, precision, limit)
-    _same(_run(monkeypatch, s, "", prm, 3), _run(monkeypatch, s, "wg", prm, 3))
+    _same(_run(monkeypatch, s, "", prm, 3), _run(monkeypatch, s, "flow", prm, 3, 1))
 
 
 @pytest.mark.parametrize("kind,blocks", [("circles", 2), ("circles", None), ("lattice", 7), ("2500", 3), ("2500", None),
