@@ -111,7 +111,8 @@ __device__ __forceinline__ void local_solve(const Rec<D, Real>& R, const Real u[
   }
   if (D == 2) rn[2] = 0;
   const Real lim = R.mu * n0;
-  const Real nrm = sqrt(nrm2);
+  // (2D: the root of a rounded square is the number's size, up to the range's ends)
+  const Real nrm = D == 2 ? fabs(rn[1]) : sqrt(nrm2);
   if (nrm > lim) {
     const Real sc = (nrm > (Real)0) ? lim / nrm : (Real)0;
 #pragma unroll
@@ -126,7 +127,7 @@ __device__ __forceinline__ T fb_err(T mu, const T* r, const T* u) {
   T uT2 = (T)0;
 #pragma unroll
   for (int a = 1; a < D; ++a) uT2 += u[a] * u[a];
-  const T un_hat = u[0] + mu * sqrt(uT2);
+  const T un_hat = u[0] + mu * (D == 2 ? fabs(u[1]) : sqrt(uT2));  // (2D as in local_solve)
   T xh[3], yh[3];
   xh[0] = mu * r[0];
   yh[0] = un_hat;
@@ -144,14 +145,14 @@ __device__ __forceinline__ T fb_err(T mu, const T* r, const T* u) {
     z1[a - 1] = (T)2 * (xh[0] * xh[a] + yh[0] * yh[a]);
     nz1 += z1[a - 1] * z1[a - 1];
   }
-  nz1 = sqrt(nz1);
+  nz1 = D == 2 ? fabs(z1[0]) : sqrt(nz1);
   const T s1 = sqrt(z0 + nz1);
   const T s2 = sqrt(fmax((T)0, z0 - nz1));
   T e = xh[0] + yh[0] - (T)0.5 * (s1 + s2);
   e = e * e;
 #pragma unroll
   for (int a = 1; a < D; ++a) {
-    const T dir = nz1 > (T)0 ? z1[a - 1] / nz1 : (T)0;
+    const T dir = !(nz1 > (T)0) ? (T)0 : D == 2 ? copysign((T)1, z1[0]) : z1[a - 1] / nz1;
     const T p = xh[a] + yh[a] - (T)0.5 * (s1 - s2) * dir;
     e += p * p;
   }
