@@ -179,7 +179,7 @@ __global__ void __launch_bounds__(kBlock) k_mlp_infer(uint32_t n, const float* _
 // 16-unit tiles of every layer and only their weight fragments (44, in registers, loaded once
 // and together instead of 78 KB staged through LDS); the activations, in the accumulators'
 // layout, which is the next layer's operand, pass through LDS. The order of every sum is that
-// of one wave's chain over kt. 2,048 samples: 8 us (one wave per tile, weights in LDS: 29 us).
+// of one wave's chain over kt. 2,048 samples: 7 us (one wave per tile, weights in LDS: 29 us).
 struct TrainBufs {
   uint16_t* h1t;
   uint16_t* h2t;
@@ -199,6 +199,14 @@ __global__ void __launch_bounds__(kBlock) k_mlp_fwdbwd(uint32_t nb, const uint32
   const int lane = threadIdx.x & 63;
   const int r = 4 * (lane >> 4), sl = lane & 15;
   const int u0 = 2 * (int)(threadIdx.x >> 6);  // the wave's unit tiles: u0, u0 + 1
+  const uint32_t ntiles = (nb + 15) / 16;
+  // the sample of this lane in tile t; read ahead of the weights and of the tile before, as its
+  // features wait for it
+  auto sample = [&](uint32_t t) {
+    const uint32_t i = t * 16 + sl;
+    return i < nb ? (idx ? idx[b0 + i] : b0 + i) : 0u;
+  };
+  uint32_t ahead = sample(blockIdx.x);
   bf16x4 w1[2], w2[2][8], w3[8], n3[2], n2[2][8];
   float b1[2][4], b2[2][4], b3[4];
 #pragma unroll
@@ -220,12 +228,11 @@ __global__ void __launch_bounds__(kBlock) k_mlp_fwdbwd(uint32_t nb, const uint32
   for (int kt = 0; kt < 8; ++kt) w3[kt] = frag(gw + kW3T, kt, lane);
 #pragma unroll
   for (int e = 0; e < 4; ++e) b3[e] = gb[kB3 + r + e];
-  const uint32_t ntiles = (nb + 15) / 16;
   float sse = 0.f;
   for (uint32_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
-    const uint32_t i = t * 16 + sl;
-    const bool valid = i < nb;
-    const uint32_t s = valid ? (idx ? idx[b0 + i] : b0 + i) : 0u;
+    const bool valid = t * 16 + sl < nb;
+    const uint32_t s = ahead;
+    ahead = sample(t + gridDim.x);
     const bf16x4 x = valid ? x_frag(X, 0xFFFFFFFFu, s, lane) : bf16x4{0, 0, 0, 0};
     float base[kMlpOut], tgt[kMlpOut];
 #pragma unroll
