@@ -47,10 +47,28 @@ __device__ __forceinline__ uint32_t block_exclusive_scan_u32(uint32_t v, uint32_
   return before + incl - v;
 }
 
+// Largest value of a wave, in every lane (all 64 lanes call it). Through the data-parallel
+// moves of the vector unit: a shuffle goes through the LDS unit, 12 of them one after the other
+// take as long as a whole residual, and the residuals of a sweep end in three such reductions.
+template <int Ctrl>
+__device__ __forceinline__ double dpp_max_f64(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = (int)b, hi = (int)(b >> 32);
+  // (a lane without a source keeps its own value)
+  const int lo2 = __builtin_amdgcn_update_dpp(lo, lo, Ctrl, 0xF, 0xF, false);
+  const int hi2 = __builtin_amdgcn_update_dpp(hi, hi, Ctrl, 0xF, 0xF, false);
+  return fmax(v, __longlong_as_double(((long long)hi2 << 32) | (uint32_t)lo2));
+}
 __device__ __forceinline__ double wave_reduce_max_f64(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
-  return v;
+  v = dpp_max_f64<0x111>(v);  // row_shr 1, 2, 4, 8: lane 15 of a row has the row's
+  v = dpp_max_f64<0x112>(v);
+  v = dpp_max_f64<0x114>(v);
+  v = dpp_max_f64<0x118>(v);
+  v = dpp_max_f64<0x142>(v);  // row_bcast 15, 31: from the rows before
+  v = dpp_max_f64<0x143>(v);
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)b, 63), hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
+  return __longlong_as_double(((long long)hi << 32) | (uint32_t)lo);
 }
 __device__ __forceinline__ double wave_reduce_min_f64(double v) {
 #pragma unroll
