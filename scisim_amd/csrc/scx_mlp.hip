@@ -325,8 +325,10 @@ struct Adam {
   float* bias;
   float lr, b1, b2, eps, c1, c2;
   __device__ __forceinline__ float step(uint32_t i, float pi, float mi, float vi, float gi) const {
-    mi = b1 * mi + (1.f - b1) * gi;
-    vi = b2 * vi + (1.f - b2) * gi * gi;
+    // (one rounding each fixed by hand: a small gradient's step has the size of the rate either
+    // way its moments round, so steps repeat only to the bit)
+    mi = fmaf(1.f - b1, gi, b1 * mi);
+    vi = fmaf(gi, (1.f - b2) * gi, b2 * vi);
     m[i] = mi;
     v[i] = vi;
     pi -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
