@@ -1085,7 +1085,7 @@ __global__ void __launch_bounds__(kGSBlock) k_gs_lds(GSArgs<Real> A) {
   Real* sw = (D == 3) ? sl + (size_t)2 * C : ss;                          // wn, wt, mu, f
   Real* sr = sw + (size_t)4 * C;                                           // impulses, 3 per contact
   __shared__ uint32_t off[kMaxColours + 1];
-  __shared__ double s_red[kGSBlock / 64];
+  __shared__ double s_red[2][kGSBlock / 64];
   const uint32_t tid = threadIdx.x;
   const uint32_t ncol = A.ctr->ncolours;
   for (uint32_t c = tid; c <= ncol; c += kGSBlock) off[c] = A.coloff[c];
@@ -1150,9 +1150,7 @@ __global__ void __launch_bounds__(kGSBlock) k_gs_lds(GSArgs<Real> A) {
     R.f = sw[4 * (size_t)k + 3];
   };
   // one contact: the k_gs update on LDS data (init: apply the stored impulse)
-  auto update = [&](uint32_t k, bool init) {
-    Rec<D, Real> R;
-    rec(k, R);
+  auto update_held = [&](uint32_t k, const Rec<D, Real>& R, const Real* r, bool init) __attribute__((always_inline)) {
     const bool hasb = R.b != kNoBody;
     V* bv = sb;
     const size_t ia = (size_t)kBodyVecs<D> * R.a, ib = (size_t)kBodyVecs<D> * R.b;
@@ -1163,7 +1161,6 @@ __global__ void __launch_bounds__(kGSBlock) k_gs_lds(GSArgs<Real> A) {
       if (D == 3) wb = bv[ib + 1];
     }
     Real* rp = sr + 3 * (size_t)k;
-    const Real r[3] = {rp[0], rp[1], rp[2]};
     Real dr[3];
     if (init) {
       dr[0] = r[0];
@@ -1211,6 +1208,16 @@ __global__ void __launch_bounds__(kGSBlock) k_gs_lds(GSArgs<Real> A) {
       }
     }
   };
+  auto update = [&](uint32_t k, bool init) {
+    Rec<D, Real> R;
+    rec(k, R);
+    const Real* rp = sr + 3 * (size_t)k;
+    const Real r[3] = {rp[0], rp[1], rp[2]};
+    update_held(k, R, r, init);
+  };
+  // A barrier for what lies in LDS: stores to memory (the best iterate) are not waited for.
+  auto lds_barrier = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+  uint32_t red = 0;
   auto residual = [&]() -> double {
     double m = 0.0;
     for (uint32_t k = tid; k < C; k += kGSBlock) {
@@ -1236,11 +1243,12 @@ __global__ void __launch_bounds__(kGSBlock) k_gs_lds(GSArgs<Real> A) {
       }
     }
     m = wave_reduce_max_f64(m);
-    if ((tid & 63) == 0) s_red[tid >> 6] = m;
-    __syncthreads();
-    double out = s_red[0];
-    for (int w = 1; w < kGSBlock / 64; ++w) out = fmax(out, s_red[w]);
-    __syncthreads();
+    red ^= 1u;  // (the other one may still be read)
+    if ((tid & 63) == 0) s_red[red][tid >> 6] = m;
+    lds_barrier();
+    double out = s_red[red][0];
+#pragma unroll
+    for (int w = 1; w < kGSBlock / 64; ++w) out = fmax(out, s_red[red][w]);
     return out;
   };
   // v = v0 + M^-1 H^T r: reset the owned bodies to v0, then apply every impulse colour by colour
@@ -1286,11 +1294,30 @@ __global__ void __launch_bounds__(kGSBlock) k_gs_lds(GSArgs<Real> A) {
   // the FP32 phase stops on an FP32 estimate with a factor-2 margin; the FP64 phase
   // that follows decides on the tolerance
   const double stop = (A.phase == 1) ? 0.5 * A.tol : A.tol;
+  // A colour is a chain of LDS reads (its offsets, the record, the bodies) and the solve: the
+  // record and impulse of a thread's first contact of the next colour, which no other thread
+  // writes, are read before the barrier, so only the bodies are left behind it.
+  Rec<D, Real> held;
+  Real held_r[3];
+  uint32_t held_k = off[0] + tid;
+  bool has = held_k < off[ncol ? 1 : 0];
+  auto hold = [&]() {
+    if (!has) return;
+    rec(held_k, held);
+    for (int d = 0; d < 3; ++d) held_r[d] = sr[3 * (size_t)held_k + d];
+  };
   if (!(err < stop)) {
+    hold();
     for (it = 1; it <= max_iters; ++it) {
       for (uint32_t col = 0; col < ncol; ++col) {
-        for (uint32_t k = off[col] + tid; k < off[col + 1]; k += kGSBlock) update(k, false);
-        __syncthreads();
+        const uint32_t next = col + 1 < ncol ? col + 1 : 0u, lo = off[next], hi = off[next + 1];
+        if (has) update_held(held_k, held, held_r, false);
+        for (uint32_t k = held_k + kGSBlock; k < off[col + 1]; k += kGSBlock) update(k, false);
+        held_k = lo + tid;
+        has = held_k < hi;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the bodies are written
+        hold();  // (on its way while the barrier is waited for)
+        asm volatile("s_barrier" ::: "memory");
       }
       if (A.eval_every > 0 && it % A.eval_every == 0) {
         err = residual();
