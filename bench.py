@@ -433,7 +433,7 @@ def main():
     if pairs_ms >= gs_ms:
         kernel, launches, kbytes, kms = "k_pairs (grid neighbour sweep + FP64 narrow phase)", 2, pairs_bytes, pairs_ms
     else:
-        kernel, launches, kbytes, kms = "k_gs (coloured Gauss-Seidel, persistent)", 1 + int(fp32), gs_bytes, gs_ms
+        kernel, launches, kbytes, kms = "Gauss-Seidel sweeps (k_gs_flow; k_gs above 2,097,152 contacts)", 1 + int(fp32), gs_bytes, gs_ms
     traffic = None
     if args.traffic:
         traffic = read_traffic(args.traffic).get("bytes_per_launch")

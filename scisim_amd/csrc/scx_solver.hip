@@ -1514,15 +1514,15 @@ static hipError_t tune_after_solve(scx_ctx* c) {
 // (shared by the two phases of a solve).
 constexpr uint32_t kFlowTagMax = 1u << 30;
 // Ahead of the sweeps with barriers at every size measured (whole solves, ms, with barriers and
-// without): spheres 16,987 contacts 15.3 and 6.2, 34,176 20.5 and 9.4, 99,626 17.1 and 8.5,
-// 423,718 30.1 and 14.9, 848,458 18.9 and 8.7, 1,283,826 18.6 and 11.8. kFlowMaxContacts bounds
+// without): spheres 16,987 contacts 14.9 and 6.2, 34,176 20.7 and 9.2, 99,626 17.1 and 8.4,
+// 423,718 30.1 and 13.9, 848,458 19.0 and 8.5, 1,283,826 18.7 and 11.4. kFlowMaxContacts bounds
 // the buffers (0.5 GB per million contacts). Workgroups: 128 contacts each, up to the CUs in use.
 constexpr uint32_t kFlowMaxContacts = 1u << 21;
 constexpr uint32_t kFlowContacts = 128;  // contacts of a workgroup
 // Up to kFlowOneXcd contacts one XCD's CUs do better than all: every slot is then a near one
 // (k_gs_flow), and more bodies live in LDS. One XCD against eight, whole solves of 300 to 2,000
-// sweeps in ms: circles 13,169 contacts 20.2 and 24.8, 24,976 8.6 and 10.1; spheres 16,987 6.2
-// and 7.4, 34,176 9.4 and 11.0, 67,457 8.7 and 8.6, 99,626 11.4 and 8.5.
+// sweeps in ms: circles 13,169 contacts 18.3 and 23.4, 24,976 7.6 and 9.6; spheres 16,987 6.2
+// and 7.6, 34,176 9.2 and 10.4, 67,457 8.4 and 8.0, 99,626 11.3 and 8.4.
 constexpr uint32_t kFlowOneXcd = 1u << 16;
 // Up to kFlowOneGroup contacts one workgroup does better than several: all its bodies live in its
 // LDS. One workgroup, two and eight, FP64 solves in ms: spheres 522 contacts 3.5, 4.9 and 5.1,

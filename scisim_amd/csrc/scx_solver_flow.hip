@@ -19,6 +19,11 @@
 // No store is waited for, nothing is read that has not been written, and the stores of a wave
 // are contiguous.
 //
+// A hop (wait, solve, store) takes 1,600 cycles through LDS, 2,200 through one XCD's L2 and up to
+// 5,000 across XCDs, and a sweep is a chain of about as many hops as there are colours. Measured,
+// per FP32 and FP64 sweep (the latter with its residual): 34,176 sphere contacts 18.5 and 36 us
+// (with barriers 44.6 and 80), 423,718 sphere contacts 28 and 55 us (59 and 124).
+//
 // The iterates are those of the colour passes bit for bit: the order of the contacts on
 // every body is the colour order, and a contact reads nothing but its own two bodies.
 // Progress: the launch is cooperative (every workgroup resident), a wave takes its contacts
