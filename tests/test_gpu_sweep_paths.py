@@ -105,13 +105,49 @@ def test_without_barriers_spread(monkeypatch, kind, xcds, blocks, precision):
     _same(ref, _run(monkeypatch, s, "flow", prm, 3, blocks))
 
 
-@pytest.mark.parametrize("blocks", [None, 3, 256])
+@pytest.mark.parametrize("side", [7, 8, 12])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_stand_alone_solve_without_barriers(monkeypatch, side, precision):
+    """Contacts in no order: 882 (one workgroup), 1,344 and 4,752 (equal shares of each colour)."""
+    print("case", side, precision, flush=True)
+    rng = np.random.default_rng(side)
+    at = np.arange(side ** 3).reshape(side, side, side)
+    a = np.concatenate([np.delete(at, -1, k).ravel() for k in range(3)])
+    b = np.concatenate([np.delete(at, 0, k).ravel() for k in range(3)])
+    axis = np.repeat(np.arange(3), a.size // 3)
+    order = rng.permutation(a.size)
+    a, b, axis = a[order], b[order], axis[order]
+    nn = -np.eye(3)[axis]
+    t1 = np.eye(3)[(axis + 1) % 3]
+    prob = dict(m=rng.uniform(1.0, 2.0, side ** 3), inertia=rng.uniform(0.1, 0.2, side ** 3),
+                v0=rng.normal(size=3 * side ** 3), omega0=rng.normal(size=3 * side ** 3), body0=a.astype(np.int32),
+                body1=b.astype(np.int32), bases=np.stack([nn, t1, np.cross(nn, t1)], 1), arm0=-0.5 * nn,
+                arm1=0.5 * nn, mu=np.full(a.size, 0.4))
+
+    def run(flow):
+        monkeypatch.setenv("SCX_FLOW_SWEEPS", flow)
+        monkeypatch.delenv("SCX_FLOW_BLOCKS", raising=False)
+        ctx = scx.Context(3, side ** 3, max_planes=8)
+        try:
+            return ctx.friction_solve(tol=1e-9, max_iters=400, eval_every=1,
+                                      precision=scx.FP64 if precision == "fp64" else scx.FP32_POLISH, **prob)
+        finally:
+            ctx.close()
+
+    ref, got = run("0"), run("1")
+    print(ref["sweeps"], ref["error"], flush=True)
+    for key, x in ref.items():
+        assert np.array_equal(x, got[key]), key
+
+
+@pytest.mark.parametrize("scenes_,blocks", [(3, None), (70, None), (70, 3), (70, 256)])
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
 @pytest.mark.parametrize("limit", ["converged", "limit", "sparse", "stagnates"])
-def test_ensemble_without_barriers(monkeypatch, blocks, precision, limit):
-    """70 piles (more than two words of the frozen mask), most of which freeze on the way."""
-    print("case", blocks, precision, limit, flush=True)
-    cat, body_off, plane_off, mus, _ = scenes.ensemble_piles(nscenes=70, nmin=20, nmax=200, seed=4, workers=4)
+def test_ensemble_without_barriers(monkeypatch, scenes_, blocks, precision, limit):
+    """70 piles (more than two words of the frozen mask), most of which freeze on the way, and 3
+    (one workgroup)."""
+    print("case", scenes_, blocks, precision, limit, flush=True)
+    cat, body_off, plane_off, mus, _ = scenes.ensemble_piles(nscenes=scenes_, nmin=20, nmax=200, seed=4, workers=4)
     prm = _params(cat, precision, limit)
 
     def run(path):
