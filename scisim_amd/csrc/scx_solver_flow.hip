@@ -71,9 +71,6 @@ struct FlowPort {
 #pragma unroll
     for (int i = 0; i < NP; ++i) x.p[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, o + 16u * i, 0, kFlowAux);
   }
-  __device__ __forceinline__ uint32_t tag(uint32_t slot) const {  // of its last piece
-    return __builtin_amdgcn_raw_buffer_load_b32(rs, at(slot) + 16u * (NP - 1) + 12u, 0, kFlowAux);
-  }
   __device__ __forceinline__ static bool is(const Raw& x, uint32_t tag) {
     bool ok = true;
 #pragma unroll
