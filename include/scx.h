@@ -297,6 +297,16 @@ typedef struct scx_sweep_counters {
 } scx_sweep_counters;
 int scx_get_sweep_counters(const scx_ctx* ctx, scx_sweep_counters* out);
 
+/* Which kernel swept the last contact set (of a step or a stand-alone solve), per phase
+ * (path[0] the FP32 phase, path[1] FP64; SCX_SWEEPS_NONE: the phase did not run), and on how
+ * many workgroups (may be NULL). Every kernel gives the same iterates; for tests and
+ * measurements. */
+#define SCX_SWEEPS_NONE 0
+#define SCX_SWEEPS_LDS 1      /* one workgroup, everything in its LDS */
+#define SCX_SWEEPS_FLOW 2     /* a contact waits for the contacts before it on its bodies alone */
+#define SCX_SWEEPS_BARRIERS 3 /* grid barriers between the colours */
+int scx_get_sweep_paths(const scx_ctx* ctx, int32_t* path, uint32_t* workgroups);
+
 /* Online autotuning of the persistent Gauss-Seidel launches (no counterpart in the
  * reference, whose So-bogus solve has no launch shape; this is for callers that step
  * one kind of scene many times). Enabled, each sweep launch runs on the cost model's

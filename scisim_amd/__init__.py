@@ -36,7 +36,7 @@ STAGGER_STABILIZED = 2
 # Every symbol include/scx.h declares.
 EXPORTS = ["scx_version", "scx_last_error", "scx_create", "scx_destroy", "scx_potential_overlaps", "scx_set_bodies",
            "scx_set_planes", "scx_get_state", "scx_step", "scx_run", "scx_get_contacts", "scx_get_v2",
-           "scx_friction_solve", "scx_unconstrained_flow", "scx_set_timing", "scx_get_timing", "scx_get_sweep_counters",
+           "scx_friction_solve", "scx_unconstrained_flow", "scx_set_timing", "scx_get_timing", "scx_get_sweep_counters", "scx_get_sweep_paths",
            "scx_set_warm_model", "scx_get_warm_model", "scx_get_samples", "scx_warm_model_gradients",
            "scx_train_warm_model", "scx_set_scenes", "scx_get_scene_stats", "scx_set_autotune", "scx_get_autotune",
            "scx_save_checkpoint", "scx_load_checkpoint", "scx_checkpoint_info", "scx_get_contact_forces", "scx_potential_overlaps_noalloc"]
@@ -126,6 +126,7 @@ def lib():
         L.scx_set_timing.argtypes = [_vp, ctypes.c_int32]
         L.scx_get_timing.argtypes = [_vp, ctypes.c_uint32, ctypes.POINTER(ctypes.c_char_p), _pd, _pu32]
         L.scx_get_sweep_counters.argtypes = [_vp, ctypes.POINTER(ScxSweepCounters)]
+        L.scx_get_sweep_paths.argtypes = [_vp, _pi32, _pu32]
         L.scx_set_autotune.argtypes = [_vp, ctypes.c_int32]
         L.scx_get_autotune.argtypes = [_vp, ctypes.c_uint32, _pu32, _pi32, _pi32, _pf, _pi32, _pu32]
         L.scx_set_warm_model.argtypes = [_vp, _pf, ctypes.c_uint32]
@@ -377,6 +378,16 @@ class Context:
         return {"full": x.full_evals, "full_fp32": x.full_evals_fp32, "skipped": x.skipped_evals,
                 "component_launches": x.component_launches, "component_overflows": x.component_overflows,
                 "component_width": x.component_width, "component_share": x.component_share}
+
+    def sweep_paths(self):
+        """The kernel that swept the last contact set and its workgroups, per phase: None or
+        "lds", "flow" (no barriers between the colours), "barriers", and the workgroups."""
+        path = np.zeros(2, dtype=np.int32)
+        groups = np.zeros(2, dtype=np.uint32)
+        self._check(lib().scx_get_sweep_paths(self._h, _p(path, _pi32), _p(groups, _pu32)),
+                    "scx_get_sweep_paths")
+        names = (None, "lds", "flow", "barriers")
+        return {"fp32": (names[path[0]], int(groups[0])), "fp64": (names[path[1]], int(groups[1]))}
 
     def set_autotune(self, on):
         """Online autotuning of the sweep launch width (results do not depend on it)."""

@@ -626,6 +626,10 @@ int scx_create(const scx_config* cfg, scx_ctx** out) {
     if (getenv("SCX_COMPONENT_SWEEPS") || getenv("SCX_COMPONENT_PERCENT") || getenv("SCX_COHERENT_SWEEPS"))
       c->flow_sweeps = false;
     if (const char* env = getenv("SCX_FLOW_SWEEPS")) c->flow_sweeps = atoi(env) != 0;
+    // SCX_FLOW_BLOCKS, SCX_FLOW_XCDS: those sweeps on a fixed number of workgroups and of XCDs
+    // (the results depend on neither; for tests)
+    if (const char* env = getenv("SCX_FLOW_BLOCKS")) c->flow_blocks = std::max(0, atoi(env));
+    if (const char* env = getenv("SCX_FLOW_XCDS")) c->flow_xcds = std::max(1, std::min(atoi(env), (int)kXcds));
     if ((e = dalloc(&d.partial, (size_t)std::max(c->gs_blocks, 1) + 1)) != hipSuccess ||
         (e = dalloc(&d.viol, (size_t)3 + kViolCap)) != hipSuccess ||
         (e = dalloc(&d.comp_cnt, (size_t)std::max(c->gs_blocks, 1) + 1)) != hipSuccess ||
@@ -1665,6 +1669,15 @@ int scx_get_sweep_counters(const scx_ctx* c, scx_sweep_counters* out) {
     out->component_width = h->comp_maxw;
   }
   out->component_share = c->comp_share;
+  return SCX_OK;
+}
+
+int scx_get_sweep_paths(const scx_ctx* c, int32_t* path, uint32_t* workgroups) {
+  if (!c || !path) return SCX_E_ARG;
+  for (int k = 0; k < 2; ++k) {
+    path[k] = c->sweep_path[k];
+    if (workgroups) workgroups[k] = c->sweep_groups[k];
+  }
   return SCX_OK;
 }
 

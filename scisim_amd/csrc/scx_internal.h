@@ -287,6 +287,11 @@ struct scx_ctx {
   bool barrier_sweeps = false;  // the last solve swept with grid barriers (k_gs)
   bool flow_sweeps = true;      // sweep without barriers between the colours (k_gs_flow)
   uint32_t flow_tag = 1;        // next unused tag of those sweeps' slots
+  int flow_blocks = 0;          // > 0: workgroups of those sweeps (tests)
+  int flow_xcds = 0;            // > 0: XCDs they are spread over (tests)
+  // kernel that swept the last contact set, per phase (FP32, FP64; SCX_SWEEPS_*), and its workgroups
+  int sweep_path[2] = {0, 0};
+  uint32_t sweep_groups[2] = {0, 0};
   // The device's cooperative queues are limited in number (HSA_QUEUE_TYPE_COOPERATIVE,
   // hsa/hsa.h: "Queues of this type may be limited in number"); while another process holds
   // them a cooperative launch fails with hipErrorIllegalState. The persistent kernels need

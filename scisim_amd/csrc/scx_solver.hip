@@ -1664,9 +1664,8 @@ static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint
   // the autotuner picks among widths around the model's (not for the solves of one workgroup)
   const int phase = std::is_same<Real, double>::value ? 1 : 0;
   const bool tune = c->tuner.enabled && c->force_blocks <= 0 && !lds_path && !(flow && one) && !c->coop_unavailable;
-  // one XCD's CUs up to flow_one_xcd contacts, all beyond
-  uint32_t xcds = A.C <= kFlowOneXcd ? 1 : kXcds;
-  if (const char* env = getenv("SCX_FLOW_XCDS")) xcds = (uint32_t)std::max(1, std::min(atoi(env), (int)kXcds));
+  // one XCD's CUs up to kFlowOneXcd contacts, all beyond
+  const uint32_t xcds = c->flow_xcds > 0 ? (uint32_t)c->flow_xcds : A.C <= kFlowOneXcd ? 1 : kXcds;
   const int flow_most = std::min(max_blocks, kFlowMaxBlocks) / (int)kXcds * (int)xcds;
   const int width =
       !flow ? model : one ? 1 : std::max(2, std::min((int)((A.C + kFlowContacts - 1) / kFlowContacts), flow_most));
@@ -1684,6 +1683,8 @@ static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint
   const int skip_early = blocks > 1 && (tail < ncol || A.comp_parent) ? 1 : 0;
   if (lds_path) {
     // the whole solve in one workgroup's LDS
+    c->sweep_path[phase] = SCX_SWEEPS_LDS;
+    c->sweep_groups[phase] = 1;
     hipError_t e = hipFuncSetAttribute((const void*)k_gs_lds<D, Real>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                        (int)lds);
     if (e != hipSuccess) return e;
@@ -1696,11 +1697,10 @@ static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint
   bool launched = false;
   if (flow) {
     FlowBufs<Real> F;
-    // SCX_FLOW_BLOCKS, SCX_FLOW_XCDS: a fixed workgroup count and spread (the results do not
-    // depend on them; for tests)
-    int fb = want;
-    if (const char* env = getenv("SCX_FLOW_BLOCKS")) fb = atoi(env);
+    const int fb = c->flow_blocks > 0 ? c->flow_blocks : want;
     const uint32_t per_xcd = ((uint32_t)std::max(1, std::min(fb, flow_most)) + xcds - 1) / xcds;
+    c->sweep_path[phase] = SCX_SWEEPS_FLOW;
+    c->sweep_groups[phase] = xcds * per_xcd;
     e = flow_prepare<D, Real>(c, A, xcds, per_xcd, linked, F);
     if (e != hipSuccess && e != hipErrorOutOfMemory) return e;
     if (e == hipSuccess) {
@@ -1714,12 +1714,15 @@ static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint
     }
   }
   c->barrier_sweeps = true;
+  c->sweep_path[phase] = SCX_SWEEPS_BARRIERS;
+  c->sweep_groups[phase] = (uint32_t)blocks;
   const void* fn = coh ? (const void*)k_gs<D, Real, true> : (const void*)k_gs<D, Real, false>;
   e = launch_cooperative(c, fn, blocks, kGSBlock, args, 0, c->stream, &launched);
   if (e == hipSuccess && !launched) {
     // one workgroup (chosen, or after a refused cooperative launch: see
     // scx_ctx::coop_unavailable) sweeps every colour itself, so there is no tail split
     A.tail_col = (uint32_t)kMaxColours;
+    c->sweep_groups[phase] = 1;
     e = hipLaunchKernel(fn, dim3(1), dim3(kGSBlock), args, 0, c->stream);
   }
   if (e == hipSuccess && tune) e = hipEventRecord(c->tuner.pend[phase].ev[1], c->stream);
@@ -1752,6 +1755,10 @@ __global__ void __launch_bounds__(kBlock) k_contact_scene(uint32_t C, const uint
 template <int D>
 static hipError_t solve_dim(scx_ctx* c, uint32_t C, const uint32_t* col_off, const scx_step_params* p) {
   hipStream_t s = c->stream;
+  for (int k = 0; k < 2; ++k) {
+    c->sweep_path[k] = SCX_SWEEPS_NONE;
+    c->sweep_groups[k] = 0;
+  }
   if (c->tuner.enabled) tune_resolve(c);
   const bool fp32 = p->precision == SCX_PRECISION_FP32_POLISH;
   const bool warm = p->warm_start != SCX_WARM_NONE;
