@@ -620,6 +620,9 @@ int scx_create(const scx_config* cfg, scx_ctx** out) {
       c->comp_share = std::min(100.0, std::max(1.0, atof(env)));
       c->comp_adapt = false;
     }
+    // SCX_LDS_SWEEPS=0: sets that one workgroup's LDS would hold whole take the other sweeps
+    // (for tests)
+    if (const char* env = getenv("SCX_LDS_SWEEPS")) c->lds_sweeps = atoi(env) != 0;
     // SCX_FLOW_SWEEPS=0: sweeps with grid barriers between the colours (the same iterates bit
     // for bit; for A/B measurements and tests). The switches of those sweeps above keep a
     // context on them unless it says otherwise.

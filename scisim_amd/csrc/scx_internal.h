@@ -285,6 +285,7 @@ struct scx_ctx {
   double comp_ceiling = 100.0;  // below the last share that overflowed (drifts back up)
   bool comp_adapt = true;
   bool barrier_sweeps = false;  // the last solve swept with grid barriers (k_gs)
+  bool lds_sweeps = true;       // small sets are swept whole in one workgroup's LDS (k_gs_lds)
   bool flow_sweeps = true;      // sweep without barriers between the colours (k_gs_flow)
   uint32_t flow_tag = 1;        // next unused tag of those sweeps' slots
   int flow_blocks = 0;          // > 0: workgroups of those sweeps (tests)

@@ -1651,7 +1651,7 @@ static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint
       c->force_blocks > 0 ? c->force_blocks : persistent_blocks(widths, nw, kGSBlock, max_blocks, coh);
   const size_t lds = LdsLayout<D, Real>::bytes(A.C);
   const bool lds_path = std::min(max_blocks, model) <= 1 && c->force_blocks <= 0 && lds <= kGSLdsMax && A.lmap &&
-                        !A.cscene;
+                        !A.cscene && c->lds_sweeps;
   const bool free_width = c->force_blocks <= 0 && !lds_path;
   // no barriers between the colours: up to kFlowMaxContacts, while the slots can be addressed
   // and the tags last; ensembles of up to kFlowMaxScenes scenes. One workgroup for small sets,

@@ -1,14 +1,21 @@
-"""Which sweep kernel serves which contact set (scx_get_sweep_paths)."""
+"""Which sweep kernel serves which contact set (scx_get_sweep_paths), and the kernels against each
+other. The iterates of all three are the same bit for bit. At a sweep limit the one-workgroup LDS
+kernel takes the velocities anew from the best impulses also where the last iterate is the best,
+which the other two leave as the sweeps made them: the same impulses, velocities that round
+differently.
+"""
 
+import numpy as np
 import pytest
 
 import scisim_amd as scx
+from scisim_amd import scenes
 
 import test_gpu_sweep_paths as base
 
 pytestmark = pytest.mark.gpu
 
-SWITCHES = ("SCX_FLOW_SWEEPS", "SCX_FLOW_BLOCKS", "SCX_FLOW_XCDS", "SCX_FORCE_PERSISTENT_BLOCKS")
+SWITCHES = ("SCX_LDS_SWEEPS", "SCX_FLOW_SWEEPS", "SCX_FLOW_BLOCKS", "SCX_FLOW_XCDS", "SCX_FORCE_PERSISTENT_BLOCKS")
 
 
 def _context(monkeypatch, s, **env):
@@ -20,6 +27,29 @@ def _context(monkeypatch, s, **env):
     ctx.set_planes(s["px"], s["pn"])
     ctx.set_bodies(s["q"], s["v"], s["r"], s["m"], inertia=s.get("inertia"))
     return ctx
+
+
+def _run(monkeypatch, s, prm, steps, **env):
+    ctx = _context(monkeypatch, s, **env)
+    try:
+        out, paths = [], []
+        for _ in range(steps):
+            st = ctx.step(scx.step_params(**prm))
+            con = ctx.contacts()
+            out.append((st, *ctx.get_state(), con["alpha"], con["beta"]))
+            if st["ncontacts"]:
+                paths.append(ctx.sweep_paths())
+        return out, paths
+    finally:
+        ctx.close()
+
+
+def _all(paths, precision, path, groups=None):
+    assert paths
+    for p in paths:
+        for phase in ("fp32", "fp64") if precision == "fp32" else ("fp64",):
+            assert p[phase][0] == path, p
+            assert groups is None or p[phase][1] == groups, p
 
 
 def test_switches_are_read_when_a_context_is_made(monkeypatch):
@@ -36,3 +66,95 @@ def test_switches_are_read_when_a_context_is_made(monkeypatch):
         assert path == "flow" and 8 < groups <= 32  # one XCD's share of 128 contacts a workgroup
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("kind", ["one", "60", "lattice"])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("limit", ["converged", "limit", "sparse", "stagnates"])
+def test_small_sets_in_all_three_kernels(monkeypatch, kind, precision, limit):
+    """Sets that one workgroup's LDS holds whole, in that kernel, in the sweeps without barriers on
+    one and two workgroups and in those with barriers."""
+    print("case", kind, precision, limit, flush=True)
+    s = base._scene(kind)
+    prm = base._params(s, precision, limit)
+    ref, paths = _run(monkeypatch, s, prm, 3, SCX_FORCE_PERSISTENT_BLOCKS=2)
+    _all(paths, precision, "barriers", 2)
+    for blocks in (1, 2):
+        got, paths = _run(monkeypatch, s, prm, 3, SCX_LDS_SWEEPS=0, SCX_FLOW_BLOCKS=blocks)
+        _all(paths, precision, "flow", blocks)
+        base._same(ref, got)
+    got, paths = _run(monkeypatch, s, prm, 3)
+    _all(paths, precision, "lds", 1)
+    # up to the first step that ends at the limit, whose velocities go into the next ones
+    upto = next((k for k, a in enumerate(ref) if not a[0]["succeeded"]), len(ref))
+    base._same(ref[:upto], got[:upto])
+    if upto < len(ref):
+        a, b = ref[upto], got[upto]
+        for key in ("ncontacts", "ncolours", "sweeps", "sweeps_fp32", "error", "succeeded"):
+            assert a[0][key] == b[0][key], key
+        for x, y in zip(a[4:], b[4:]):  # impulses
+            assert np.array_equal(x, y)
+
+
+def _grid(m):
+    """m x m circles that overlap their neighbours by a little: 2 m (m - 1) contacts."""
+    q = np.stack(np.meshgrid(np.arange(m), np.arange(m)), -1).reshape(-1, 2) * 0.0999
+    return dict(dim=2, q=q.ravel(), v=np.random.default_rng(m).normal(0.0, 0.1, 2 * m * m), r=np.full(m * m, 0.05),
+                m=np.ones(m * m), px=np.array([[0.0, -10.0]]), pn=np.array([[0.0, 1.0]]))
+
+
+@pytest.mark.parametrize("m,groups", [(160, 32), (200, 256), (1020, 256), (1030, None)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_large_sets(monkeypatch, m, groups, precision):
+    """One XCD's workgroups below 65,536 contacts (50,880 here), every XCD's above (79,600), up to
+    2,097,152 contacts (2,078,760); grid barriers beyond (2,119,740)."""
+    print("case", m, precision, flush=True)
+    s = _grid(m)
+    prm = dict(base._params(s, precision, "limit"), max_iters=24, g=[0.0, 0.0])
+    ref, paths = _run(monkeypatch, s, prm, 1, SCX_FLOW_SWEEPS=0)
+    _all(paths, precision, "barriers")
+    assert ref[0][0]["ncontacts"] >= 2 * m * (m - 1)
+    got, paths = _run(monkeypatch, s, prm, 1)
+    print(ref[0][0], paths, flush=True)
+    _all(paths, precision, "flow" if groups else "barriers", groups)
+    base._same(ref, got)
+
+
+def _paths_at_close(monkeypatch):
+    seen, close = [], scx.Context.close
+
+    def record(self):
+        seen.append(self.sweep_paths())
+        close(self)
+
+    monkeypatch.setattr(scx.Context, "close", record)
+    monkeypatch.setenv("SCX_FLOW_SWEEPS", "0")
+    return seen
+
+
+@pytest.mark.parametrize("limit", ["converged", "sweep_limit"])
+def test_compacted_ensembles_with_barriers(monkeypatch, limit):
+    """The compaction belongs to the sweeps with barriers, which serve the largest ensembles."""
+    import test_gpu_ensemble_compaction as t
+
+    seen = _paths_at_close(monkeypatch)
+    piles = scenes.ensemble_piles(nscenes=96, nmin=100, nmax=2000, seed=3, workers=8)
+    t.test_compacted_sweeps_match_uncompacted_bit_for_bit(monkeypatch, piles, 0, limit)
+    _all(seen, "fp32", "barriers")
+    assert len(seen) == 2 and all(p["fp32"][1] > 1 for p in seen)
+
+
+@pytest.mark.parametrize("mode", ["transport", "cold", "fp64", "fp64_limit"])
+def test_skipped_evaluations_with_barriers(monkeypatch, mode):
+    """The list of contacts near the maximum belongs to the sweeps with barriers."""
+    import test_gpu_violator_skip as t
+
+    seen = _paths_at_close(monkeypatch)
+
+    class Request:
+        def getfixturevalue(self, kind):
+            return scenes.spheres_pile(n=8000, seed=9)
+
+    t.test_skipped_evaluations_change_nothing(monkeypatch, Request(), "pile", 0, mode)
+    _all(seen, "fp64" if mode.startswith("fp64") else "fp32", "barriers")
+    assert all(p["fp64"][1] > 1 for p in seen)
