@@ -633,6 +633,9 @@ int scx_create(const scx_config* cfg, scx_ctx** out) {
     // (the results depend on neither; for tests)
     if (const char* env = getenv("SCX_FLOW_BLOCKS")) c->flow_blocks = std::max(0, atoi(env));
     if (const char* env = getenv("SCX_FLOW_XCDS")) c->flow_xcds = std::max(1, std::min(atoi(env), (int)kXcds));
+    // SCX_FLOW_POLLS: the looks after which a wait for a body in those sweeps has run out and the
+    // step fails (for tests of that failure)
+    if (const char* env = getenv("SCX_FLOW_POLLS")) c->flow_polls = (uint32_t)std::max(0, atoi(env));
     if ((e = dalloc(&d.partial, (size_t)std::max(c->gs_blocks, 1) + 1)) != hipSuccess ||
         (e = dalloc(&d.viol, (size_t)3 + kViolCap)) != hipSuccess ||
         (e = dalloc(&d.comp_cnt, (size_t)std::max(c->gs_blocks, 1) + 1)) != hipSuccess ||

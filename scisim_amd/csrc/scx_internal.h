@@ -290,6 +290,7 @@ struct scx_ctx {
   uint32_t flow_tag = 1;        // next unused tag of those sweeps' slots
   int flow_blocks = 0;          // > 0: workgroups of those sweeps (tests)
   int flow_xcds = 0;            // > 0: XCDs they are spread over (tests)
+  uint32_t flow_polls = 0;      // > 0: looks of a wait for a body, at most (tests)
   // kernel that swept the last contact set, per phase (FP32, FP64; SCX_SWEEPS_*), and its workgroups
   int sweep_path[2] = {0, 0};
   uint32_t sweep_groups[2] = {0, 0};

@@ -1705,6 +1705,7 @@ static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint
     if (e != hipSuccess && e != hipErrorOutOfMemory) return e;
     if (e == hipSuccess) {
       F.skip_early = skip_early;
+      F.polls = c->flow_polls ? c->flow_polls : kFlowPolls;
       if (A.cscene) e = hipMemsetAsync(A.scene_acc, 0, sizeof(unsigned long long) * 3 * A.nscenes, c->stream);
       if (e == hipSuccess) e = launch_gs_flow<D, Real>(c, A, F, per_xcd, &launched);
       if (e == hipSuccess && launched && tune) e = hipEventRecord(c->tuner.pend[phase].ev[1], c->stream);

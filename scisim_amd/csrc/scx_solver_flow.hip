@@ -30,7 +30,8 @@
 // in colour order, and a contact waits only for contacts of lower colours of its sweep or of
 // the sweep before; the order (sweep, colour) has no cycle. A slot is written again only by
 // the same contact one sweep later, which follows its reader on the body's cycle. Every wait
-// also ends after kSpinLimit polls: the workgroup then leaves its sweeps and the step fails.
+// also ends after kFlowPolls looks: the wave then waits no more, its workgroup leaves its sweeps
+// when they next meet, every wave reports at the kernel's end and the step fails.
 #pragma clang fp contract(on)
 
 #include "scx_device.h"
@@ -44,7 +45,6 @@ namespace scx {
 typedef uint32_t u32x4f __attribute__((ext_vector_type(4)));
 
 constexpr int kFlowThreads = 512;
-constexpr uint32_t kSpinLimit = 1u << 21;  // about a second of polls
 constexpr size_t kFlowLdsMax = 138 * 1024;  // beside the kernel's static arrays
 constexpr int kFlowAux = 16;               // agent scope (SC1)
 
@@ -186,7 +186,8 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
   const __amdgpu_buffer_rsrc_t frs = __builtin_amdgcn_make_buffer_rsrc(F.flags, (short)0, (int)(4u * kFlowMaxBlocks), 0x00020000);
   const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(F.parts, (short)0, (int)(32u * kFlowMaxBlocks), 0x00020000);
   uint32_t tag = F.tag0;  // of the sweep under way
-  bool dead = false;      // a wait of this wave ran out
+  bool dead = false;      // a wait of this lane ran out
+  uint32_t polls = kFlowPolls;  // of a wait for bodies; F.polls during the sweeps
   // Exchanges so far. Their parts lie in two buffers in turn: a workgroup that publishes for
   // exchange n + 2 has seen every part of exchange n + 1, whose owners had read all of n.
   uint32_t nex = 0;
@@ -330,7 +331,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
         if (check) late = (sa && Port::beyond(ra, ta)) || (sb && Port::beyond(rb, tb));
       }
       ok = oka && (okb || !hasb);
-      if (++n >= kSpinLimit) dead = true;
+      if (!ok && ++n >= polls) dead = true;
     }
     __builtin_amdgcn_s_setprio(3);
     return ok;
@@ -479,7 +480,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
               __builtin_amdgcn_raw_buffer_load_b128(prs, (nex & 1u) * 16u * kFlowMaxBlocks + g * 16u, 0, kFlowAux);
           ok = x[3] == tag;
           if (ok) all = fmax(all, __longlong_as_double((long long)(((unsigned long long)x[1] << 32) | x[0])));
-          if (n >= kSpinLimit) dead = true;
+          if (n >= kFlowPolls) dead = true;
         }
       }
       all = wave_reduce_max_f64(all);
@@ -597,7 +598,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
           const u32x4f y = __builtin_amdgcn_raw_buffer_load_b128(prs, g / per_xcd * per_xcd * 16u, 0, kFlowAux);
           ok = x[3] == tag && y[3] == tag;
           same = same && (!ok || x[0] == y[0]);
-          if (n >= kSpinLimit) dead = true;
+          if (n >= kFlowPolls) dead = true;
         }
       }
       const bool all = __all(same && !dead);
@@ -681,7 +682,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
             }
             skip = __any(any);
             all = skip || __all(here);
-            if (n >= kSpinLimit) dead = true;
+            if (n >= kFlowPolls) dead = true;
           }
           if (lane == 0) {
             s_skip[f] = skip ? 1u : 0u;
@@ -749,6 +750,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
       return false;
     };
     begin_sweep();
+    polls = F.polls;
     if (lane < cur.y >> 8) load(cur.x + lane, c0);
     if constexpr (Ens) {  // one copy of the larger evaluation
       for (bool odd = false;; odd = !odd)
@@ -805,7 +807,9 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
       if (D == 3) rec[1] = w;
     }
   });
-  if (tid == 0 && (dead || s_dead)) atomicOr(&A.ctr->overflow, 16u);
+  // (a wait may have run out after the waves last met)
+  const bool ran_out = __any(dead) || s_dead;
+  if (lane == 0 && ran_out) atomicOr(&A.ctr->overflow, 16u);
   if (wg == 0 && tid == 0) {
     if (A.phase == 1) {
       A.ctr->sweeps_fp32 = it;

@@ -355,6 +355,9 @@ __device__ __forceinline__ void pack_rec(const Rec<D, Real>& R, const typename V
 // Working memory of the sweeps without barriers (k_gs_flow), in colour order.
 constexpr uint32_t kFlowMaxScenes = 2048;  // an ensemble's residuals, in every workgroup's LDS
 constexpr int kFlowMaxBlocks = 256;  // one wave reads every workgroup's flag
+// Looks after which a wait has run out: about a second for a body in a slot or another workgroup's
+// part, a tenth to two tenths for a body in LDS.
+constexpr uint32_t kFlowPolls = 1u << 21;
 // Slots of side b follow those of side a, the near ones (read on one XCD alone) of both follow
 // the far ones, so that no line holds both kinds; kFlowLine consecutive ones fill at least two lines.
 constexpr uint32_t kFlowLine = 16;
@@ -385,6 +388,7 @@ struct FlowBufs {
   // so that its stagnation test knows the best residual of those sweeps too, and the
   // threshold here is the best residual from the start.
   int skip_early;
+  uint32_t polls;     // looks of a wait for bodies during the sweeps, at most (kFlowPolls but in tests)
   uint32_t home;      // bodies of a workgroup that its LDS holds, and 64 more
   uint32_t rows;      // rows of a workgroup's contacts, at most
   uint32_t kept;      // contacts of a workgroup that its LDS holds

@@ -1,0 +1,58 @@
+"""A wait of the sweeps without barriers that runs out fails the call. SCX_FLOW_POLLS=1 lets a wait
+for a body run out at the first look that does not find it; the kernel goes on without waiting and
+ends as always.
+"""
+
+import numpy as np
+import pytest
+
+import scisim_amd as scx
+
+pytestmark = pytest.mark.gpu
+
+
+def _grid(m, gap=-1e-4):
+    """m x m circles a gap from their neighbours, at rest: 2 m (m - 1) contacts in a few colours,
+    each in rows of its own, so all waves but the first wait for another's."""
+    d = 0.1 + gap
+    q = np.stack(np.meshgrid(np.arange(m), np.arange(m)), -1).reshape(-1, 2) * d
+    return dict(q=q.ravel(), v=np.zeros(2 * m * m), r=np.full(m * m, 0.05), m=np.ones(m * m))
+
+
+def _context(monkeypatch, s, polls):
+    for key in ("SCX_FLOW_SWEEPS", "SCX_FLOW_BLOCKS", "SCX_FLOW_XCDS", "SCX_FORCE_PERSISTENT_BLOCKS"):
+        monkeypatch.delenv(key, raising=False)
+    monkeypatch.setenv("SCX_LDS_SWEEPS", "0")
+    if polls:
+        monkeypatch.setenv("SCX_FLOW_POLLS", str(polls))
+    else:
+        monkeypatch.delenv("SCX_FLOW_POLLS", raising=False)
+    ctx = scx.Context(2, s["r"].size, max_planes=8)
+    ctx.set_bodies(s["q"], s["v"], s["r"], s["m"])
+    return ctx
+
+
+def _params(**kw):
+    return scx.step_params(**dict(dict(dt=0.01, g=[0.0, 0.0], mu=0.4, CoR=0.0, tol=1e-10, max_iters=50, eval_every=1,
+                                       integrator=0, precision=scx.FP64, warm_start=scx.WARM_TRANSPORT), **kw))
+
+
+def test_any_wave_reports_a_wait_that_ran_out(monkeypatch):
+    """One FP32 sweep that nothing evaluates: its waves do not meet after their waits, and the first
+    one, whose contacts are of the first colour, waits for nothing."""
+    s = _grid(8)
+    s["v"] = np.random.default_rng(1).normal(0.0, 0.1, s["v"].size)
+    prm = _params(precision=scx.FP32_POLISH, max_iters=1, eval_every=5)
+    ctx = _context(monkeypatch, s, None)
+    try:
+        st = ctx.step(prm)
+        print(st, ctx.sweep_paths(), flush=True)
+        assert st["sweeps_fp32"] == st["sweeps"] == 1 and ctx.sweep_paths()["fp32"] == ("flow", 1)
+    finally:
+        ctx.close()
+    ctx = _context(monkeypatch, s, 1)
+    try:
+        with pytest.raises(scx.ScxError, match="ran out"):
+            ctx.step(prm)
+    finally:
+        ctx.close()
