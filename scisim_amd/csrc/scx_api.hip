@@ -317,15 +317,25 @@ void timing_collect(scx_ctx* c) {
   c->event_names.clear();
 }
 
+// A wait of the sweeps ran out: the bodies are those of the start of that step already; the impulses
+// it left are no warm start and no training targets.
+int waits_failed(scx_ctx* c) {
+  c->d.prev_count = 0;
+  c->d.features_valid = false;
+  timing_collect(c);
+  return fail(c, SCX_E_HIP, "a wait between sweep workgroups ran out");
+}
+
 // One geometric-map step. Returns SCX_OK, or SCX_E_CAPACITY after growing a buffer
-// (the caller retries the step from the untouched start-of-step state).
-int step_once(scx_ctx* c, const scx_step_params* p, scx_step_stats* st, bool want_stats) {
+// (the caller retries the step from the untouched start-of-step state). follows: the step before
+// it belongs to the same call, and its counters may not have been read.
+int step_once(scx_ctx* c, const scx_step_params* p, scx_step_stats* st, bool want_stats, bool follows) {
   hipStream_t s = c->stream;
   DeviceBuffers& d = c->d;
   const uint32_t n = c->n;
   const int D = c->dim;
   if (c->events.empty()) timing_mark(c, "start");
-  HIPC(hipMemsetAsync(d.ctr, 0, sizeof(StepCounters), s));
+  HIPC(hipMemsetAsync(d.ctr, 0, follows ? offsetof(StepCounters, wait_ran_out) : sizeof(StepCounters), s));
   d.features_valid = false;
   if (!c->order_valid) {
     HIPC(launch_order_reset(c, n));
@@ -383,6 +393,12 @@ int step_once(scx_ctx* c, const scx_step_params* p, scx_step_stats* st, bool wan
   const uint32_t nbb = d.host_u32[0];
   if (nbuckets > 0) npl = d.host_u32[1];
   const uint64_t nentries = d.ctr_host->nentries;
+  if (d.ctr_host->wait_ran_out) {  // in the step before
+    std::swap(d.q, d.q0);
+    std::swap(d.v, d.v0);
+    std::swap(d.w, d.w0);
+    return waits_failed(c);
+  }
   if ((d.ctr_host->overflow & 1u) || nentries > c->cap_entries) {
     std::swap(d.q, d.q0);
     std::swap(d.v, d.v0);
@@ -478,7 +494,7 @@ int step_once(scx_ctx* c, const scx_step_params* p, scx_step_stats* st, bool wan
     HIPC(hipMemcpyAsync(d.ctr_host, d.ctr, sizeof(StepCounters), hipMemcpyDeviceToHost, s));
     HIPC(hipStreamSynchronize(s));
     c->last_ncolours = d.ctr_host->ncolours;
-    if (d.ctr_host->overflow & 16u) return fail(c, SCX_E_HIP, "a wait between sweep workgroups ran out");
+    if (d.ctr_host->wait_ran_out) return waits_failed(c);
     comp_adapt_share(c, *d.ctr_host);
     if (c->violator_skip == 2 && p->precision == SCX_PRECISION_FP32_POLISH && c->nscenes == 0 &&
         d.ctr_host->sweeps_fp32 >= 64 && d.ctr_host->evals_skipped == 0)
@@ -910,7 +926,7 @@ int scx_step(scx_ctx* c, const scx_step_params* p, scx_step_stats* stats) {
   if (rc != SCX_OK) return rc;
   HIPC(hipSetDevice(c->device));
   for (int attempt = 0; attempt < 8; ++attempt) {
-    rc = step_once(c, p, stats, true);
+    rc = step_once(c, p, stats, true, false);
     if (rc != SCX_E_CAPACITY) return rc;
   }
   return fail(c, SCX_E_CAPACITY, "buffers kept overflowing");
@@ -927,7 +943,7 @@ int scx_run(scx_ctx* c, const scx_step_params* p, uint32_t nsteps, scx_step_stat
     const bool last = (k + 1 == nsteps);
     int attempt = 0;
     for (; attempt < 8; ++attempt) {
-      rc = step_once(c, &q, last ? stats : nullptr, last);
+      rc = step_once(c, &q, last ? stats : nullptr, last, k > 0);
       if (rc != SCX_E_CAPACITY) break;
     }
     if (rc != SCX_OK) return attempt >= 8 ? fail(c, SCX_E_CAPACITY, "buffers kept overflowing") : rc;
@@ -1191,7 +1207,7 @@ int scx_friction_solve(scx_ctx* c, uint32_t nbodies, const double* m, const doub
   }
   HIPC(hipMemcpyAsync(d.ctr_host, d.ctr, sizeof(StepCounters), hipMemcpyDeviceToHost, s));
   HIPC(hipStreamSynchronize(s));
-  if (d.ctr_host->overflow & 16u) return fail(c, SCX_E_HIP, "a wait between sweep workgroups ran out");
+  if (d.ctr_host->wait_ran_out) return fail(c, SCX_E_HIP, "a wait between sweep workgroups ran out");
   for (uint32_t i = 0; i < nbodies; ++i) {
     if (v2)
       for (int q = 0; q < D; ++q) v2[(size_t)D * i + q] = bv[rec * i + q];

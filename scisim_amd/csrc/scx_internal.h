@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -56,7 +57,7 @@ struct GridParams {
 // Device-side counters of one step, read back by the host at the sync points.
 struct StepCounters {
   unsigned long long nentries;   // grid entries
-  uint32_t overflow;             // bit 0 entries, bit 1 pairs, bit 2 contacts, bit 3 colours, bit 4 a sweep wait ran out
+  uint32_t overflow;             // bit 0 entries, bit 1 pairs, bit 2 contacts, bit 3 colours
   uint32_t ncolours;
   uint32_t nrounds;
   uint32_t remaining;            // uncoloured contacts
@@ -72,6 +73,11 @@ struct StepCounters {
   uint32_t pad;
   double error;                  // best residual of the last phase
   double error_fp32;
+  // Not cleared by a step of scx_run, which reads the counters of its last step alone at the end:
+  // set when a wait of the sweeps ran out. The step's bodies are then put back to its start
+  // (k_finish_bodies), and the next read of the counters fails the call.
+  uint32_t wait_ran_out;
+  uint32_t pad2;
 };
 
 // Per-contact record in colour order used by the sweeps. Real = float or double.

@@ -1413,13 +1413,26 @@ __global__ void __launch_bounds__(kBlock) k_promote_r(uint32_t C, const float* _
 template <int D>
 __global__ void __launch_bounds__(kBlock) k_finish_bodies(uint32_t n, const uint32_t* __restrict__ slot_of,
                                                           const double* __restrict__ body64,
-                                                          const double* __restrict__ q0, const double* __restrict__ m,
+                                                          const double* __restrict__ q0,
+                                                          const double* __restrict__ v0,
+                                                          const double* __restrict__ w0, const double* __restrict__ m,
                                                           double dt, double gx, double gy, double gz, int integrator,
+                                                          const StepCounters* __restrict__ ctr,
                                                           double* __restrict__ q, double* __restrict__ v,
                                                           double* __restrict__ w, double* __restrict__ v2,
                                                           double* __restrict__ w2) {
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
+  if (ctr->wait_ran_out) {  // the sweeps were given up: the step's start state stays
+    for (int d = 0; d < D; ++d) {
+      const size_t k = (size_t)D * i + d;
+      q[k] = q0[k];
+      v2[k] = v[k] = v0[k];
+    }
+    if (D == 3)
+      for (int d = 0; d < 3; ++d) w2[3 * (size_t)i + d] = w[3 * (size_t)i + d] = w0[3 * (size_t)i + d];
+    return;
+  }
   const double g[3] = {gx, gy, gz};
   const double4* rec = reinterpret_cast<const double4*>(body64) + (size_t)kBodyVecs<D> * (slot_of ? slot_of[i] : i);
   const double4 bvi = rec[0];
@@ -1860,11 +1873,13 @@ hipError_t launch_finish(scx_ctx* c, uint32_t C, const scx_step_params* p) {
   const uint32_t nb = (c->n + kBlock - 1) / kBlock;
   if (nb) {
     if (c->dim == 2)
-      k_finish_bodies<2><<<nb, kBlock, 0, s>>>(c->n, c->d.slot_map, c->d.bv64, c->d.q0, c->d.m, p->dt, p->g[0], p->g[1],
-                                               p->g[2], integ, c->d.q, c->d.v, c->d.w, c->d.v2, c->d.w2);
+      k_finish_bodies<2><<<nb, kBlock, 0, s>>>(c->n, c->d.slot_map, c->d.bv64, c->d.q0, c->d.v0, c->d.w0, c->d.m, p->dt,
+                                               p->g[0], p->g[1], p->g[2], integ, c->d.ctr, c->d.q, c->d.v, c->d.w,
+                                               c->d.v2, c->d.w2);
     else
-      k_finish_bodies<3><<<nb, kBlock, 0, s>>>(c->n, c->d.slot_map, c->d.bv64, c->d.q0, c->d.m, p->dt, p->g[0], p->g[1],
-                                               p->g[2], integ, c->d.q, c->d.v, c->d.w, c->d.v2, c->d.w2);
+      k_finish_bodies<3><<<nb, kBlock, 0, s>>>(c->n, c->d.slot_map, c->d.bv64, c->d.q0, c->d.v0, c->d.w0, c->d.m, p->dt,
+                                               p->g[0], p->g[1], p->g[2], integ, c->d.ctr, c->d.q, c->d.v, c->d.w,
+                                               c->d.v2, c->d.w2);
   }
   const uint32_t nc = (C + kBlock - 1) / kBlock;
   if (nc) k_impulses_out<<<nc, kBlock, 0, s>>>(C, c->dim, c->d.perm, c->d.c64.r, c->d.calpha, c->d.cbeta, p->mu);

@@ -809,7 +809,7 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
   });
   // (a wait may have run out after the waves last met)
   const bool ran_out = __any(dead) || s_dead;
-  if (lane == 0 && ran_out) atomicOr(&A.ctr->overflow, 16u);
+  if (lane == 0 && ran_out) atomicOr(&A.ctr->wait_ran_out, 1u);
   if (wg == 0 && tid == 0) {
     if (A.phase == 1) {
       A.ctr->sweeps_fp32 = it;

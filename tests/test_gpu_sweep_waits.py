@@ -56,3 +56,61 @@ def test_any_wave_reports_a_wait_that_ran_out(monkeypatch):
             ctx.step(prm)
     finally:
         ctx.close()
+
+
+def test_run_reports_a_wait_of_any_step(monkeypatch):
+    """Overlapping circles that move apart: contacts, and waits, in the first steps only. Where a
+    contact's impulse is zero the abandoned sweeps change nothing, so nothing else would tell (a
+    tolerance of 0: sweeps up to the limit all the same)."""
+    s = _grid(8)
+    q = s["q"].reshape(-1, 2)
+    s["v"] = (0.005 * (q - q.mean(0))).ravel()  # a gap 1e-4 smaller than a diameter opens in 20 steps
+    ctx = _context(monkeypatch, s, None)
+    try:
+        contacts = [ctx.step(_params(tol=0.0))["ncontacts"] for _ in range(40)]
+        print(contacts, flush=True)
+        assert contacts[0] == 112 and contacts[-1] == 0
+    finally:
+        ctx.close()
+    ctx = _context(monkeypatch, s, 1)
+    try:
+        with pytest.raises(scx.ScxError, match="ran out"):
+            ctx.run(_params(tol=0.0), 40)
+        q, v, _ = ctx.get_state()
+        assert np.array_equal(q, s["q"]) and np.array_equal(v, s["v"])  # the first step's start
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("call", ["step", "run"])
+@pytest.mark.parametrize("staggering", [scx.STAGGER_GEOMETRIC, scx.STAGGER_SYMPLECTIC_EULER])
+def test_the_step_that_failed_leaves_its_start_state(monkeypatch, call, staggering):
+    """Bodies as at the start of the step, and no impulses of it in the cache: loaded into a fresh
+    context, the checkpoint goes on as a fresh scene does from the same bodies."""
+    s = _grid(8)
+    s["v"] = np.random.default_rng(2).normal(0.0, 0.1, s["v"].size)
+    prm = _params(staggering=staggering)
+    ctx = _context(monkeypatch, s, 1)
+    try:
+        with pytest.raises(scx.ScxError, match="ran out"):
+            ctx.step(prm) if call == "step" else ctx.run(prm, 3)
+        q, v, _ = ctx.get_state()
+        assert np.array_equal(q, s["q"]) and np.array_equal(v, s["v"])
+        with pytest.raises(scx.ScxError):  # (warm start 3 computes features, of a step that succeeds)
+            ctx.samples()
+        image = ctx.save_checkpoint()
+        assert scx.checkpoint_info(image)["cache_entries"] == 0
+    finally:
+        ctx.close()
+    out = []
+    for loaded in (False, True):
+        ctx = _context(monkeypatch, s, None)
+        try:
+            if loaded:
+                ctx.load_checkpoint(image)
+            st = ctx.step(prm)
+            assert st["sweeps"] > 1 and ctx.sweep_paths()["fp64"][0] == "flow"
+            out.append(ctx.get_state()[:2])
+        finally:
+            ctx.close()
+    assert all(np.array_equal(x, y) for x, y in zip(*out))
