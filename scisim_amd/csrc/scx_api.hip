@@ -1207,7 +1207,13 @@ int scx_friction_solve(scx_ctx* c, uint32_t nbodies, const double* m, const doub
   }
   HIPC(hipMemcpyAsync(d.ctr_host, d.ctr, sizeof(StepCounters), hipMemcpyDeviceToHost, s));
   HIPC(hipStreamSynchronize(s));
-  if (d.ctr_host->wait_ran_out) return fail(c, SCX_E_HIP, "a wait between sweep workgroups ran out");
+  if (d.ctr_host->wait_ran_out) {  // the caller's impulses stay the warm start they were
+    for (uint32_t k = 0; k < C; ++k) {
+      alpha[k] = rinit[(size_t)D * k];
+      for (int q = 1; q < D; ++q) beta[(size_t)(D - 1) * k + q - 1] = rinit[(size_t)D * k + q];
+    }
+    return fail(c, SCX_E_HIP, "a wait between sweep workgroups ran out");
+  }
   for (uint32_t i = 0; i < nbodies; ++i) {
     if (v2)
       for (int q = 0; q < D; ++q) v2[(size_t)D * i + q] = bv[rec * i + q];

@@ -3,6 +3,8 @@ for a body run out at the first look that does not find it; the kernel goes on w
 ends as always.
 """
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -114,3 +116,30 @@ def test_the_step_that_failed_leaves_its_start_state(monkeypatch, call, staggeri
         finally:
             ctx.close()
     assert all(np.array_equal(x, y) for x, y in zip(*out))
+
+
+@pytest.mark.parametrize("warm", [0.0, 0.01])
+def test_the_solve_that_failed_leaves_the_impulses(monkeypatch, warm):
+    """The impulses of a stand-alone solve are warm start and result; a failed one leaves them."""
+    m = 8
+    at = np.arange(m * m, dtype=np.int32).reshape(m, m)
+    body0 = np.concatenate([at[:, :-1].ravel(), at[:-1].ravel()])
+    body1 = np.concatenate([at[:, 1:].ravel(), at[1:].ravel()])
+    n = np.repeat(-np.eye(2), body0.size // 2, 0)
+    bases = np.stack([n, np.stack([-n[:, 1], n[:, 0]], 1)], 1).ravel()
+    mass, v0, mu = np.ones(m * m), np.random.default_rng(3).normal(size=2 * m * m), np.full(body0.size, 0.4)
+    cs = scx.ScxContactSet(ncontacts=body0.size, body0=scx._p(body0, scx._pi32), body1=scx._p(body1, scx._pi32),
+                           bases=scx._p(bases), mu=scx._p(mu))
+    for polls in (1, None):
+        alpha, beta = np.full(body0.size, warm), np.full(body0.size, -0.1 * warm)
+        ctx = _context(monkeypatch, _grid(m), polls)
+        try:
+            rc = scx.lib().scx_friction_solve(ctx.handle, m * m, scx._p(mass), None, scx._p(v0), None,
+                                              ctypes.byref(cs), 1e-10, 50, 1, scx.FP64, scx._p(alpha), scx._p(beta),
+                                              None, None, None, None, None, None)
+            assert (rc == scx.SCX_OK) == (polls is None)
+            assert ctx.sweep_paths()["fp64"][0] == "flow"
+            unchanged = np.all(alpha == warm) and np.all(beta == -0.1 * warm)
+            assert unchanged == (polls is not None)
+        finally:
+            ctx.close()
