@@ -26,12 +26,14 @@
 //
 // The iterates are those of the colour passes bit for bit: the order of the contacts on
 // every body is the colour order, and a contact reads nothing but its own two bodies.
-// Progress: the launch is cooperative (every workgroup resident), a wave takes its contacts
-// in colour order, and a contact waits only for contacts of lower colours of its sweep or of
-// the sweep before; the order (sweep, colour) has no cycle. A slot is written again only by
-// the same contact one sweep later, which follows its reader on the body's cycle. Every wait
-// also ends after kFlowPolls looks: the wave then waits no more, its workgroup leaves its sweeps
-// when they next meet, every wave reports at the kernel's end and the step fails.
+// Progress: the launch is cooperative (every workgroup gets its place once other kernels have
+// left it), and the first exchange waits for all of them without a limit. Then a wave takes its
+// contacts in colour order, and a contact waits only for contacts of lower colours of its sweep
+// or of the sweep before; the order (sweep, colour) has no cycle. A slot is written again only
+// by the same contact one sweep later, which follows its reader on the body's cycle. Every wait
+// but the first also ends after kFlowPolls looks: the wave then waits no more, its workgroup
+// leaves its sweeps when its waves next meet, every wave reports at the kernel's end and the
+// step fails.
 #pragma clang fp contract(on)
 
 #include "scx_device.h"
@@ -584,26 +586,26 @@ __global__ void __launch_bounds__(kFlowThreads) k_gs_flow(GSArgs<Real> A, FlowBu
     for (int d = 0; d < D; ++d) l_r[(size_t)d * kept + i] = F.r[(size_t)(D == 3 ? 4 : 2) * j + d];
   });
   {
-    // every workgroup's XCD, published and read like the residuals
+    // Every workgroup's XCD, published and read like the residuals. This is also the wait for the
+    // workgroups to become resident: one needs nearly a whole CU's LDS, and a kernel of another
+    // context may hold that for as long as it runs, so it has no limit.
     if (tid < 64) {
       const uint32_t xcc = __builtin_amdgcn_s_getreg(20 | (0 << 6) | (3 << 11));  // XCC_ID
       const u32x4f mine = {xcc, 0u, 0u, tag};
       if (lane == 0) __builtin_amdgcn_raw_buffer_store_b128(mine, prs, wg * 16u, 0, kFlowAux);
       bool same = true;
       for (uint32_t g = lane; g < G; g += 64) {
-        bool ok = false;
-        for (uint32_t n = 0; !ok && !dead; ++n) {
+        for (bool ok = false; !ok;) {
           asm volatile("" ::: "memory");
           const u32x4f x = __builtin_amdgcn_raw_buffer_load_b128(prs, g * 16u, 0, kFlowAux);
           const u32x4f y = __builtin_amdgcn_raw_buffer_load_b128(prs, g / per_xcd * per_xcd * 16u, 0, kFlowAux);
           ok = x[3] == tag && y[3] == tag;
           same = same && (!ok || x[0] == y[0]);
-          if (n >= kFlowPolls) dead = true;
+          if (!ok) __builtin_amdgcn_s_sleep(1);
         }
       }
-      const bool all = __all(same && !dead);
+      const bool all = __all(same);
       if (lane == 0) s_skip[0] = all ? 1u : 0u;
-      if (__any(dead) && lane == 0) s_dead = 1;
     }
     __syncthreads();
     one_l2 = s_skip[0] != 0u;

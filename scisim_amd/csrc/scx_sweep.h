@@ -355,9 +355,10 @@ __device__ __forceinline__ void pack_rec(const Rec<D, Real>& R, const typename V
 // Working memory of the sweeps without barriers (k_gs_flow), in colour order.
 constexpr uint32_t kFlowMaxScenes = 2048;  // an ensemble's residuals, in every workgroup's LDS
 constexpr int kFlowMaxBlocks = 256;  // one wave reads every workgroup's flag
-// Looks after which a wait has run out: about a second for a body in a slot or another workgroup's
-// part, a tenth to two tenths for a body in LDS.
-constexpr uint32_t kFlowPolls = 1u << 21;
+// Looks after which a wait has run out, once every workgroup is resident: about eight seconds for
+// a body in a slot or another workgroup's part, one for a body in LDS. A wait takes microseconds,
+// or as long as other processes have the XCD of the waves that are waited for.
+constexpr uint32_t kFlowPolls = 1u << 24;
 // Slots of side b follow those of side a, the near ones (read on one XCD alone) of both follow
 // the far ones, so that no line holds both kinds; kFlowLine consecutive ones fill at least two lines.
 constexpr uint32_t kFlowLine = 16;

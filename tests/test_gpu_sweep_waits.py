@@ -4,6 +4,8 @@ ends as always.
 """
 
 import ctypes
+import threading
+import time
 
 import numpy as np
 import pytest
@@ -21,10 +23,10 @@ def _grid(m, gap=-1e-4):
     return dict(q=q.ravel(), v=np.zeros(2 * m * m), r=np.full(m * m, 0.05), m=np.ones(m * m))
 
 
-def _context(monkeypatch, s, polls):
+def _context(monkeypatch, s, polls, lds="0"):
     for key in ("SCX_FLOW_SWEEPS", "SCX_FLOW_BLOCKS", "SCX_FLOW_XCDS", "SCX_FORCE_PERSISTENT_BLOCKS"):
         monkeypatch.delenv(key, raising=False)
-    monkeypatch.setenv("SCX_LDS_SWEEPS", "0")
+    monkeypatch.setenv("SCX_LDS_SWEEPS", lds)
     if polls:
         monkeypatch.setenv("SCX_FLOW_POLLS", str(polls))
     else:
@@ -143,3 +145,39 @@ def test_the_solve_that_failed_leaves_the_impulses(monkeypatch, warm):
             assert unchanged == (polls is not None)
         finally:
             ctx.close()
+
+
+def test_a_launch_waits_for_its_workgroups(monkeypatch):
+    """A solve of some seconds in one workgroup of another context leaves one CU short of LDS: sweeps
+    that need all of them wait for it to end."""
+    small, large = _grid(16), _grid(400)
+    for s in (small, large):
+        s["v"] = np.random.default_rng(4).normal(0.0, 0.1, s["v"].size)
+    out, took = [], []
+    for beside in (False, True):
+        ctx = _context(monkeypatch, large, None)
+        try:
+            if beside:
+                other = _context(monkeypatch, small, None, lds="1")
+                done = []
+                t = threading.Thread(target=lambda: done.append(
+                    (other.step(_params(tol=0.0, max_iters=1500000, eval_every=1000)), time.perf_counter())))
+                t.start()
+                time.sleep(0.5)
+            t0 = time.perf_counter()
+            st = ctx.step(_params(max_iters=30))
+            t1 = time.perf_counter()
+            print(st, ctx.sweep_paths(), t1 - t0, flush=True)
+            assert ctx.sweep_paths()["fp64"] == ("flow", 256)
+            if beside:
+                t.join()
+                print(done, other.sweep_paths(), flush=True)
+                assert other.sweep_paths()["fp64"] == ("lds", 1) and done[0][0]["sweeps"] == 1500000
+                other.close()
+            took.append(t1 - t0)
+            out.append(ctx.get_state()[:2])
+        finally:
+            ctx.close()
+    assert all(np.array_equal(x, y) for x, y in zip(*out))
+    print("seconds", took, flush=True)
+    assert took[1] > 1.0  # it did wait
