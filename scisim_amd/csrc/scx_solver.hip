@@ -1671,7 +1671,8 @@ static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint
   // larger ones where nothing is known of the bodies' neighbours (a range of contacts then
   // shares its bodies with all others).
   const bool one = A.C <= (c->d.slot_map ? kFlowOneGroup : kFlowOneGroupUnsorted);
-  const bool flow = free_width && c->flow_sweeps && (one || !c->coop_unavailable) && max_blocks >= (int)kXcds &&
+  const bool flow = free_width && c->flow_sweeps && (one || !c->coop_unavailable) &&
+                    flow_width_limit(max_blocks, c->num_cus, kFlowMaxBlocks, 1) > 0 &&
                     A.C <= kFlowMaxContacts && A.nscenes <= kFlowMaxScenes && A.max_iters < kFlowTagMax / 4 &&
                     (uint64_t)flow_places(A.C) * (D == 3 ? 32 : 16) * sizeof(Real) < (1ull << 31);
   // the autotuner picks among widths around the model's (not for the solves of one workgroup)
@@ -1679,7 +1680,8 @@ static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint
   const bool tune = c->tuner.enabled && c->force_blocks <= 0 && !lds_path && !(flow && one) && !c->coop_unavailable;
   // one XCD's CUs up to kFlowOneXcd contacts, all beyond
   const uint32_t xcds = c->flow_xcds > 0 ? (uint32_t)c->flow_xcds : A.C <= kFlowOneXcd ? 1 : kXcds;
-  const int flow_most = std::min(max_blocks, kFlowMaxBlocks) / (int)kXcds * (int)xcds;
+  static_assert(kXcds == 8, "flow_width_limit");
+  const int flow_most = flow_width_limit(max_blocks, c->num_cus, kFlowMaxBlocks, (int)xcds);
   const int width =
       !flow ? model : one ? 1 : std::max(2, std::min((int)((A.C + kFlowContacts - 1) / kFlowContacts), flow_most));
   const int want = tune ? tune_pick(c, phase, tune_key(D, phase, A.cscene != nullptr, A.C, nw), width,

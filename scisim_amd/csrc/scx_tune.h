@@ -167,4 +167,15 @@ inline void comp_share_update(double& share, double& ceiling, uint32_t overflows
   }
 }
 
+// Workgroups of a launch of the sweeps without barriers, at most, on `xcds` of the 8 XCDs that
+// the dispatcher deals workgroups to in turn. The grid has 8 workgroups for each one per XCD, all
+// of them resident at once; one fills most of a CU's LDS, so a CU holds one, also where the
+// persistent kernels with barriers may have more (max_blocks). A wave reads the words of all of
+// them, `most`. 0: the device is too small for these sweeps.
+inline int flow_width_limit(int max_blocks, int num_cus, int most, int xcds) {
+  int b = max_blocks < num_cus ? max_blocks : num_cus;
+  if (b > most) b = most;
+  return b / 8 * xcds;
+}
+
 }  // namespace scx
