@@ -17,6 +17,7 @@
 #include "scx_device.h"
 #include "scx_flow.h"
 #include "scx_internal.h"
+#include "scx_sweep.h"
 
 using namespace scx;
 
@@ -649,6 +650,9 @@ int scx_create(const scx_config* cfg, scx_ctx** out) {
     // (the results depend on neither; for tests)
     if (const char* env = getenv("SCX_FLOW_BLOCKS")) c->flow_blocks = std::max(0, atoi(env));
     if (const char* env = getenv("SCX_FLOW_XCDS")) c->flow_xcds = std::max(1, std::min(atoi(env), (int)kXcds));
+    // SCX_FLOW_TAG: the first sweep tag of the context (for tests of the tags' end)
+    if (const char* env = getenv("SCX_FLOW_TAG"))
+      c->flow_tag = (uint32_t)std::max<long>(1, std::min<long>(atol(env), kFlowTagMax - 1));
     // SCX_FLOW_POLLS: the looks after which a wait for a body in those sweeps has run out and the
     // step fails (for tests of that failure)
     if (const char* env = getenv("SCX_FLOW_POLLS")) c->flow_polls = (uint32_t)std::max(0, atoi(env));

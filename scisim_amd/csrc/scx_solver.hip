@@ -1525,7 +1525,6 @@ static hipError_t tune_after_solve(scx_ctx* c) {
 // Sweeps without barriers between the colours (k_gs_flow): their buffers, in the context's
 // arenas (grown when a larger contact set takes the path), and the links of this contact set
 // (shared by the two phases of a solve).
-constexpr uint32_t kFlowTagMax = 1u << 30;
 // Ahead of the sweeps with barriers at every size measured (whole solves, ms, with barriers and
 // without): spheres 16,987 contacts 14.9 and 6.2, 34,176 20.7 and 9.2, 99,626 17.1 and 8.4,
 // 423,718 30.1 and 13.9, 848,458 19.0 and 8.5, 1,283,826 18.7 and 11.4. kFlowMaxContacts bounds

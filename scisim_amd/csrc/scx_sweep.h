@@ -354,6 +354,7 @@ __device__ __forceinline__ void pack_rec(const Rec<D, Real>& R, const typename V
 
 // Working memory of the sweeps without barriers (k_gs_flow), in colour order.
 constexpr uint32_t kFlowMaxScenes = 2048;  // an ensemble's residuals, in every workgroup's LDS
+constexpr uint32_t kFlowTagMax = 1u << 30;  // the tags of a context start over on cleared slots
 constexpr int kFlowMaxBlocks = 256;  // one wave reads every workgroup's flag
 // Looks after which a wait has run out, once every workgroup is resident: about eight seconds for
 // a body in a slot or another workgroup's part, one for a body in LDS. A wait takes microseconds,

@@ -15,7 +15,7 @@ import test_gpu_sweep_paths as base
 
 pytestmark = pytest.mark.gpu
 
-SWITCHES = ("SCX_LDS_SWEEPS", "SCX_FLOW_SWEEPS", "SCX_FLOW_BLOCKS", "SCX_FLOW_XCDS", "SCX_FORCE_PERSISTENT_BLOCKS")
+SWITCHES = ("SCX_LDS_SWEEPS", "SCX_FLOW_SWEEPS", "SCX_FLOW_BLOCKS", "SCX_FLOW_XCDS", "SCX_FORCE_PERSISTENT_BLOCKS", "SCX_FLOW_TAG")
 
 
 def _context(monkeypatch, s, **env):
@@ -117,6 +117,21 @@ def test_large_sets(monkeypatch, m, groups, precision):
     got, paths = _run(monkeypatch, s, prm, 1)
     print(ref[0][0], paths, flush=True)
     _all(paths, precision, "flow" if groups else "barriers", groups)
+    base._same(ref, got)
+
+
+@pytest.mark.parametrize("kind", ["700", "9000"])
+@pytest.mark.parametrize("short", [1, 166, 167, 300, 500])
+def test_tags_start_over(monkeypatch, kind, short):
+    """A launch takes its limit of 150 sweeps and 16 more tags. With fewer left, the tags start over on
+    cleared slots: before the first launch, between the two phases of a step, or in a later step
+    (300, 500); the steps are those of a context at its first tags."""
+    print("case", kind, short, flush=True)
+    s = base._scene(kind)
+    prm = base._params(s, "fp32", "limit")
+    ref, paths = _run(monkeypatch, s, prm, 4, SCX_LDS_SWEEPS=0)
+    _all(paths, "fp32", "flow")
+    got, _ = _run(monkeypatch, s, prm, 4, SCX_LDS_SWEEPS=0, SCX_FLOW_TAG=2 ** 30 - short)
     base._same(ref, got)
 
 
