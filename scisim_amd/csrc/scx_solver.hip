@@ -1538,9 +1538,14 @@ constexpr uint32_t kFlowContacts = 128;  // contacts of a workgroup
 constexpr uint32_t kFlowOneXcd = 1u << 16;
 // Up to kFlowOneGroup contacts one workgroup does better than several: all its bodies live in its
 // LDS. One workgroup, two and eight, FP64 solves in ms: spheres 522 contacts 3.5, 4.9 and 5.1,
-// 1,377 6.1, 6.8 and 7.6, 2,454 10.7, 7.2 and 7.2; a stand-alone solve of 2,600 sphere contacts,
-// whose bodies come in no order, 11.6, 13.8 and 14.2 (32 workgroups: 12.3).
-constexpr uint32_t kFlowOneGroup = 1536, kFlowOneGroupUnsorted = 3072;
+// 1,377 6.1, 6.8 and 7.6, 2,454 10.7, 7.2 and 7.2. Stand-alone solves, whose bodies come in no
+// order, so that several workgroups share most of them: one workgroup and one for every 128
+// contacts, 300 sweeps in ms, FP64 with a residual every sweep, every 20, and FP32 with the polish:
+// spheres 2,194 contacts 7.6 and 8.5, 4.7 and 6.8, 6.5 and 6.9; 2,650 7.8 and 8.2, 5.2 and 7.0, 7.0
+// and 6.8; 2,867 8.9 and 7.8, 6.4 and 6.6, 7.7 and 6.8; 3,285 12.9 and 8.7, 8.8 and 7.0, 10.7 and
+// 7.2; circles 2,380 4.4 and 3.8, 2.5 and 2.6, 3.9 and 3.4; 2,964 5.4 and 3.8, 3.0 and 2.6, 4.8
+// and 3.6. The line lies where several win whatever the residuals.
+constexpr uint32_t kFlowOneGroup = 1536, kFlowOneGroupUnsorted = 2816;
 
 static hipError_t flow_arena(unsigned char** p, size_t* cap, size_t need, hipStream_t s) {
   if (need <= *cap) return hipSuccess;

@@ -120,6 +120,40 @@ def test_large_sets(monkeypatch, m, groups, precision):
     base._same(ref, got)
 
 
+@pytest.mark.parametrize("dim,side,one", [(3, 10, True), (3, 11, False), (2, 38, True), (2, 39, False)])
+def test_stand_alone_solves(monkeypatch, dim, side, one):
+    """Contacts of bodies in no order, 2,700 and 3,630 of spheres, 2,812 and 2,964 of circles: one
+    workgroup up to 2,816."""
+    rng = np.random.default_rng(side)
+    n = side ** dim
+    at = rng.permutation(n).reshape((side,) * dim)
+    a = np.concatenate([np.delete(at, -1, k).ravel() for k in range(dim)]).astype(np.int32)
+    b = np.concatenate([np.delete(at, 0, k).ravel() for k in range(dim)]).astype(np.int32)
+    nn = -np.eye(dim)[np.repeat(np.arange(dim), a.size // dim)]
+    t1 = np.roll(nn, 1, 1) * (1.0 if dim == 3 else [[-1.0, 1.0]])
+    prob = dict(m=rng.uniform(1.0, 2.0, n), v0=rng.normal(size=dim * n), body0=a, body1=b, mu=np.full(a.size, 0.4))
+    if dim == 3:
+        prob.update(inertia=rng.uniform(0.1, 0.2, n), omega0=rng.normal(size=3 * n), arm0=-0.5 * nn, arm1=0.5 * nn,
+                    bases=np.stack([nn, t1, np.cross(nn, t1)], 1))
+    else:
+        prob.update(bases=np.stack([nn, t1], 1))
+    out = []
+    for flow in ("0", "1"):
+        for key in SWITCHES:
+            monkeypatch.delenv(key, raising=False)
+        monkeypatch.setenv("SCX_FLOW_SWEEPS", flow)
+        ctx = scx.Context(dim, n, max_planes=8)
+        try:
+            out.append(ctx.friction_solve(tol=1e-9, max_iters=200, eval_every=1, precision=scx.FP64, **prob))
+            path, groups = ctx.sweep_paths()["fp64"]
+        finally:
+            ctx.close()
+    print(a.size, out[1]["sweeps"], path, groups, flush=True)
+    assert path == "flow" and (groups == 1) == one
+    for key, x in out[0].items():
+        assert np.array_equal(x, out[1][key]), key
+
+
 @pytest.mark.parametrize("kind", ["700", "9000"])
 @pytest.mark.parametrize("short", [1, 166, 167, 300, 500])
 def test_tags_start_over(monkeypatch, kind, short):
