@@ -178,7 +178,9 @@ int scx_get_scene_stats(scx_ctx* ctx, uint32_t nscenes, uint32_t* ncontacts, dou
 int scx_get_state(scx_ctx* ctx, double* q, double* v, double* omega);
 
 /* One impact-friction map step on the resident state (GeometricImpactFrictionMap, or the
- * staggering named by p->staggering). stats may be NULL. */
+ * staggering named by p->staggering). stats may be NULL. A step whose sweeps were given up
+ * (a wait between their workgroups that did not end, SCX_E_HIP; scx_run: in any of its steps)
+ * leaves the bodies of its start and an empty impulse cache. */
 int scx_step(scx_ctx* ctx, const scx_step_params* p, scx_step_stats* stats);
 /* Several steps without host synchronisation between them except where the
  * pipeline needs counts; stats (may be NULL) receives the last step's stats. */

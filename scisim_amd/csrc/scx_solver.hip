@@ -1528,7 +1528,8 @@ static hipError_t tune_after_solve(scx_ctx* c) {
 // Ahead of the sweeps with barriers at every size measured (whole solves, ms, with barriers and
 // without): spheres 16,987 contacts 14.9 and 6.2, 34,176 20.7 and 9.2, 99,626 17.1 and 8.4,
 // 423,718 30.1 and 13.9, 848,458 19.0 and 8.5, 1,283,826 18.7 and 11.4. kFlowMaxContacts bounds
-// the buffers (0.5 GB per million contacts). Workgroups: 128 contacts each, up to the CUs in use.
+// the buffers (per million contacts 0.57 GB for spheres, 0.31 for circles, a quarter of it in hand for
+// growth). Workgroups: 128 contacts each, up to the CUs in use.
 constexpr uint32_t kFlowMaxContacts = 1u << 21;
 constexpr uint32_t kFlowContacts = 128;  // contacts of a workgroup
 // Up to kFlowOneXcd contacts one XCD's CUs do better than all: every slot is then a near one

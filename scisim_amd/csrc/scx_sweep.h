@@ -188,11 +188,11 @@ struct GSArgs {
   uint32_t* lmap;           // per body slot: owning endpoint in the LDS solve (all ones when idle)
   uint32_t tail_col;        // colours [tail_col, ncolours) are swept by workgroup 0 alone (small)
   // ensembles (else cscene == nullptr): per contact (colour order) its scene; per scene the
-  // residual of the last two evaluations (max ||FB||^2 bits, double-buffered) and the sweep
-  // at which it met the tolerance (kNoBody until then). A scene that meets the tolerance is
-  // frozen: its contacts are skipped until the solve ends.
+  // residual of the last evaluations (max ||FB||^2 bits; k_gs uses two buffers in turn,
+  // k_gs_flow three) and the sweep at which it met the tolerance (kNoBody until then). A scene
+  // that meets the tolerance is frozen: its contacts are skipped until the solve ends.
   const uint32_t* cscene;
-  unsigned long long* scene_acc;  // 2 x nscenes
+  unsigned long long* scene_acc;  // 3 x nscenes
   uint32_t* scene_sweeps;         // nscenes
   uint32_t nscenes;
   // ensembles: the contacts of scenes not yet frozen, compacted colour by colour once
@@ -231,7 +231,8 @@ struct Loaded {
 // One contact of a colour pass from its loaded record, on body vectors ia and ib (3D: ia + 1
 // and ib + 1 are the angular halves of the same records) read and written through ld/st,
 // the new impulse stored through st_r(d, x). rbest: first store the contact's impulse as it
-// was before this sweep there (the previous sweep's iterate was the best one so far). Every update of a contact goes through this code, wherever its bodies are held.
+// was before this sweep there (the previous sweep's iterate was the best one so far). Every
+// update of a contact goes through this code, wherever its bodies are held.
 template <int D, typename Real, typename Ld, typename St, typename StR>
 __device__ __forceinline__ void update_core(const Loaded<D, Real>& L, bool init, Real* rbest, size_t ia, size_t ib,
                                             Ld&& ld, St&& st, StR&& st_r) {
@@ -352,7 +353,8 @@ __device__ __forceinline__ void pack_rec(const Rec<D, Real>& R, const typename V
   }
 }
 
-// Working memory of the sweeps without barriers (k_gs_flow), in colour order.
+// Working memory of the sweeps without barriers (k_gs_flow). Contacts have places: workgroup
+// after workgroup, within one in colour order.
 constexpr uint32_t kFlowMaxScenes = 2048;  // an ensemble's residuals, in every workgroup's LDS
 constexpr uint32_t kFlowTagMax = 1u << 30;  // the tags of a context start over on cleared slots
 constexpr int kFlowMaxBlocks = 256;  // one wave reads every workgroup's flag
