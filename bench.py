@@ -22,7 +22,8 @@ final update) with the state resident in HBM. --steps sets only the number of ti
 training, the comparison) is untimed and fixed by its own options. value = bodies * steps
 / wall time of the timed steps. roofline: the dominant kernel by device time, its
 algorithmic bytes per launch (scisim_amd/roofline.py) over its mean launch duration from
-HIP events on the library's stream; traffic is null unless --traffic gives HBM bytes per
+HIP events on the library's stream (for the sweeps without barriers, which keep most of their
+data in LDS and are bound by latency, these are modelled bytes and no HBM rate); traffic is null unless --traffic gives HBM bytes per
 launch measured by rocprofv3 --pmc in the same command. cpu_baseline: the FP64 oracle (the
 project's restatement of the reference path: natural-order Gauss-Seidel from a cold
 start, as the reference) on the state in the middle of the timed steps, on all host cores
@@ -428,12 +429,17 @@ def main():
     value = n * args.steps / wall
     # dominant kernel: the neighbour sweep (two launches per step) or the Gauss-Seidel
     # sweeps (one FP32 and one FP64 launch per step), by device time
+    # The sweeps without barriers keep bodies, impulses and records in LDS and are bound by the
+    # chain of waits along the colours: their byte count is a model (the bytes of sweeps that keep
+    # nothing on chip), not HBM traffic.
+    flow = "flow" in (ctx.sweep_paths()["fp32"][0], ctx.sweep_paths()["fp64"][0])
+    gs_kernel = "Gauss-Seidel sweeps (%s)" % ("k_gs_flow, no barriers between the colours" if flow else "k_gs")
     pairs_ms = phase_ms.get("pairs_count", 0.0) + phase_ms.get("pairs_write", 0.0)
     gs_ms = phase_ms.get("gs_fp32", 0.0) + phase_ms.get("gs_fp64", 0.0)
     if pairs_ms >= gs_ms:
         kernel, launches, kbytes, kms = "k_pairs (grid neighbour sweep + FP64 narrow phase)", 2, pairs_bytes, pairs_ms
     else:
-        kernel, launches, kbytes, kms = "Gauss-Seidel sweeps (k_gs_flow; k_gs above 2,097,152 contacts)", 1 + int(fp32), gs_bytes, gs_ms
+        kernel, launches, kbytes, kms = gs_kernel, 1 + int(fp32), gs_bytes, gs_ms
     traffic = None
     if args.traffic:
         traffic = read_traffic(args.traffic).get("bytes_per_launch")
@@ -490,7 +496,9 @@ def main():
         "dtype": "f32 sweeps + f64 residual/polish" if fp32 else "f64",
         "data": "synthetic",
         "config": config,
-        "roofline": {"bound": "hbm", "kernel": kernel, "achieved": achieved, "peak": rl.HBM_PEAK_GBS, "unit": "GB/s",
+        "roofline": {"bound": "latency" if kernel == gs_kernel and flow else "hbm", "kernel": kernel,
+                     "bytes": "modelled per contact and sweep, not HBM traffic" if kernel == gs_kernel and flow
+                     else "algorithmic", "achieved": achieved, "peak": rl.HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / rl.HBM_PEAK_GBS, "traffic": traffic,
                      "bytes_per_launch": kbytes / (launches * args.steps),
                      "us_per_launch": 1000.0 * kms / (launches * args.steps)},

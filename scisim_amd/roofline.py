@@ -3,7 +3,9 @@
 Counting convention: compulsory traffic. Each distinct array a launch must read or
 write counts once per launch (re-reads served by caches are not counted), except the
 Gauss-Seidel sweeps, which count the per-contact gather/scatter of body velocities on
-every sweep because every colour pass touches the bodies again.
+every sweep because every colour pass touches the bodies again. (The sweeps without
+barriers keep most bodies, impulses and records in LDS, so for them this is a model: in the FP32
+phase of a 262,144-sphere pile they move 44 of the 186 bytes through HBM, in FP64 376 of 554.)
 
 Units: N bodies, E grid entries (covered cells summed over all boxes), G grid cells,
 P emitted pairs, C contacts, S sweeps.
