@@ -1547,6 +1547,17 @@ constexpr uint32_t kFlowOneXcd = 1u << 16;
 // 7.2; circles 2,380 4.4 and 3.8, 2.5 and 2.6, 3.9 and 3.4; 2,964 5.4 and 3.8, 3.0 and 2.6, 4.8
 // and 3.6. The line lies where several win whatever the residuals.
 constexpr uint32_t kFlowOneGroup = 1536, kFlowOneGroupUnsorted = 2816;
+// Stand-alone solves of spheres in FP64 above one XCD's sets: with the bodies in no order nearly
+// every hop goes across XCDs, and grid barriers with the component phase do better up to about half
+// a million contacts. 300 sweeps in ms with barriers and without, contacts in the order of a poured
+// pile and shuffled, a residual every sweep: 63,153 contacts (one XCD) 29.8 and 27.0, 32.0 and
+// 29.5; 90,475 30.9 and 38.1, 33.5 and 34.2; 145,085 33.3 and 42.5, 36.8 and 43.9; 361,939 39.9
+// and 35.9, 43.0 and 54.6; 496,814 45.3 and 38.2, 47.9 and 61.1; 723,701 66.2 and 36.5, 70.2 and
+// 66.5. Every 20 sweeps: 90,475 25.7 and 37.7, 28.9 and 32.5; 361,939 30.0 and 30.1, 32.3 and
+// 56.3; 723,701 50.4 and 23.2, 53.0 and 58.9. FP32 phases are level or ahead without (145,085 with
+// the polish behind barriers 18.1 and 20.5, all with barriers 21.3 and 24.7), circles ahead
+// everywhere (217,140 20.4 and 11.9, 24.7 and 16.0).
+constexpr uint32_t kFlowScattered = 1u << 19;
 
 static hipError_t flow_arena(unsigned char** p, size_t* cap, size_t need, hipStream_t s) {
   if (need <= *cap) return hipSuccess;
@@ -1676,7 +1687,9 @@ static hipError_t coop_gs(scx_ctx* c, GSArgs<Real> A, int max_blocks, const uint
   // larger ones where nothing is known of the bodies' neighbours (a range of contacts then
   // shares its bodies with all others).
   const bool one = A.C <= (c->d.slot_map ? kFlowOneGroup : kFlowOneGroupUnsorted);
-  const bool flow = free_width && c->flow_sweeps && (one || !c->coop_unavailable) &&
+  const bool scattered = !c->d.slot_map && D == 3 && std::is_same<Real, double>::value && A.C > kFlowOneXcd &&
+                         A.C <= kFlowScattered;
+  const bool flow = free_width && c->flow_sweeps && !scattered && (one || !c->coop_unavailable) &&
                     flow_width_limit(max_blocks, c->num_cus, kFlowMaxBlocks, 1) > 0 &&
                     A.C <= kFlowMaxContacts && A.nscenes <= kFlowMaxScenes && A.max_iters < kFlowTagMax / 4 &&
                     (uint64_t)flow_places(A.C) * (D == 3 ? 32 : 16) * sizeof(Real) < (1ull << 31);

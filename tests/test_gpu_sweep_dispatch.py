@@ -120,10 +120,15 @@ def test_large_sets(monkeypatch, m, groups, precision):
     base._same(ref, got)
 
 
-@pytest.mark.parametrize("dim,side,one", [(3, 10, True), (3, 11, False), (2, 38, True), (2, 39, False)])
-def test_stand_alone_solves(monkeypatch, dim, side, one):
-    """Contacts of bodies in no order, 2,700 and 3,630 of spheres, 2,812 and 2,964 of circles: one
-    workgroup up to 2,816."""
+@pytest.mark.parametrize("dim,side,path,precision",
+                         [(3, 10, "flow 1", "fp64"), (3, 11, "flow 29", "fp64"), (2, 38, "flow 1", "fp64"),
+                          (2, 39, "flow 24", "fp64"), (3, 28, "flow 32", "fp64"), (3, 29, "barriers", "fp64"),
+                          (3, 29, "barriers", "fp32"), (3, 56, "barriers", "fp64"), (3, 57, "flow 256", "fp64"),
+                          (2, 190, "flow 256", "fp64")])
+def test_stand_alone_solves(monkeypatch, dim, side, path, precision):
+    """Contacts of bodies in no order, spheres on a cubic lattice and circles on a square one: one
+    workgroup up to 2,816 contacts, one XCD up to 65,536; spheres in FP64 with grid barriers from
+    there (63,504 and 70,644 here) to 524,288 (517,440 and 545,832)."""
     rng = np.random.default_rng(side)
     n = side ** dim
     at = rng.permutation(n).reshape((side,) * dim)
@@ -144,12 +149,14 @@ def test_stand_alone_solves(monkeypatch, dim, side, one):
         monkeypatch.setenv("SCX_FLOW_SWEEPS", flow)
         ctx = scx.Context(dim, n, max_planes=8)
         try:
-            out.append(ctx.friction_solve(tol=1e-9, max_iters=200, eval_every=1, precision=scx.FP64, **prob))
-            path, groups = ctx.sweep_paths()["fp64"]
+            out.append(ctx.friction_solve(tol=1e-9, max_iters=200 if a.size < 9000 else 20, eval_every=1,
+                                          precision=scx.FP64 if precision == "fp64" else scx.FP32_POLISH, **prob))
+            paths = ctx.sweep_paths()
         finally:
             ctx.close()
-    print(a.size, out[1]["sweeps"], path, groups, flush=True)
-    assert path == "flow" and (groups == 1) == one
+    print(a.size, out[1]["sweeps"], paths, flush=True)
+    assert ("%s %d" % paths["fp64"]).startswith(path)
+    assert paths["fp32"][0] == (None if precision == "fp64" else "flow")
     for key, x in out[0].items():
         assert np.array_equal(x, out[1][key]), key
 
